@@ -18,13 +18,12 @@ records ms/step: parameters of the power-of-two lengths at N (256), those of
 the radix-3 lengths from 192 up (NS3D_R3_*) at N3 (192).  ``select`` keeps, for each parameter, the value with the
 lowest time when it beats the baseline by more than ``--margin`` (parameters
 of different passes act on different kernels, so their gains add), and
-writes ``csrc/tuned.hpp``, which ns3d_api.hip includes before the defaults.
+writes ``csrc/tuned.hpp``, which launch.hpp includes before the defaults.
 Variant libraries and timings stay in DIR (default ns3dperiodic_amd/_tune).
 """
 import argparse
 import json
 import os
-import subprocess
 import sys
 import time
 from concurrent.futures import ThreadPoolExecutor
@@ -36,16 +35,12 @@ DEFAULT_OUT = os.path.join(HERE, "_tune")
 # parameter -> (source default, candidates, precisions whose step it changes,
 #               lengths it applies to: "pow2" timed at N, "r3" (radix-3, >= 192) at N3)
 SPACE = {
-    "NS3D_EXINV64": (4, [4, 8], ["fp64"], "pow2"),
     "NS3D_EYINV64": (4, [4, 8], ["fp64"], "pow2"),
-    "NS3D_EXFWD64": (8, [4, 8], ["fp64"], "pow2"),
     "NS3D_PXINV64": (8, [4, 8], ["fp64"], "pow2"),
     "NS3D_PYINV64": (8, [4, 8], ["fp64"], "pow2"),
     "NS3D_PZT64": (128, [64, 128, 256], ["fp64"], "pow2"),
     "NS3D_ZSWZ": (8, [0, 8, 16], ["fp64"], "pow2"),
     "NS3D_ZILP": (1, [0, 1], ["fp64"], "pow2"),
-    "NS3D_XFWD_ILP": (2, [0, 1, 2], ["fp64", "fp32", "fp32s", "fp32i"], "pow2"),
-    "NS3D_EXINV32": (8, [4, 8], ["fp32", "fp32s", "fp32i"], "pow2"),
     "NS3D_EYINV32": (4, [4, 8], ["fp32", "fp32s", "fp32i"], "pow2"),
     "NS3D_PXINV32": (8, [4, 8, 16], ["fp32", "fp32s", "fp32i"], "pow2"),
     "NS3D_PYINV32": (8, [4, 8, 16], ["fp32", "fp32s", "fp32i"], "pow2"),
@@ -54,7 +49,6 @@ SPACE = {
     "NS3D_PZT32": (128, [64, 128, 256], ["fp32", "fp32s", "fp32i"], "pow2"),
     "NS3D_ZPLAN32": (8, [4, 8], ["fp32", "fp32s", "fp32i"], "pow2"),
     "NS3D_ZSWZ32": (16, [0, 16], ["fp32", "fp32s", "fp32i"], "pow2"),
-    "NS3D_EXFWD32": (4, [4, 8], ["fp32", "fp32s", "fp32i"], "pow2"),
     "NS3D_ZILP32": (0, [0, 1], ["fp32", "fp32s", "fp32i"], "pow2"),
     "NS3D_ZWAVE": (1, [0, 1], ["fp64", "fp32", "fp32s", "fp32i"], "pow2"),
     "NS3D_ZTWREG": (1, [0, 1], ["fp64"], "pow2"),
@@ -107,12 +101,8 @@ def _build_one(out_dir, name, overrides, base):
     vals.update(overrides)
     flags = [f"-D{k}={v}" for k, v in sorted(vals.items())]
     lib = os.path.join(out_dir, f"lib_{name.replace('=', '_')}.so")
-    src = os.path.join(HERE, "csrc", "ns3d_api.hip")
-    cmd = [B.hipcc(), *B.HIPCC_FLAGS, "-DNS3D_NO_TUNED_HEADER", *flags, src, "-o", lib]
     t0 = time.time()
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    if r.returncode:
-        raise RuntimeError(f"variant {name} failed to build:\n{r.stderr[-2000:]}")
+    B.compile_library(lib, ["-DNS3D_NO_TUNED_HEADER", *flags], jobs=1)
     return name, lib, time.time() - t0
 
 

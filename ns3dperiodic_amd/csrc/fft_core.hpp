@@ -58,10 +58,18 @@ template <> struct Radix<5> {
         const cplx<T> a0 = v[0];
         const cplx<T> t1 = v[1] + v[4], t2 = v[2] + v[3];
         const cplx<T> t3 = v[1] - v[4], t4 = v[2] - v[3];
-        const cplx<T> m1 = mk<T>(a0.x + c1 * t1.x + c2 * t2.x, a0.y + c1 * t1.y + c2 * t2.y);
-        const cplx<T> m2 = mk<T>(a0.x + c2 * t1.x + c1 * t2.x, a0.y + c2 * t1.y + c1 * t2.y);
-        const cplx<T> n1 = mul_i<DIR>(mk<T>(s1 * t3.x + s2 * t4.x, s1 * t3.y + s2 * t4.y));
-        const cplx<T> n2 = mul_i<DIR>(mk<T>(s2 * t3.x - s1 * t4.x, s2 * t3.y - s1 * t4.y));
+        cplx<T> m1, m2, n1, n2;
+        if constexpr (sizeof(T) == 8) {  // contraction spelled out, as in cmul
+            m1 = mk<T>(__builtin_fma(c2, t2.x, __builtin_fma(c1, t1.x, a0.x)), __builtin_fma(c2, t2.y, __builtin_fma(c1, t1.y, a0.y)));
+            m2 = mk<T>(__builtin_fma(c1, t2.x, __builtin_fma(c2, t1.x, a0.x)), __builtin_fma(c1, t2.y, __builtin_fma(c2, t1.y, a0.y)));
+            n1 = mul_i<DIR>(mk<T>(__builtin_fma(s1, t3.x, s2 * t4.x), __builtin_fma(s1, t3.y, s2 * t4.y)));
+            n2 = mul_i<DIR>(mk<T>(__builtin_fma(s2, t3.x, -(s1 * t4.x)), __builtin_fma(s2, t3.y, -(s1 * t4.y))));
+        } else {
+            m1 = mk<T>(a0.x + c1 * t1.x + c2 * t2.x, a0.y + c1 * t1.y + c2 * t2.y);
+            m2 = mk<T>(a0.x + c2 * t1.x + c1 * t2.x, a0.y + c2 * t1.y + c1 * t2.y);
+            n1 = mul_i<DIR>(mk<T>(s1 * t3.x + s2 * t4.x, s1 * t3.y + s2 * t4.y));
+            n2 = mul_i<DIR>(mk<T>(s2 * t3.x - s1 * t4.x, s2 * t3.y - s1 * t4.y));
+        }
         v[0] = a0 + t1 + t2;
         v[1] = m1 + n1;
         v[4] = m1 - n1;

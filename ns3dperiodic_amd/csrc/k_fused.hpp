@@ -25,13 +25,6 @@ template <typename T, int N> struct PtrArr { T* p[N]; };
 #ifndef NS3D_WAVES_XY
 #define NS3D_WAVES_XY 2
 #endif
-// Two transforms in step (PencilFFT::run2, a second exchange buffer) for the
-// first two components of the x-forward pass: 0 off, 1 FP64 only, 2 both
-// precisions (measured at 256^3: FP64 pass 0.407 -> 0.401 ms, its register
-// spill gone; the x- and y-inverse passes, at 4-7 waves/SIMD, gained nothing).
-#ifndef NS3D_XFWD_ILP
-#define NS3D_XFWD_ILP 2
-#endif
 #ifndef NS3D_WAVES_Z
 #define NS3D_WAVES_Z 2
 #endif
@@ -65,6 +58,13 @@ template <typename T, int N> struct PtrArr { T* p[N]; };
 #ifndef NS3D_TW_LATE
 #define NS3D_TW_LATE 1
 #endif
+// Runs put(true_type) or put(false_type): the nontemporal and the ordinary form of a store loop.
+template <class F> __device__ __forceinline__ void by_nt(int nt, F&& put) {
+    if (nt)
+        put(std::true_type{});
+    else
+        put(std::false_type{});
+}
 template <int REV>
 __device__ __forceinline__ int tile_order(int bid, int nb) {
     return REV ? nb - 1 - bid : bid;
@@ -77,6 +77,33 @@ __device__ __forceinline__ int tile_order(int bid, int nb) {
 #ifndef NS3D_WAVES_XFWD32
 #define NS3D_WAVES_XFWD32 2
 #endif
+// Minimum waves per SIMD of the FP64 x-forward pass.
+#ifndef NS3D_WAVES_XFWD64
+#define NS3D_WAVES_XFWD64 2
+#endif
+// x-forward pass: modes of one component per operand unit, and units in flight
+// (k_x_fwd_epi), for FP64 with 4 and 8 points per thread and for FP32.
+#ifndef NS3D_XFWD_UM64
+#define NS3D_XFWD_UM64 4
+#endif
+#ifndef NS3D_XFWD_RING64
+#define NS3D_XFWD_RING64 2
+#endif
+#ifndef NS3D_XFWD_RING64_8
+#define NS3D_XFWD_RING64_8 1
+#endif
+#ifndef NS3D_XFWD_UM32
+#define NS3D_XFWD_UM32 1
+#endif
+#ifndef NS3D_XFWD_RING32
+#define NS3D_XFWD_RING32 2
+#endif
+template <typename TB> constexpr int XFWD_UM = sizeof(TB) == 8 ? NS3D_XFWD_UM64 : NS3D_XFWD_UM32;
+template <typename TB, int NX, int E>
+constexpr int XFWD_RING = sizeof(TB) == 8 ? (E == 8 ? NS3D_XFWD_RING64_8 : NS3D_XFWD_RING64)
+                                          : (NX >= 256 ? 1 : NS3D_XFWD_RING32);
+template <typename TB, int NX>
+constexpr int XFWD_WAVES = sizeof(TB) == 8 ? NS3D_WAVES_XFWD64 : (NX >= 256 ? 4 : NS3D_WAVES_XFWD32);
 // x/y-pass plan: E = 8 points per thread (Plan) or 4 (ZPlan); chosen per kernel
 // and precision by the host from measurements.
 template <int N, int E> struct XYSel { using type = Plan<N>; };
@@ -106,14 +133,25 @@ __device__ __forceinline__ bool member_idle(const MemberMask& m) { return m.left
 // (w_b or dx w_b) and the input is read by two blocks.
 // TS: scalar type of the state w (double, or float for the FP32-state RK3 loop).
 // ADD = 1: the transformed field is w + w2 (w2 of the same type and layout; the
-// FP32-increment RK3 loop's stage value base + increment), summed in FP64.
+// FP32-increment RK3 loop's stage value base + increment where no x-forward pass
+// leaves P1's output), summed in FP64.
+// The plan: XYPlan, or for FP64 where the x-forward pass carries P1 too, the mirror image
+// of its plan (XInvPlan), so that both kernels give the same bits.
+template <typename TB, int NX> constexpr bool MIRROR_P1 = sizeof(TB) == 8 && NX <= 256;
+template <typename TB, int NX, int E>
+using XInvPlan = typename std::conditional<MIRROR_P1<TB, NX>, typename SeqRev<typename XYPlan<NX, E>::R>::type,
+                                           typename XYPlan<NX, E>::R>::type;
+// i kx w: the products rounded by themselves (the transform's additions must not absorb them).
+template <typename TB> __device__ __forceinline__ cplx<TB> ikx(cplx<double> s, double kx) {
+    return mk<TB>((TB)mul_rounded(-s.y, kx), (TB)mul_rounded(s.x, kx));
+}
 template <typename TB, int NX, int P, int NF, int E, int OS, typename TS = double, int ADD = 0>
 __global__ void __attribute__((amdgpu_waves_per_eu(NS3D_WAVES_XY, 8))) __launch_bounds__((P * XYPlan<NX, E>::TPP))
 k_x_inv_grad(PtrArr<const cplx<TS>, 3 * NF> w, cplx<TB>* __restrict__ A, long nc, int Ny, int Mz, int Mw, int Ms,
-             int nlt, int nb, SpecTables tab, const cplx<TB>* __restrict__ twg, long bwi = 0, long bsc = 0,
-             PtrArr<const cplx<TS>, 3> w2 = {}, MemberMask mm = {}) {
+             int nlt, int nb, SpecTables tab, const cplx<TB>* __restrict__ twg, int nt, long bwi, long bsc,
+             MemberMask mm, PtrArr<const cplx<TS>, 3> w2 = {}) {
     constexpr int TPP = XYPlan<NX, E>::TPP;
-    using F = PencilFFT<TB, NX, TPP, +1, typename XYPlan<NX, E>::R, IndexMajor<P>>;
+    using F = PencilFFT<TB, NX, TPP, +1, XInvPlan<TB, NX, E>, IndexMajor<P>>;
     __shared__ cplx<TB> lds[NX * P];
     __shared__ cplx<TB> tw[NX];
     const int bid0 = xcd_tile();
@@ -163,7 +201,7 @@ k_x_inv_grad(PtrArr<const cplx<TS>, 3 * NF> w, cplx<TB>* __restrict__ A, long nc
             cplx<double> s = cvt<double>(raw[i]);
             if constexpr (ADD != 0) s = s + cvt<double>(raw2[i]);
             const double kx = F::in_active(t, q) ? tab.kx[j] : 0.0;
-            const cplx<TB> dv = mk<TB>((TB)(-s.y * kx), (TB)(s.x * kx));
+            const cplx<TB> dv = ikx<TB>(s, kx);
             if constexpr (OS) {
                 v[q * F::R0 + r] = which ? dv : cvt<TB>(s);
             } else {
@@ -177,18 +215,18 @@ k_x_inv_grad(PtrArr<const cplx<TS>, 3 * NF> w, cplx<TB>* __restrict__ A, long nc
     cplx<TB>* __restrict__ od = A + (long)(s_ * 6 + 3 + b) * nc;
     F::run(v, lds, tw, t, p);
     if constexpr (!OS) F::run(d, lds, tw, t, p);
-    if (keep) {
+    if (keep) by_nt(nt, [&](auto NT) {
 #pragma unroll
         for (int q = 0; q < F::BL; q++) {
             if (!F::out_active(t, q)) continue;
 #pragma unroll
             for (int r = 0; r < F::RL; r++) {
                 const long g = baseo + F::out_index(t, q, r) * So;
-                ow[g] = v[q * F::RL + r];
-                if constexpr (!OS) od[g] = d[q * F::RL + r];
+                st_cplx<NT.value>(ow + g, v[q * F::RL + r]);
+                if constexpr (!OS) st_cplx<NT.value>(od + g, d[q * F::RL + r]);
             }
         }
-    }
+    });
 }
 
 // ---------------------------------------------------------------- P2
@@ -198,7 +236,7 @@ k_x_inv_grad(PtrArr<const cplx<TS>, 3 * NF> w, cplx<TB>* __restrict__ A, long nc
 template <typename TB, int NY, int P, int NF, int E, int OS>
 __global__ void __attribute__((amdgpu_waves_per_eu(NS3D_WAVES_XY, 8))) __launch_bounds__((P * XYPlan<NY, E>::TPP))
 k_y_inv_grad(const cplx<TB>* __restrict__ A, cplx<TB>* __restrict__ B, long nc, int Ny, int Mz, int Ms, int nlt,
-             int nb, SpecTables tab, const cplx<TB>* __restrict__ twg, long bsc = 0, MemberMask mm = {}) {
+             int nb, SpecTables tab, const cplx<TB>* __restrict__ twg, int nt, long bsc, MemberMask mm) {
     constexpr int TPP = XYPlan<NY, E>::TPP;
     using F = PencilFFT<TB, NY, TPP, +1, typename XYPlan<NY, E>::R, IndexMajor<P>>;
     __shared__ cplx<TB> lds[NY * P];
@@ -272,18 +310,18 @@ k_y_inv_grad(const cplx<TB>* __restrict__ A, cplx<TB>* __restrict__ B, long nc, 
         if constexpr (!OS) F::run(d, lds, tw, t, p);
         cplx<TB>* __restrict__ ow = B + (long)(s_ * 9 + (OS && which == 1 ? 6 : 0) + b) * nc;
         cplx<TB>* __restrict__ od = B + (long)(s_ * 9 + 6 + b) * nc;
-        if (lv) {
+        if (lv) by_nt(nt, [&](auto NT) {
 #pragma unroll
             for (int q = 0; q < F::BL; q++) {
                 if (!F::out_active(t, q)) continue;
 #pragma unroll
                 for (int r = 0; r < F::RL; r++) {
                     const long g = base + F::out_index(t, q, r) * S;
-                    ow[g] = v[q * F::RL + r];
-                    if constexpr (!OS) od[g] = d[q * F::RL + r];
+                    st_cplx<NT.value>(ow + g, v[q * F::RL + r]);
+                    if constexpr (!OS) st_cplx<NT.value>(od + g, d[q * F::RL + r]);
                 }
             }
-        }
+        });
     }
     // x-derivative component: plain y-inverse
     if (!OS || which == 2) {
@@ -308,14 +346,14 @@ k_y_inv_grad(const cplx<TB>* __restrict__ A, cplx<TB>* __restrict__ B, long nc, 
         if (NS3D_TW_LATE && OS) stage_twiddles<TB, NY>(tw, twg);
         F::run(v, lds, tw, t, p);
         cplx<TB>* __restrict__ ow = B + (long)(s_ * 9 + 3 + b) * nc;
-        if (lv) {
+        if (lv) by_nt(nt, [&](auto NT) {
 #pragma unroll
             for (int q = 0; q < F::BL; q++) {
                 if (!F::out_active(t, q)) continue;
 #pragma unroll
-                for (int r = 0; r < F::RL; r++) ow[base + F::out_index(t, q, r) * S] = v[q * F::RL + r];
+                for (int r = 0; r < F::RL; r++) st_cplx<NT.value>(ow + (base + F::out_index(t, q, r) * S), v[q * F::RL + r]);
             }
-        }
+        });
     }
 }
 
@@ -535,7 +573,7 @@ struct ZPencil {
     __device__ __forceinline__ static void r2c_two(const TB* q1, const TB* q2, const TB* q3, cplx<TB>* __restrict__ o1,
                                                    cplx<TB>* __restrict__ o2, cplx<TB>* __restrict__ o3, bool valid,
                                                    cplx<TB>* la, cplx<TB>* lb, const cplx<TB>* tw, int t, int p,
-                                                   const typename FI::TwReg& twr) {
+                                                   const typename FI::TwReg& twr, int nt) {
         cplx<TB> va[E], vb[E];
 #pragma unroll
         for (int e = 0; e < NPT; e++) {
@@ -556,22 +594,22 @@ struct ZPencil {
             }
         }
         exch_sync<WAVE>();
-        if (valid) {
+        if (valid) by_nt(nt, [&](auto NT) {
             for (int n = t; n <= NZ / 2; n += TPP) {
                 const cplx<TB> zn = la[LA::at(p, n)];
                 const cplx<TB> zm = la[LA::at(p, (NZ - n) % NZ)];
-                o1[n] = mk<TB>((TB)0.5 * (zn.x + zm.x), (TB)0.5 * (zn.y - zm.y));
-                o2[n] = mk<TB>((TB)0.5 * (zn.y + zm.y), (TB)0.5 * (zm.x - zn.x));
-                o3[n] = lb[LA::at(p, n)];
+                st_cplx<NT.value>(o1 + n, mk<TB>((TB)0.5 * (zn.x + zm.x), (TB)0.5 * (zn.y - zm.y)));
+                st_cplx<NT.value>(o2 + n, mk<TB>((TB)0.5 * (zn.y + zm.y), (TB)0.5 * (zm.x - zn.x)));
+                st_cplx<NT.value>(o3 + n, lb[LA::at(p, n)]);
             }
-        }
+        });
         exch_sync<WAVE>();
     }
 
     // Forward-transform (q1 + i q2) and store the two half spectra (q2 may be null).
     __device__ __forceinline__ static void r2c_pair(const TB* q1, const TB* q2, cplx<TB>* __restrict__ o1,
                                                     cplx<TB>* __restrict__ o2, bool valid, cplx<TB>* lds,
-                                                    const cplx<TB>* tw, int t, int p) {
+                                                    const cplx<TB>* tw, int t, int p, int nt = 0) {
         cplx<TB> v[E];
 #pragma unroll
         for (int e = 0; e < NPT; e++) v[e] = mk<TB>(q1[e], q2 ? q2[e] : (TB)0);
@@ -583,18 +621,18 @@ struct ZPencil {
             for (int r = 0; r < FF::RL; r++) lds[LA::at(p, FF::out_index(t, q, r))] = v[q * FF::RL + r];
         }
         exch_sync<WAVE>();
-        if (valid) {
+        if (valid) by_nt(nt, [&](auto NT) {
             for (int n = t; n <= NZ / 2; n += TPP) {
                 const cplx<TB> zn = lds[LA::at(p, n)];
                 if (q2) {
                     const cplx<TB> zm = lds[LA::at(p, (NZ - n) % NZ)];
-                    o1[n] = mk<TB>((TB)0.5 * (zn.x + zm.x), (TB)0.5 * (zn.y - zm.y));
-                    o2[n] = mk<TB>((TB)0.5 * (zn.y + zm.y), (TB)0.5 * (zm.x - zn.x));
+                    st_cplx<NT.value>(o1 + n, mk<TB>((TB)0.5 * (zn.x + zm.x), (TB)0.5 * (zn.y - zm.y)));
+                    st_cplx<NT.value>(o2 + n, mk<TB>((TB)0.5 * (zn.y + zm.y), (TB)0.5 * (zm.x - zn.x)));
                 } else {
-                    o1[n] = zn;
+                    st_cplx<NT.value>(o1 + n, zn);
                 }
             }
-        }
+        });
         exch_sync<WAVE>();
     }
 };
@@ -615,8 +653,8 @@ __global__ void __attribute__((amdgpu_waves_per_eu(NF == 1 ? (sizeof(TB) == 4 ? 
                                                           : (sizeof(TB) == 4 ? NS3D_WAVES_Z2_32 : NS3D_WAVES_Z2), 8)))
 __launch_bounds__((P * ZPlanT<TB, NZ>::TPP))
 k_z_product(const cplx<TB>* __restrict__ Bf, cplx<TB>* __restrict__ C, long nc, long npen, int Mz, int nb,
-            SpecTables tab, const cplx<TB>* __restrict__ twg, TB scale, TB* __restrict__ uphys, long nr, long bsc = 0,
-            MemberMask mm = {}) {
+            SpecTables tab, const cplx<TB>* __restrict__ twg, TB scale, TB* __restrict__ uphys, long nr, int nt, long bsc,
+            MemberMask mm) {
     // B is zero on z-planes l > lmax (never written by the y pass): TRUNC skips them
     using Z = ZPencil<TB, NZ, P, true>;
     constexpr int TPP = Z::TPP, NPT = Z::NPT;
@@ -830,10 +868,10 @@ k_z_product(const cplx<TB>* __restrict__ Bf, cplx<TB>* __restrict__ C, long nc, 
     cplx<TB>* o2 = C + 2 * nc + off;
     if constexpr (ILP) {
         Z::template r2c_two<TWR && NS3D_ZTWFWD != 0>(Q[0], Q[1], Q[2], o0, o1, o2, valid, lds, lds + P * (NZ + Z::PAD),
-                                                     tw, t, p, twi);
+                                                     tw, t, p, twi, nt);
     } else {
-        Z::r2c_pair(Q[0], Q[1], o0, o1, valid, lds, tw, t, p);
-        Z::r2c_pair(Q[2], nullptr, o2, nullptr, valid, lds, tw, t, p);
+        Z::r2c_pair(Q[0], Q[1], o0, o1, valid, lds, tw, t, p, nt);
+        Z::r2c_pair(Q[2], nullptr, o2, nullptr, valid, lds, tw, t, p, nt);
     }
 }
 
@@ -843,7 +881,7 @@ k_z_product(const cplx<TB>* __restrict__ Bf, cplx<TB>* __restrict__ C, long nc, 
 template <typename TB, int NA, int P, int DIR, int AXIS, int E>
 __global__ void __attribute__((amdgpu_waves_per_eu(NS3D_WAVES_XY, 8))) __launch_bounds__((P * XYPlan<NA, E>::TPP))
 k_axis_c2c(const cplx<TB>* in, cplx<TB>* out, int nf, long nc, int Ny, int Mz, int Ms, int nlt, int nb,
-           const cplx<TB>* __restrict__ twg, long bsc = 0, MemberMask mm = {}) {
+           const cplx<TB>* __restrict__ twg, int nt = 0, long bsc = 0, MemberMask mm = {}) {
     constexpr int TPP = XYPlan<NA, E>::TPP;
     using F = PencilFFT<TB, NA, TPP, DIR, typename XYPlan<NA, E>::R, IndexMajor<P>>;
     __shared__ cplx<TB> lds[NA * P];
@@ -876,14 +914,14 @@ k_axis_c2c(const cplx<TB>* in, cplx<TB>* out, int nf, long nc, int Ny, int Mz, i
         }
         __syncthreads();  // in-place use: every pencil element is read before any is written
         F::run(v, lds, tw, t, p);
-        if (lv) {
+        if (lv) by_nt(nt, [&](auto NT) {
 #pragma unroll
             for (int q = 0; q < F::BL; q++) {
                 if (!F::out_active(t, q)) continue;
 #pragma unroll
-                for (int r = 0; r < F::RL; r++) dst[base + F::out_index(t, q, r) * S] = v[q * F::RL + r];
+                for (int r = 0; r < F::RL; r++) st_cplx<NT.value>(dst + (base + F::out_index(t, q, r) * S), v[q * F::RL + r]);
             }
-        }
+        });
     }
 }
 
@@ -1065,14 +1103,52 @@ __device__ __forceinline__ void ipq_rule(cplx<double>& Qx, cplx<double>& Qy, cpl
     }
 }
 
-template <typename TB, int NX, int P, int MODE, int E>
-__global__ void __attribute__((amdgpu_waves_per_eu(sizeof(TB) == 4 ? NS3D_WAVES_XFWD32 : NS3D_WAVES_XY, 8))) __launch_bounds__((P * XYPlan<NX, E>::TPP))
-k_x_fwd_epi(const cplx<TB>* __restrict__ D, long nc, int Ny, int Mz, int Ms, int nlt, int nb, SpecTables tab,
-            const cplx<TB>* __restrict__ twg, EpiArgs ea, long bsc = 0, MemberMask mm = {}) {
-    constexpr int TPP = XYPlan<NX, E>::TPP;
-    using F = PencilFFT<TB, NX, TPP, -1, typename XYPlan<NX, E>::R, IndexMajor<P>>;
-    constexpr bool ILP = NS3D_HOIST && (NS3D_XFWD_ILP == 2 || (NS3D_XFWD_ILP == 1 && sizeof(TB) == 8));
-    __shared__ cplx<TB> lds[(ILP ? 2 : 1) * NX * P];
+// ---- P5 kernel: the epilogue above, its operands read ahead.
+// Scalar type of the state operands w, u0 and out in memory.
+template <int MODE>
+using EpiState = typename std::conditional<MODE == EPI_STAGE32 || MODE == EPI_INC || MODE == EPI_INC_FINAL, float,
+                                           double>::type;
+// The operands of UM consecutive modes of one component (what MODE does not read stays unused).
+template <int MODE, int UM> struct EpiUnit {
+    cplx<EpiState<MODE>> w[UM], u0[UM];
+    cplx<float> lo[UM];
+    cplx<double> f[UM];
+};
+// Wavenumber factor of x-index j, as the host table's 2*pi/Lx*m.
+template <int NX> __device__ __forceinline__ double kx_of(const SpecTables& tab, int j) {
+    return tab.kb1 * (double)(j >= NX / 2 ? j - NX : j);
+}
+
+// P5: x-forward transform and epilogue.  Bound by HBM at 256^3 and above (12 fields
+// moved in 8-mode row segments) and by the latency of its gathers below.  The state,
+// base and forcing operands are read ahead through buffer resources, UM modes of one
+// component at a time (a unit) with RING units in flight, the first ones under the
+// transforms, because loads issued mode by mode behind the stores of the mode before
+// (which may alias them) left one round trip to each of a thread's modes exposed:
+// 32^3 step 110 -> 84 us, 128^3 pass 70 -> 45 us, 256^3 0.402 -> 0.375 ms (FP64).  FP64
+// keeps 4 modes a thread (202 VGPRs, 2 waves per SIMD; 8 modes leave no room for the
+// operands and spill); from 256 points FP32 takes one unit at a time to stay under
+// 128 VGPRs (two 512-thread blocks on a CU: 0.333 -> 0.299 ms).
+//
+// CHAIN: the P1 of the next stage on the columns just updated: w^ -> M w^ and
+// M (i kx w^), both transformed back in x and written to A, so the next stage
+// starts at P2 and its P1 never reads the state.  Both precisions repeat the plan of
+// the standalone P1, so the results are bitwise its own: FP64 by the mirror image of
+// the forward plan, which starts from the values as the epilogue leaves them; FP32 by
+// the 8-point plan (EI points per thread) on half of a pencil's threads for each of the
+// two transforms, after one exchange through LDS.  256^3 FP64: 0.44 ms on average
+// against 0.185 + 0.375 for the two passes; 128^3 57 against 27 + 45 us.
+template <typename TB, int NX, int P, int MODE, int E, int CHAIN, int EI = E>
+__global__ void __attribute__((amdgpu_waves_per_eu(XFWD_WAVES<TB, NX>, 8))) __launch_bounds__((P * XYPlan<NX, E>::TPP))
+k_x_fwd_epi(const cplx<TB>* D, cplx<TB>* A, long nc, int Ny, int Mz, int Ms, int nlt, int nb, SpecTables tab,
+            const cplx<TB>* __restrict__ twg, EpiArgs ea, int nt, long bsc, MemberMask mm) {
+    using Plan_ = XYPlan<NX, E>;
+    constexpr int TPP = Plan_::TPP;
+    using F = PencilFFT<TB, NX, TPP, -1, typename Plan_::R, IndexMajor<P>>;
+    using TS = EpiState<MODE>;
+    constexpr bool F64 = sizeof(TB) == 8;
+    constexpr int NO = F::BL * F::RL;    // modes of each component a thread holds after the transform
+    __shared__ cplx<TB> lds[2 * NX * P];
     __shared__ cplx<TB> tw[NX];
     const int bid0 = xcd_tile();
     if (bid0 >= nb || member_idle(mm)) return;
@@ -1082,8 +1158,6 @@ k_x_fwd_epi(const cplx<TB>* __restrict__ D, long nc, int Ny, int Mz, int Ms, int
     const int k = bid / nlt, lt = bid % nlt;
     const int l = lt * P + p;
     const bool lv = l < Mz;
-    const long Si = (long)Ny * Ms;       // D: rows padded to Ms
-    const long basei = (long)k * Ms + l;
     if (ea.dtv) {                        // per-member time step and Reynolds number
         const double dtm = ea.dtv[blockIdx.z], rem = ea.rev[blockIdx.z];
         ea.dt = dtm;
@@ -1091,53 +1165,292 @@ k_x_fwd_epi(const cplx<TB>* __restrict__ D, long nc, int Ny, int Mz, int Ms, int
         ea.nu = 1.0 / rem;
         ea.dtnu = dtm / rem;
     }
-    if (blockIdx.z) {                    // batch member z
-        const long z = blockIdx.z;
-        D += z * bsc;
+    const long z = blockIdx.z;           // batch member
+    D += z * bsc;
+    A += z * bsc;
+    // chain: the masked modes of this thread's column, and whether any lane has some
+    unsigned kept = 0;
+    bool chained = false;
+    if constexpr (CHAIN) {
+        const bool col = lv && column_kept(tab, k, l);
+        chained = __syncthreads_or(col);
+        if (col) {
 #pragma unroll
-        for (int b = 0; b < 3; b++) {
-            ea.w[b] += z * ea.bw;
-            if (ea.u0[b]) ea.u0[b] += z * ea.bu0;
-            ea.out[b] += z * ea.bo;
-        }
-    }
-    cplx<TB> qv[3][F::E];
-    // the three components are all live until the epilogue: load them together
-#pragma unroll
-    for (int b = 0; b < 3; b++) {
-        const cplx<TB>* src = D + (long)b * nc;
-#pragma unroll
-        for (int q = 0; q < F::B0; q++) {
-#pragma unroll
-            for (int r = 0; r < F::R0; r++) {
-                cplx<TB> s = mk<TB>(0, 0);
-                if (F::in_active(t, q) && lv) s = src[basei + F::in_index(t, q, r) * Si];
-                qv[b][q * F::R0 + r] = s;
+            for (int e = 0; e < NO; e++) {
+                const int q = e / F::RL, j = F::out_index(t, q, e % F::RL);
+                if (F::out_active(t, q) && mask_keep(tab, j, k, l)) kept |= 1u << e;
             }
         }
-        if (!NS3D_HOIST) F::run(qv[b], lds, tw, t, p);
     }
-    if constexpr (ILP) {
-        F::run2(qv[0], qv[1], lds, lds + NX * P, tw, t, p);
-        F::run(qv[2], lds, tw, t, p);
-    } else if (NS3D_HOIST) {
+    // D: this thread's elements, plane stride Ny*Ms
+    const int strD = Ny * Ms * (int)sizeof(cplx<TB>);
+    const int offD = lv ? (k * Ms + l) * (int)sizeof(cplx<TB>) : BUF_OOB;
+    const int bytesD = (int)(nc * (long)sizeof(cplx<TB>));
+    cplx<TB> qv[3][F::E];
 #pragma unroll
-        for (int b = 0; b < 3; b++) F::run(qv[b], lds, tw, t, p);
-    }
-    if (!lv) return;
+    for (int b = 0; b < 3; b++) {
+        const auto src = buf_rsrc(D + (long)b * nc, bytesD);
 #pragma unroll
-    for (int q = 0; q < F::BL; q++) {
-        if (!F::out_active(t, q)) continue;
+        for (int q = 0; q < F::B0; q++) {
+            const int o = F::in_active(t, q) ? offD + t * strD : BUF_OOB;
 #pragma unroll
-        for (int r = 0; r < F::RL; r++) {
-            const int j = F::out_index(t, q, r);
-            cplx<double> Qx = cvt<double>(qv[0][q * F::RL + r]);
-            cplx<double> Qy = cvt<double>(qv[1][q * F::RL + r]);
-            cplx<double> Qz = cvt<double>(qv[2][q * F::RL + r]);
-            ipq_rule(Qx, Qy, Qz, ea.ipq, (j | k | l) == 0);
-            epilogue<MODE>(ea, tab, j, k, l, Qx, Qy, Qz);
+            for (int r = 0; r < F::R0; r++)
+                qv[b][q * F::R0 + r] = buf_load<TB>(src, lv ? o : BUF_OOB, (F::in_index(0, q, r)) * strD);
         }
     }
+    // ---- operands: unit u = modes e0..e0+UM-1 of component b, u = b*UPC + e0/UM
+    constexpr int UM = XFWD_UM<TB> < NO ? XFWD_UM<TB> : NO;
+    constexpr int UPC = NO / UM, NU = 3 * UPC;
+    static_assert(NO % UM == 0, "units cover a component");
+    constexpr int RING = XFWD_RING<TB, NX, E> < NU ? XFWD_RING<TB, NX, E> : NU;
+    constexpr bool HAS_U0 = MODE == EPI_STAGE || MODE == EPI_STAGE32 || MODE == EPI_INC || MODE == EPI_INC_FINAL;
+    constexpr bool HAS_F = HAS_U0 || MODE == EPI_RHS;
+    EpiUnit<MODE, UM> un[RING];
+    const long nrow = (long)NX * Ny;
+    auto rsrc_of = [&](const void* ptr, long shift, int m, int esz) __attribute__((always_inline)) {
+        return buf_rsrc((const char*)ptr + shift * esz, (int)(nrow * m * esz));
+    };
+    auto voff = [&](int m, int esz, int q) __attribute__((always_inline)) {
+        return lv && F::out_active(t, q) ? ((t * Ny + k) * m + l) * esz : BUF_OOB;
+    };
+    auto load_unit = [&](auto UC) __attribute__((always_inline)) {
+        constexpr int u = decltype(UC)::value, b = u / UPC, e0 = (u % UPC) * UM;
+        EpiUnit<MODE, UM>& U = un[u % RING];
+        constexpr int es = (int)sizeof(cplx<TS>);
+        const auto rw = rsrc_of(ea.w[b], z * ea.bw, ea.mw, es);
+#pragma unroll
+        for (int i = 0; i < UM; i++) {
+            const int e = e0 + i;
+            const int q = e / F::RL, so = F::out_index(0, q, e % F::RL) * Ny;
+            if constexpr (MODE != EPI_Q) U.w[i] = buf_load<TS>(rw, voff(ea.mw, es, q), so * ea.mw * es);
+        }
+        if constexpr (HAS_U0) {
+            if (ea.u0[b]) {
+                const auto ru = rsrc_of(ea.u0[b], z * ea.bu0, ea.mu0, es);
+#pragma unroll
+                for (int i = 0; i < UM; i++) {
+                    const int e = e0 + i;
+                    const int q = e / F::RL, so = F::out_index(0, q, e % F::RL) * Ny;
+                    U.u0[i] = buf_load<TS>(ru, voff(ea.mu0, es, q), so * ea.mu0 * es);
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < UM; i++) U.u0[i] = mk<TS>(0, 0);
+            }
+        }
+        if constexpr (MODE == EPI_INC_FINAL) {
+            const auto rl = rsrc_of(ea.out32[b], 0, ea.mw, es);
+#pragma unroll
+            for (int i = 0; i < UM; i++) {
+                const int e = e0 + i;
+                const int q = e / F::RL, so = F::out_index(0, q, e % F::RL) * Ny;
+                U.lo[i] = buf_load<float>(rl, voff(ea.mw, es, q), so * ea.mw * es);
+            }
+        }
+        if constexpr (HAS_F) {
+            if (ea.f[b]) {
+                const auto rf = rsrc_of(ea.f[b], 0, ea.mf, 16);
+#pragma unroll
+                for (int i = 0; i < UM; i++) {
+                    const int e = e0 + i;
+                    const int q = e / F::RL, so = F::out_index(0, q, e % F::RL) * Ny;
+                    U.f[i] = buf_load<double>(rf, voff(ea.mf, 16, q), so * ea.mf * 16);
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < UM; i++) U.f[i] = mk<double>(0.0, 0.0);
+            }
+        }
+    };
+    // the first RING - 1 units are in flight while the transforms run
+    if constexpr (MODE != EPI_Q) static_for<0, RING - 1>([&](auto UC) __attribute__((always_inline)) { load_unit(UC); });
+    F::run2(qv[0], qv[1], lds, lds + NX * P, tw, t, p);
+    F::run(qv[2], lds, tw, t, p);
+    const double ky = tab.ky[k], kz = lv ? tab.kz[l] : 0.0;
+    const double kyz2 = ky * ky + kz * kz;
+    // projection: AM Q - Q with AM Q = kv (kv.Q)/|k|^2.  FP64: R replaces Q;
+    // FP32: Q stays in FP32 and kd = (kv.Q)/|k|^2 is kept in FP64.
+    cplx<double> kd[(F64 || MODE == EPI_Q) ? 1 : NO];
+    const double qs = MODE == EPI_RHS || MODE == EPI_UV_RHS ? 1.0 : ea.dt;   // weight of (AM Q - Q)
+#pragma unroll
+    for (int e = 0; e < NO; e++) {
+        const int j = F::out_index(t, e / F::RL, e % F::RL);
+        cplx<double> Q[3] = {cvt<double>(qv[0][e]), cvt<double>(qv[1][e]), cvt<double>(qv[2][e])};
+        ipq_rule(Q[0], Q[1], Q[2], ea.ipq, (j | k | l) == 0);
+        if constexpr (MODE == EPI_Q) {
+#pragma unroll
+            for (int b = 0; b < 3; b++) qv[b][e] = cvt<TB>(Q[b]);
+        } else {
+            const double kx = kx_of<NX>(tab, j);
+            const double k2 = kx * kx + kyz2;
+            const double inv = (j | k | l) == 0 ? 0.0 : 1.0 / k2;
+            cplx<double> d;
+            d.x = (kx * Q[0].x + ky * Q[1].x + kz * Q[2].x) * inv;
+            d.y = (kx * Q[0].y + ky * Q[1].y + kz * Q[2].y) * inv;
+            const double kv[3] = {kx, ky, kz};
+            if constexpr (F64) {
+#pragma unroll
+                for (int b = 0; b < 3; b++) qv[b][e] = mk<TB>(qs * (kv[b] * d.x - Q[b].x), qs * (kv[b] * d.y - Q[b].y));
+            } else {
+                kd[e] = d;
+#pragma unroll
+                for (int b = 0; b < 3; b++) qv[b][e] = cvt<TB>(Q[b]);   // after the IPQ rule
+            }
+        }
+    }
+    // chain: inverse transforms of one component's w and dx w, stored to A
+    auto chain = [&](int b, cplx<TB>* v, cplx<TB>* d) __attribute__((always_inline)) {
+        const bool col = lv && column_kept(tab, k, l);
+        auto put = [&](auto FC, cplx<TB>* x, int field, int ti) __attribute__((always_inline)) {
+            using FX = decltype(FC);
+            const auto ra = buf_rsrc(A + (long)field * nc, bytesD);
+            by_nt(nt, [&](auto NT) __attribute__((always_inline)) {
+#pragma unroll
+                for (int q = 0; q < FX::BL; q++) {
+                    const int o = col && FX::out_active(ti, q) ? offD + ti * strD : BUF_OOB;
+#pragma unroll
+                    for (int r = 0; r < FX::RL; r++)
+                        buf_store<TB, NT.value>(ra, x[q * FX::RL + r], o, FX::out_index(0, q, r) * strD);
+                }
+            });
+        };
+        if constexpr (F64) {
+            // the mirror-image plan: its first pass reads what the last forward pass holds
+            static_assert(!CHAIN || MIRROR_P1<TB, NX>, "the standalone P1 runs the same plan");
+            using FI = PencilFFT<TB, NX, TPP, +1, XInvPlan<TB, NX, E>, IndexMajor<P>>;
+            FI::run2(v, d, lds, lds + NX * P, tw, t, p);
+            put(FI{}, v, b, t);
+            put(FI{}, d, 3 + b, t);
+        } else {
+            // the standalone P1's plan on half the threads for each transform
+            constexpr int TPI = XYPlan<NX, EI>::TPP;
+            static_assert(!CHAIN || TPP == 2 * TPI, "half of a pencil's threads run each of its two inverse transforms");
+            using FI = PencilFFT<TB, NX, TPI, +1, typename XYPlan<NX, EI>::R, IndexMajor<P>>;
+#pragma unroll
+            for (int e = 0; e < NO; e++) {
+                const int q = e / F::RL, j = F::out_index(t, q, e % F::RL);
+                if (!F::out_active(t, q)) continue;
+                lds[j * P + p] = v[e];
+                lds[NX * P + j * P + p] = d[e];
+            }
+            __syncthreads();
+            const int h = t >= TPI ? 1 : 0, ti = t - h * TPI;
+            cplx<TB>* half = lds + h * NX * P;
+            cplx<TB> x[FI::E];
+#pragma unroll
+            for (int q = 0; q < FI::B0; q++) {
+                if (!FI::in_active(ti, q)) continue;
+#pragma unroll
+                for (int r = 0; r < FI::R0; r++) x[q * FI::R0 + r] = half[FI::in_index(ti, q, r) * P + p];
+            }
+            __syncthreads();
+            FI::run(x, half, tw, ti, p);
+            cplx<TB>* dst = A + (long)(b + 3 * h) * nc + ((long)k * Ms + l);
+            const long str = (long)Ny * Ms;
+            if (col) by_nt(nt, [&](auto NT) __attribute__((always_inline)) {
+#pragma unroll
+                for (int q = 0; q < FI::BL; q++) {
+                    if (!FI::out_active(ti, q)) continue;
+#pragma unroll
+                    for (int r = 0; r < FI::RL; r++) st_cplx<NT.value>(dst + FI::out_index(ti, q, r) * str, x[q * FI::RL + r]);
+                }
+            });
+        }
+    };
+    bool bad = false;
+    cplx<TB> cv[CHAIN ? F::E : 1], cd[CHAIN ? F::E : 1];   // (F::E: also the mirror-image plan's registers)
+    static_for<0, NU>([&](auto UC) __attribute__((always_inline)) {
+        constexpr int u = decltype(UC)::value, b = u / UPC, e0 = (u % UPC) * UM;
+        if constexpr (MODE != EPI_Q && u + RING - 1 < NU) load_unit(std::integral_constant<int, u + RING - 1>{});
+        const EpiUnit<MODE, UM>& U = un[u % RING];
+        constexpr int es = (int)sizeof(cplx<TS>);
+        // UV, UV_RHS and IUV update w in place
+        constexpr bool INPLACE = MODE == EPI_UV || MODE == EPI_UV_RHS || MODE == EPI_IUV || MODE == EPI_INC_FINAL;
+        const int mo = INPLACE ? ea.mw : ea.mo;
+        const auto ro = rsrc_of(INPLACE ? ea.w[b] : ea.out[b], INPLACE ? z * ea.bw : z * ea.bo, mo, es);
+#pragma unroll
+        for (int i = 0; i < UM; i++) {
+            const int e = e0 + i;
+            const int q = e / F::RL, jo = F::out_index(0, q, e % F::RL), j = t + jo;
+            const int vo = voff(mo, es, q), so = jo * Ny * mo * es;
+            if constexpr (MODE == EPI_Q) {
+                const cplx<double> r = cvt<double>(qv[b][e]);
+                buf_store<double>(ro, r, vo, so);
+                bad |= vo >= 0 && !finite2(r);
+                continue;
+            } else {
+                const double kx = kx_of<NX>(tab, j);
+                const double k2 = kx * kx + kyz2;
+                cplx<double> R;
+                if constexpr (F64) {
+                    R = qv[b][e];
+                } else {
+                    const double kb = b == 0 ? kx : (b == 1 ? ky : kz);
+                    const cplx<double> Q = cvt<double>(qv[b][e]);
+                    R = mk<double>(qs * (kb * kd[e].x - Q.x), qs * (kb * kd[e].y - Q.y));
+                }
+                cplx<double> r, w = cvt<double>(U.w[i]);
+                cplx<TS> keepv = mk<TS>(0, 0);   // the stage value as written
+                if constexpr (MODE == EPI_STAGE || MODE == EPI_STAGE32) {
+                    const double G = 1.0 - k2 * ea.dtnu;
+                    r.x = R.x + G * w.x + ea.dt * U.f[i].x;
+                    r.y = R.y + G * w.y + ea.dt * U.f[i].y;
+                    r.x = ea.a0 * (double)U.u0[i].x + ea.a1 * r.x;
+                    r.y = ea.a0 * (double)U.u0[i].y + ea.a1 * r.y;
+                    keepv = cvt<TS>(r);
+                    buf_store<TS>(ro, keepv, vo, so);
+                    bad |= vo >= 0 && !finite2(keepv);
+                } else if constexpr (MODE == EPI_INC || MODE == EPI_INC_FINAL) {
+                    cplx<double> base = w;
+                    if constexpr (MODE == EPI_INC_FINAL) base = base + cvt<double>(U.lo[i]);
+                    const cplx<double> d = cvt<double>(U.u0[i]);
+                    const double Gd = k2 * ea.dtnu;
+                    r.x = ea.a1 * (d.x + (R.x - Gd * (base.x + d.x) + ea.dt * U.f[i].x));
+                    r.y = ea.a1 * (d.y + (R.y - Gd * (base.y + d.y) + ea.dt * U.f[i].y));
+                    if constexpr (MODE == EPI_INC) {
+                        keepv = cvt<TS>(r);
+                        buf_store<TS>(ro, keepv, vo, so);
+                        bad |= vo >= 0 && !finite2(keepv);
+                    } else {
+                        r = r + base;
+                        keepv = cvt<TS>(r);
+                        buf_store<TS>(ro, keepv, vo, so);
+                        buf_store<float>(rsrc_of(ea.out32[b], 0, ea.mw, es),
+                                         mk<float>((float)(r.x - (double)keepv.x), (float)(r.y - (double)keepv.y)), vo, so);
+                        bad |= vo >= 0 && !finite2(r);
+                    }
+                } else if constexpr (MODE == EPI_RHS || MODE == EPI_UV_RHS) {
+                    const double G = -k2 * ea.nu;
+                    r.x = R.x + G * w.x;
+                    r.y = R.y + G * w.y;
+                    if constexpr (MODE == EPI_RHS) r = r + U.f[i];
+                    buf_store<double>(ro, r, vo, so);
+                    bad |= vo >= 0 && !finite2(r);
+                } else if constexpr (MODE == EPI_UV) {
+                    const double G = 1.0 - k2 * ea.dtnu;
+                    r = mk<double>(R.x + G * w.x, R.y + G * w.y);
+                    buf_store<double>(ro, r, vo, so);
+                    bad |= vo >= 0 && !finite2(r);
+                } else {  // EPI_IUV
+                    const double G = 1.0 + k2 * ea.dtnu;
+                    r = mk<double>((w.x + R.x) / G, (w.y + R.y) / G);
+                    buf_store<double>(ro, r, vo, so);
+                    bad |= vo >= 0 && !finite2(r);
+                }
+                if constexpr (CHAIN) {
+                    cplx<double> s = cvt<double>(keepv);
+                    if constexpr (MODE == EPI_INC) s = w + s;   // base + increment
+                    if (!(kept >> e & 1u)) s = mk<double>(0.0, 0.0);
+                    cv[e] = cvt<TB>(s);
+                    cd[e] = ikx<TB>(s, kx);
+                }
+            }
+        }
+        if constexpr (CHAIN && u % UPC == UPC - 1) {
+            if (chained) chain(b, cv, cd);
+        }
+    });
+    flag_nonfinite(ea.nf, bad);
 }
 
 // Pointwise epilogue from stored Q^ (the standalone solve_advection_diffusion_projection*).
@@ -1151,6 +1464,65 @@ k_update(const cplx<double>* __restrict__ Qx, const cplx<double>* __restrict__ Q
     const long t1 = g / Mz;
     const int k = (int)(t1 % Ny), j = (int)(t1 / Ny);
     epilogue<MODE>(ea, tab, j, k, l, Qx[g], Qy[g], Qz[g]);
+}
+
+// ---------------------------------------------------------------- z C2R / R2C (single fields)
+// Two neighbouring (x,y) pencils share one complex FFT: Y = X_p0 + i X_p1.
+template <typename TB, int NZ, int P>
+__global__ void __launch_bounds__((P * ZPlanT<TB, NZ>::TPP))
+k_z_c2r(const cplx<TB>* __restrict__ in, TB* __restrict__ out, long npairs, int Mz, int nb, SpecTables tab,
+        const cplx<TB>* __restrict__ twg, TB scale) {
+    using Z = ZPencil<TB, NZ, P>;
+    constexpr int TPP = Z::TPP;
+    __shared__ cplx<TB> lds[P * (NZ + Z::PAD)];
+    __shared__ cplx<TB> tw[NZ];
+    const int bid = xcd_tile();
+    if (bid >= nb) return;
+    stage_twiddles<TB, NZ>(tw, twg);
+    const int tid = threadIdx.x, t = tid % TPP, p = tid / TPP;
+    const long pair = (long)bid * P + p;
+    const bool valid = pair < npairs;
+    const long p0 = valid ? 2 * pair : 0, p1 = p0 + 1;
+    TB x1[Z::NPT], x2[Z::NPT];
+    Z::c2r_pair(x1, x2, in + p0 * Mz, false, in + p1 * Mz, false, valid, tab, lds, tw, t, p, scale);
+    if (!valid) return;
+#pragma unroll
+    for (int q = 0; q < Z::FI::BL; q++) {
+#pragma unroll
+        for (int r = 0; r < Z::FI::RL; r++) {
+            const int n = Z::FI::out_index(t, q, r);
+            out[p0 * NZ + n] = x1[q * Z::FI::RL + r];
+            out[p1 * NZ + n] = x2[q * Z::FI::RL + r];
+        }
+    }
+}
+
+template <typename TB, int NZ, int P>
+__global__ void __launch_bounds__((P * ZPlanT<TB, NZ>::TPP))
+k_z_r2c(const TB* __restrict__ in, cplx<TB>* __restrict__ out, long npairs, int Mz, int nb,
+        const cplx<TB>* __restrict__ twg) {
+    using Z = ZPencil<TB, NZ, P>;
+    constexpr int TPP = Z::TPP;
+    __shared__ cplx<TB> lds[P * (NZ + Z::PAD)];
+    __shared__ cplx<TB> tw[NZ];
+    const int bid = xcd_tile();
+    if (bid >= nb) return;
+    stage_twiddles<TB, NZ>(tw, twg);
+    const int tid = threadIdx.x, t = tid % TPP, p = tid / TPP;
+    const long pair = (long)bid * P + p;
+    const bool valid = pair < npairs;
+    const long p0 = valid ? 2 * pair : 0, p1 = p0 + 1;
+    TB q1[Z::NPT], q2[Z::NPT];
+#pragma unroll
+    for (int q = 0; q < Z::FF::B0; q++) {
+#pragma unroll
+        for (int r = 0; r < Z::FF::R0; r++) {
+            const int n = Z::FF::in_index(t, q, r);
+            q1[q * Z::FF::R0 + r] = valid ? in[p0 * NZ + n] : (TB)0;
+            q2[q * Z::FF::R0 + r] = valid ? in[p1 * NZ + n] : (TB)0;
+        }
+    }
+    Z::r2c_pair(q1, q2, out + p0 * Mz, out + p1 * Mz, valid, lds, tw, t, p);
 }
 
 }  // namespace ns3d

@@ -1,67 +1,8 @@
-// k_misc.hpp -- standalone transforms, pointwise operators, WENO, reductions.
+// k_misc.hpp -- precision conversion, pointwise operators, WENO, reductions.
 #pragma once
 #include "k_fused.hpp"
 
 namespace ns3d {
-
-// ------------------------------------------------------- z C2R / R2C (single fields)
-// Two neighbouring (x,y) pencils share one complex FFT: Y = X_p0 + i X_p1.
-template <typename TB, int NZ, int P>
-__global__ void __launch_bounds__((P * ZPlanT<TB, NZ>::TPP))
-k_z_c2r(const cplx<TB>* __restrict__ in, TB* __restrict__ out, long npairs, int Mz, int nb, SpecTables tab,
-        const cplx<TB>* __restrict__ twg, TB scale) {
-    using Z = ZPencil<TB, NZ, P>;
-    constexpr int TPP = Z::TPP;
-    __shared__ cplx<TB> lds[P * (NZ + Z::PAD)];
-    __shared__ cplx<TB> tw[NZ];
-    const int bid = xcd_tile();
-    if (bid >= nb) return;
-    stage_twiddles<TB, NZ>(tw, twg);
-    const int tid = threadIdx.x, t = tid % TPP, p = tid / TPP;
-    const long pair = (long)bid * P + p;
-    const bool valid = pair < npairs;
-    const long p0 = valid ? 2 * pair : 0, p1 = p0 + 1;
-    TB x1[Z::NPT], x2[Z::NPT];
-    Z::c2r_pair(x1, x2, in + p0 * Mz, false, in + p1 * Mz, false, valid, tab, lds, tw, t, p, scale);
-    if (!valid) return;
-#pragma unroll
-    for (int q = 0; q < Z::FI::BL; q++) {
-#pragma unroll
-        for (int r = 0; r < Z::FI::RL; r++) {
-            const int n = Z::FI::out_index(t, q, r);
-            out[p0 * NZ + n] = x1[q * Z::FI::RL + r];
-            out[p1 * NZ + n] = x2[q * Z::FI::RL + r];
-        }
-    }
-}
-
-template <typename TB, int NZ, int P>
-__global__ void __launch_bounds__((P * ZPlanT<TB, NZ>::TPP))
-k_z_r2c(const TB* __restrict__ in, cplx<TB>* __restrict__ out, long npairs, int Mz, int nb,
-        const cplx<TB>* __restrict__ twg) {
-    using Z = ZPencil<TB, NZ, P>;
-    constexpr int TPP = Z::TPP;
-    __shared__ cplx<TB> lds[P * (NZ + Z::PAD)];
-    __shared__ cplx<TB> tw[NZ];
-    const int bid = xcd_tile();
-    if (bid >= nb) return;
-    stage_twiddles<TB, NZ>(tw, twg);
-    const int tid = threadIdx.x, t = tid % TPP, p = tid / TPP;
-    const long pair = (long)bid * P + p;
-    const bool valid = pair < npairs;
-    const long p0 = valid ? 2 * pair : 0, p1 = p0 + 1;
-    TB q1[Z::NPT], q2[Z::NPT];
-#pragma unroll
-    for (int q = 0; q < Z::FF::B0; q++) {
-#pragma unroll
-        for (int r = 0; r < Z::FF::R0; r++) {
-            const int n = Z::FF::in_index(t, q, r);
-            q1[q * Z::FF::R0 + r] = valid ? in[p0 * NZ + n] : (TB)0;
-            q2[q * Z::FF::R0 + r] = valid ? in[p1 * NZ + n] : (TB)0;
-        }
-    }
-    Z::r2c_pair(q1, q2, out + p0 * Mz, out + p1 * Mz, valid, lds, tw, t, p);
-}
 
 // ------------------------------------------------------- precision conversion
 __global__ void k_d2f_c(const cplx<double>* __restrict__ in, cplx<float>* __restrict__ out, long n) {

@@ -1,5 +1,6 @@
 // ns3d_api.hip -- context, launch plumbing and the extern "C" entry points of
-// include/ns3d.h.  One translation unit; compiled for gfx950 only.
+// include/ns3d.h; compiled for gfx950 only.  The kernels and launches of each grid
+// length are in ns3d_len.hip.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -8,24 +9,15 @@
 #include <cstring>
 #include <mutex>
 #include <new>
-#include <type_traits>
 #include <vector>
 
-#include "../../include/ns3d.h"
-// tile shapes and plans chosen by ns3dperiodic_amd/autotune.py; the #ifndef
-// defaults in the kernel headers apply to whatever it does not set
-#if !defined(NS3D_NO_TUNED_HEADER) && __has_include("tuned.hpp")
-#include "tuned.hpp"
-#endif
+#include "launch.hpp"
 #include "k_misc.hpp"
 #include "k_krylov.hpp"
 #include "k_diag.hpp"
 
-using namespace ns3d;
 
 namespace {
-
-typedef cplx<double> zd;
 
 template <class F>
 int with_size(int n, F&& f) {
@@ -53,106 +45,6 @@ bool size_ok(int n) {
            n == 192 || n == 256 || n == 320 || n == 384 || n == 512;
 }
 
-// pencils per block in the x/y passes: rows of 128 B
-#ifndef NS3D_PXY32
-#define NS3D_PXY32 16
-#endif
-template <typename TB> constexpr int PXY0 = sizeof(TB) == 8 ? 8 : NS3D_PXY32;
-// Blocks are capped at NS3D_XY_MAXT threads: 1024-thread blocks, which fill
-// a CU's 16 waves with one block, lose to 512 (measured at 256^3 and 512^3).
-#ifndef NS3D_XY_MAXT
-#define NS3D_XY_MAXT 512
-#endif
-template <typename TB, int N, int E>
-constexpr int PXY = PXY0<TB> * XYPlan<N, E>::TPP <= NS3D_XY_MAXT ? PXY0<TB>
-                                                                 : (NS3D_XY_MAXT / XYPlan<N, E>::TPP > 0 ? NS3D_XY_MAXT / XYPlan<N, E>::TPP : 1);
-// Pencils per block of each fused x/y pass, by precision.
-#ifndef NS3D_PXINV32
-#define NS3D_PXINV32 8
-#endif
-#ifndef NS3D_PYINV32
-#define NS3D_PYINV32 8
-#endif
-#ifndef NS3D_PYFWD32
-#define NS3D_PYFWD32 16
-#endif
-#ifndef NS3D_PXFWD32
-#define NS3D_PXFWD32 8
-#endif
-#ifndef NS3D_PXINV64
-#define NS3D_PXINV64 8
-#endif
-#ifndef NS3D_PYINV64
-#define NS3D_PYINV64 8
-#endif
-template <typename TB, int N, int E, int P32, int P64>
-constexpr int PXY_T = (sizeof(TB) == 8 ? P64 : P32) * XYPlan<N, E>::TPP <= NS3D_XY_MAXT
-                          ? (sizeof(TB) == 8 ? P64 : P32)
-                          : (NS3D_XY_MAXT / XYPlan<N, E>::TPP > 0 ? NS3D_XY_MAXT / XYPlan<N, E>::TPP : 1);
-// Points per thread of each x/y pass, by precision (measured at 256^3 on MI355X):
-// FP64 favours 4 points in the inverse passes, 8 in the forward ones; FP32 the mix below.
-#ifndef NS3D_EXINV32
-#define NS3D_EXINV32 8
-#endif
-#ifndef NS3D_EYINV32
-#define NS3D_EYINV32 4
-#endif
-#ifndef NS3D_EXINV64
-#define NS3D_EXINV64 4
-#endif
-#ifndef NS3D_EYINV64
-#define NS3D_EYINV64 4
-#endif
-#ifndef NS3D_EXFWD64
-#define NS3D_EXFWD64 8
-#endif
-template <typename TB> constexpr int E_XINV = sizeof(TB) == 8 ? NS3D_EXINV64 : NS3D_EXINV32;
-template <typename TB> constexpr int E_YINV = sizeof(TB) == 8 ? NS3D_EYINV64 : NS3D_EYINV32;
-template <typename TB> constexpr int E_C2C = 8;
-#ifndef NS3D_EXFWD32
-#define NS3D_EXFWD32 4
-#endif
-template <typename TB> constexpr int E_XFWD = sizeof(TB) == 8 ? NS3D_EXFWD64 : NS3D_EXFWD32;
-// one output field per block in the inverse passes (input re-read by 2 or 3 blocks)
-#ifndef NS3D_OS_XINV
-#define NS3D_OS_XINV 0
-#endif
-#ifndef NS3D_OS_YINV
-#define NS3D_OS_YINV 0
-#endif
-// pencils per block in the z pass: ~128 threads (FP32: NS3D_PZT32)
-#ifndef NS3D_PZT32
-#define NS3D_PZT32 128
-#endif
-// (measured: smaller blocks beat whole-wavefront ones, e.g. 96 vs 192 threads at 192^3)
-#ifndef NS3D_PZT64
-#define NS3D_PZT64 128
-#endif
-// Radix-3 lengths from 192 up have their own block shapes (NS3D_R3_*, and
-// NS3D_R3_ZSWZ in the z pass), swept at 192^3 (FP64 366 -> 419, FP32 680 ->
-// 700, FP32 state 725 -> 768 steps/s); at 48 and 96 these shapes were slower
-// than the ones above (swept at 256^3), which those lengths keep.
-#ifndef NS3D_R3_PXINV64
-#define NS3D_R3_PXINV64 4
-#endif
-#ifndef NS3D_R3_PYINV64
-#define NS3D_R3_PYINV64 4
-#endif
-#ifndef NS3D_R3_PZT64
-#define NS3D_R3_PZT64 256
-#endif
-#ifndef NS3D_R3_PXFWD32
-#define NS3D_R3_PXFWD32 16
-#endif
-#ifndef NS3D_R3_PYINV32
-#define NS3D_R3_PYINV32 4
-#endif
-#define NS3D_BY_RADIX(N, A, R3) ((N) % 3 == 0 && (N) >= 192 ? (R3) : (A))
-template <typename TB, int N>
-constexpr int PZT = sizeof(TB) == 8 ? NS3D_BY_RADIX(N, NS3D_PZT64, NS3D_R3_PZT64) : NS3D_PZT32;
-template <typename TB, int N>
-constexpr int PZ = (PZT<TB, N> / ZPlanT<TB, N>::TPP) > 0 ? (PZT<TB, N> / ZPlanT<TB, N>::TPP) : 1;
-
 #define HIPCHK(x)                                         \
     do {                                                  \
         hipError_t e_ = (x);                              \
@@ -166,87 +58,6 @@ constexpr int PZ = (PZT<TB, N> / ZPlanT<TB, N>::TPP) > 0 ? (PZT<TB, N> / ZPlanT<
 // symbol for hipGetSymbolAddress, never an address (see scratch_ptr).
 constexpr size_t NS3D_NOALLOC_SCRATCH_BYTES = (size_t)64 << 20;
 static __device__ __align__(256) unsigned char scratch[NS3D_NOALLOC_SCRATCH_BYTES];
-
-struct ns3d_ctx {
-    int Nx, Ny, Nz, Mz;
-    long nc, nr, npen;
-    long nci;  // modes per scratch field of the fused passes (rows padded from Mz to mi_of(c))
-    int m8, m16;     // Mz rounded up to a multiple of NS3D_ROWPAD64 / NS3D_ROWPAD32 (FP64 / FP32 rows)
-    long nc8, nc16;  // Nx*Ny*m8, Nx*Ny*m16
-    double Lx, Ly, Lz, Re, dt;
-    int precision;
-    unsigned flags;
-    hipStream_t stream;
-    int device;
-    int last_error;
-    // device tables
-    double* dtab = nullptr;
-    SpecTables tab;
-    void* tw64[3] = {nullptr, nullptr, nullptr};  // x, y, z twiddles (double)
-    void* tw32[3] = {nullptr, nullptr, nullptr};  // (float)
-    // bulk scratch (A|B regions) in bulk precision; capacity in fields
-    void* scratch = nullptr;
-    int scratch_fields = 0;
-    // incremented whenever a buffer that a captured RK3 step addresses is reallocated
-    long long generation = 0;
-    // FP64 stage buffers and a Q^ buffer
-    zd* stage = nullptr;  // 9 fields: u1[3], u2[3], q[3]
-    zd* extra = nullptr;  // 6 fields: tangent map v1[3] + spare
-    cplx<float>* s32 = nullptr;  // NS3D_FP32_STATE RK3 loop: state[3], u1[3], u2[3] in FP32
-    double* red = nullptr;  // reduction partials (2*RED_BLOCKS + 2)
-    double* red_host = nullptr;  // pinned
-    void* real_scratch = nullptr;  // physical-space scratch (FP64 or FP32), 4 fields
-    // registered base flow for the Krylov callbacks
-    zd* base[3] = {nullptr, nullptr, nullptr};
-    const zd* bforce[3] = {nullptr, nullptr, nullptr};
-    int timesteps_period = 1;
-    double tau = 1.0;
-    zd* kry = nullptr;  // 3 fields for J.v unpacking
-    // Krylov vector kernels: reduction partials, results, pinned host copies, small dense matrix
-    double* kv_partial = nullptr;
-    double* kv_out = nullptr;
-    double* kv_host = nullptr;
-    double* kq = nullptr;
-    double* kq_host = nullptr;
-    // a captured graph of nsteps RK3 steps for fixed state/forcing pointers, dt and Re
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t graph_exec = nullptr;
-    const void* graph_key[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-    int graph_steps = -1;
-    double graph_dt = 0.0, graph_Re = 0.0;
-    // passive scalar: physical velocity written by the z pass (bulk precision, 3 real fields)
-    void* uphys = nullptr;
-    void* uphys_out = nullptr;  // non-null only while a scalar step wants it
-    double* theta_stage = nullptr;  // 2 real FP64 fields
-    // batches of same-size fields advanced by one set of launches (grid.z = member):
-    // members in flight, scratch stride per member (elements), stage buffers per member
-    int batch = 1;
-    long bsc = 0;
-    zd* bstage = nullptr;  // batch members' u1[3], u2[3]: 6 fields of nc8 each per member
-    int bstage_members = 0;
-    // members sitting out steps, and per-member dt / Re (ns3d_rk3_ssp_batch_members)
-    MemberMask mm = {nullptr, 0};
-    const double* mdt = nullptr;
-    const double* mre = nullptr;
-    // graph of ns3d_rk3_ssp_batch_members for fixed pointers, nbatch and nsteps
-    hipGraph_t mgraph = nullptr;
-    hipGraphExec_t mgraph_exec = nullptr;
-    const void* mgraph_key[8] = {};
-    int mgraph_nb = -1, mgraph_steps = -1;
-    // optional per-pass timing with HIP events on the context stream
-    bool prof_on = false;
-    std::vector<hipEvent_t> ev_pool;
-    std::vector<std::pair<int, int>> ev_used;  // (pass id, index of start event; stop = +1)
-    hipEvent_t ev_open = nullptr;
-    int ev_open_pass = -1;
-    // sticky non-finite flag written by the fused epilogues and the scalar stage
-    int* nf = nullptr;
-    int* nf_host = nullptr;  // pinned
-    // batched probe: partial sums and results (device), results (pinned host)
-    double* pb = nullptr;
-    double* pb_host = nullptr;
-    size_t pb_cap = 0;
-};
 
 namespace {
 
@@ -348,6 +159,7 @@ int build_tables(ns3d_ctx* c) {
     t.px = d; d += Nx; t.py = d; d += Ny; t.pz = d; d += Mz;
     t.fm = d; d += Nx; t.fn = d; d += Ny; t.fq = d; d += Mz;
     t.mx = d; d += Nx; t.my = d; d += Ny; t.mz = d;
+    t.kb1 = k1;
     t.k1k2 = k1 * k2;
     t.k1k3 = k1 * k3;
     t.k2k3 = k2 * k3;
@@ -383,34 +195,6 @@ int build_twiddles(ns3d_ctx* c) {
         HIPCHK(hipMemcpy(c->tw32[a], h32.data(), sizeof(cplx<float>) * n, hipMemcpyHostToDevice));
     }
     return NS3D_OK;
-}
-
-template <typename TB> const cplx<TB>* twp(const ns3d_ctx* c, int axis) {
-    return (const cplx<TB>*)(sizeof(TB) == 8 ? c->tw64[axis] : c->tw32[axis]);
-}
-
-size_t bulk_bytes(const ns3d_ctx* c) { return c->precision == NS3D_FP64 ? sizeof(zd) : sizeof(cplx<float>); }
-
-// Row stride of the fused passes' scratch fields: Mz rounded up so that every
-// P-mode row tile of the x/y passes (128 B) starts on a 128-B line.
-#ifndef NS3D_PAD_ROWS
-#define NS3D_PAD_ROWS 1
-#endif
-// Row padding (modes) of the library's own FP64 and FP32 fields: 8 modes, so
-// FP64 rows start on 128-B and FP32 rows on 64-B boundaries, which the x and y
-// tiles' 8-mode segments need.  256^3, rows of 136 against 144: FP32 steps
-// -1.0% (bulk), -1.8% (state), -2.1% (increments), chiefly the x-forward pass
-// (-4%: x-planes 136*256 modes apart map onto HBM better than 144*256); FP64
-// rows of 144 gained only 0.4% for 6% more memory.
-#ifndef NS3D_ROWPAD64
-#define NS3D_ROWPAD64 8
-#endif
-#ifndef NS3D_ROWPAD32
-#define NS3D_ROWPAD32 8
-#endif
-int mi_of(const ns3d_ctx* c) {
-    const int a = NS3D_PAD_ROWS ? (c->precision == NS3D_FP64 ? NS3D_ROWPAD64 : NS3D_ROWPAD32) : 1;
-    return (c->Mz + a - 1) / a * a;
 }
 
 // Forget a captured RK3 graph (its nodes hold scratch pointers, table values and the stream).
@@ -455,134 +239,58 @@ int ensure_fp64(ns3d_ctx* c, zd** p, int fields) {
     return NS3D_OK;
 }
 
-inline unsigned nblk(long n, int t) { return (unsigned)((n + t - 1) / t); }
-// grid for the XCD-remapped pencil kernels: block count padded to a multiple of 8
-inline dim3 xgrid(long nb, int nfy = 1, int nz = 1) {
-    return dim3((unsigned)(((nb + 7) / 8) * 8), (unsigned)nfy, (unsigned)nz);
+// Whether this grid's x-forward pass carries the next stage's P1 (CHAINS).
+bool can_chain(const ns3d_ctx* c) {
+    bool r = false;
+    with_size(c->Nx, [&](auto NXc) -> int {
+        constexpr int NX = decltype(NXc)::value;
+        r = c->precision == NS3D_FP64 ? CHAINS<double, NX> : CHAINS<float, NX>;
+        return 0;
+    });
+    return r;
 }
 
 // ---------------------------------------------------------------- fused pipeline
-// Runs P1..P4 for NF vector fields and leaves D (3 fields) at scratch + 3*nci.
+// Runs P1..P4 for NF vector fields and leaves D (3 fields) at the head of region B
+// (scratch + 6*nf*nci), so that A is free for the P1 output of the next stage.
 // mw: row stride of the input fields (0: Mz, the reference layout)
 // bin: batch member stride of the inputs (c->batch members, scratch c->bsc apart).
+// has_a: the previous stage's x-forward pass left P1's output in A (CHAIN), in is not read.
 // in2 (nf = 1 only, may be null): a second field of in's type and layout added
 // to the input before the transforms (the FP32-increment loop's base + increment).
 template <typename TB, typename TS = double>
-int run_nonlinear_passes(ns3d_ctx* c, const cplx<TS>* const* in, int nf, int mw = 0, long bin = 0,
+int run_nonlinear_passes(ns3d_ctx* c, const cplx<TS>* const* in, int nf, int mw = 0, long bin = 0, bool has_a = false,
                          const cplx<TS>* const* in2 = nullptr) {
+    has_a = has_a && can_chain(c);
     if (mw == 0) mw = c->Mz;
     int st = ensure_scratch(c, 15 * nf * c->batch);
     if (st) return st;
-    const int nz = c->batch;
-    const long bsc = c->bsc;
-    // scratch fields: rows padded to Mi (128-B aligned pencil tiles), nci modes each
-    const long nc = c->nci;
-    const int Mi = mi_of(c);
-    cplx<TB>* A = (cplx<TB>*)c->scratch;
-    cplx<TB>* B = A + (long)6 * nf * nc;
-    hipStream_t s = c->stream;
-    // P1 x-inverse
-    prof_begin(c, 0);
-    st = with_size(c->Nx, [&](auto NXc) -> int {
-        constexpr int NX = decltype(NXc)::value;
-        constexpr int E = E_XINV<TB>;
-        constexpr int P = PXY_T<TB, NX, E, NS3D_PXINV32, NS3D_BY_RADIX(NX, NS3D_PXINV64, NS3D_R3_PXINV64)>;
-        const int nlt = (c->Mz + P - 1) / P;
-        const int nb = c->Ny * nlt;
-        constexpr int OS = NS3D_OS_XINV;
-        dim3 grid = xgrid(nb, 3 * nf * (OS ? 2 : 1), nz), blk(P * XYPlan<NX, E>::TPP);
-        if (nf == 1 && in2) {
-            PtrArr<const cplx<TS>, 3> w{{in[0], in[1], in[2]}};
-            PtrArr<const cplx<TS>, 3> w2{{in2[0], in2[1], in2[2]}};
-            hipLaunchKernelGGL((k_x_inv_grad<TB, NX, P, 1, E, OS, TS, 1>), grid, blk, 0, s, w, A, nc, c->Ny, c->Mz, mw, Mi, nlt, nb,
-                               c->tab, twp<TB>(c, 0), bin, bsc, w2, c->mm);
-        } else if (nf == 1) {
-            PtrArr<const cplx<TS>, 3> w{{in[0], in[1], in[2]}};
-            hipLaunchKernelGGL((k_x_inv_grad<TB, NX, P, 1, E, OS, TS>), grid, blk, 0, s, w, A, nc, c->Ny, c->Mz, mw, Mi, nlt, nb, c->tab,
-                               twp<TB>(c, 0), bin, bsc, PtrArr<const cplx<TS>, 3>{}, c->mm);
-        } else if constexpr (std::is_same<TS, double>::value) {
-            PtrArr<const zd, 6> w{{in[0], in[1], in[2], in[3], in[4], in[5]}};
-            hipLaunchKernelGGL((k_x_inv_grad<TB, NX, P, 2, E, OS>), grid, blk, 0, s, w, A, nc, c->Ny, c->Mz, mw, Mi, nlt, nb, c->tab,
-                               twp<TB>(c, 0), bin, bsc, PtrArr<const zd, 3>{}, c->mm);
-        } else {
-            return NS3D_ERR_ARG;
-        }
-        return NS3D_OK;
-    });
-    prof_end(c);
-    if (st) return st;
-    // P2 y-inverse
+    if (!has_a) {
+        prof_begin(c, 0);
+        st = with_size(c->Nx, [&](auto N) { return launch_x_inv<TB, TS, decltype(N)::value>(c, in, in2, nf, mw, bin); });
+        prof_end(c);
+        if (st) return st;
+    }
     prof_begin(c, 1);
-    st = with_size(c->Ny, [&](auto NYc) -> int {
-        constexpr int NY = decltype(NYc)::value;
-        constexpr int E = E_YINV<TB>;
-        constexpr int P = PXY_T<TB, NY, E, NS3D_BY_RADIX(NY, NS3D_PYINV32, NS3D_R3_PYINV32),
-                                NS3D_BY_RADIX(NY, NS3D_PYINV64, NS3D_R3_PYINV64)>;
-        const int nlt = (c->Mz + P - 1) / P;
-        const int nb = c->Nx * nlt;
-        constexpr int OS = NS3D_OS_YINV;
-        dim3 grid = xgrid(nb, 3 * nf * (OS ? 3 : 1), nz), blk(P * XYPlan<NY, E>::TPP);
-        if (nf == 1)
-            hipLaunchKernelGGL((k_y_inv_grad<TB, NY, P, 1, E, OS>), grid, blk, 0, s, A, B, nc, c->Ny, c->Mz, Mi, nlt, nb, c->tab,
-                               twp<TB>(c, 1), bsc, c->mm);
-        else
-            hipLaunchKernelGGL((k_y_inv_grad<TB, NY, P, 2, E, OS>), grid, blk, 0, s, A, B, nc, c->Ny, c->Mz, Mi, nlt, nb, c->tab,
-                               twp<TB>(c, 1), bsc, c->mm);
-        return NS3D_OK;
-    });
+    st = with_size(c->Ny, [&](auto N) { return launch_y_inv<TB, decltype(N)::value>(c, nf); });
     prof_end(c);
     if (st) return st;
-    // P3 z: C2R, product, R2C -> C at A
     prof_begin(c, 2);
-    st = with_size(c->Nz, [&](auto NZc) -> int {
-        constexpr int NZ = decltype(NZc)::value;
-        constexpr int P = PZ<TB, NZ>;
-        const int nb = (int)nblk(c->npen, P);
-        dim3 grid = xgrid(nb, 1, nz), blk(P * ZPlanT<TB, NZ>::TPP);
-        const TB scale = (TB)(1.0 / (1.0 * c->Nx * c->Ny * c->Nz));
-        TB* up = nf == 1 ? (TB*)c->uphys_out : nullptr;
-        if (nf == 1)
-            hipLaunchKernelGGL((k_z_product<TB, NZ, P, 1>), grid, blk, 0, s, B, A, nc, c->npen, Mi, nb, c->tab, twp<TB>(c, 2), scale,
-                               up, c->nr, bsc, c->mm);
-        else
-            hipLaunchKernelGGL((k_z_product<TB, NZ, P, 2>), grid, blk, 0, s, B, A, nc, c->npen, Mi, nb, c->tab, twp<TB>(c, 2), scale,
-                               (TB*)nullptr, c->nr, bsc, c->mm);
-        return NS3D_OK;
-    });
+    st = with_size(c->Nz, [&](auto N) { return launch_z<TB, decltype(N)::value>(c, nf); });
     prof_end(c);
     if (st) return st;
-    // P4 y-forward C -> D
     prof_begin(c, 3);
-    st = with_size(c->Ny, [&](auto NYc) -> int {
-        constexpr int NY = decltype(NYc)::value;
-        constexpr int E = E_C2C<TB>;
-        constexpr int P = PXY_T<TB, NY, E, NS3D_PYFWD32, 8>;
-        const int nlt = (c->Mz + P - 1) / P;
-        const int nb = c->Nx * nlt;
-        dim3 grid = xgrid(nb, 3, nz), blk(P * XYPlan<NY, E>::TPP);
-        hipLaunchKernelGGL((k_axis_c2c<TB, NY, P, -1, 1, E>), grid, blk, 0, s, A, A + 3 * nc, 3, nc, c->Ny, c->Mz, Mi, nlt, nb,
-                           twp<TB>(c, 1), bsc, c->mm);
-        return NS3D_OK;
-    });
+    st = with_size(c->Ny, [&](auto N) { return launch_y_fwd<TB, decltype(N)::value>(c, nf); });
     prof_end(c);
     return st;
 }
 
+// P5 for nf fields' D; chain: with the P1 of the next stage (the RK3 loops' modes).
 template <typename TB, int MODE>
-int run_x_forward_epilogue(ns3d_ctx* c, const EpiArgs& ea) {
-    const cplx<TB>* D = (const cplx<TB>*)c->scratch + 3 * c->nci;
+int run_x_forward_epilogue(ns3d_ctx* c, const EpiArgs& ea, int nf = 1, bool chain = false) {
+    chain = chain && can_chain(c);
     prof_begin(c, 4);
-    int st = with_size(c->Nx, [&](auto NXc) -> int {
-        constexpr int NX = decltype(NXc)::value;
-        constexpr int E = E_XFWD<TB>;
-        constexpr int P = PXY_T<TB, NX, E, NS3D_BY_RADIX(NX, NS3D_PXFWD32, NS3D_R3_PXFWD32), 8>;
-        const int nlt = (c->Mz + P - 1) / P;
-        const int nb = c->Ny * nlt;
-        dim3 grid = xgrid(nb, 1, c->batch), blk(P * XYPlan<NX, E>::TPP);
-        hipLaunchKernelGGL((k_x_fwd_epi<TB, NX, P, MODE, E>), grid, blk, 0, c->stream, D, c->nci, c->Ny, c->Mz, mi_of(c), nlt, nb,
-                           c->tab, twp<TB>(c, 0), ea, c->bsc, c->mm);
-        return NS3D_OK;
-    });
+    int st = with_size(c->Nx, [&](auto N) { return launch_x_fwd<TB, MODE, decltype(N)::value>(c, ea, nf, chain); });
     prof_end(c);
     return st;
 }
@@ -606,17 +314,18 @@ EpiArgs make_epi(const ns3d_ctx* c) {
 }
 
 // nonlinear term of nf fields followed by the MODE epilogue
+// has_a: P1's output is in A already; chain: leave the next stage's there
 template <int MODE>
-int fused(ns3d_ctx* c, const zd* const* in, int nf, const EpiArgs& ea) {
+int fused(ns3d_ctx* c, const zd* const* in, int nf, const EpiArgs& ea, bool has_a = false, bool chain = false) {
     int st;
     if (c->precision == NS3D_FP64) {
-        st = run_nonlinear_passes<double>(c, in, nf, ea.mw, ea.bw);
+        st = run_nonlinear_passes<double>(c, in, nf, ea.mw, ea.bw, has_a);
         if (st) return st;
-        st = run_x_forward_epilogue<double, MODE>(c, ea);
+        st = run_x_forward_epilogue<double, MODE>(c, ea, nf, chain);
     } else {
-        st = run_nonlinear_passes<float>(c, in, nf, ea.mw, ea.bw);
+        st = run_nonlinear_passes<float>(c, in, nf, ea.mw, ea.bw, has_a);
         if (st) return st;
-        st = run_x_forward_epilogue<float, MODE>(c, ea);
+        st = run_x_forward_epilogue<float, MODE>(c, ea, nf, chain);
     }
     if (st) return st;
     return hipGetLastError() == hipSuccess ? NS3D_OK : NS3D_ERR_HIP;
@@ -625,7 +334,8 @@ int fused(ns3d_ctx* c, const zd* const* in, int nf, const EpiArgs& ea) {
 // E(w) stage: out = a0*u0 + a1*(w + dt*L(w)); mw/mu0/mo: row strides (0: Mz)
 // bw, bu0, bo: batch member strides of w, u0 and out (when c->batch > 1)
 int stage_into(ns3d_ctx* c, const zd* const w[3], const zd* const u0[3], double a0, double a1, zd* const out[3],
-               const zd* const f[3], int mw = 0, int mu0 = 0, int mo = 0, long bw = 0, long bu0 = 0, long bo = 0) {
+               const zd* const f[3], int mw = 0, int mu0 = 0, int mo = 0, long bw = 0, long bu0 = 0, long bo = 0,
+               bool has_a = false, bool chain = false) {
     EpiArgs ea = make_epi(c);
     if (mw) ea.mw = mw;
     if (mu0) ea.mu0 = mu0;
@@ -641,10 +351,12 @@ int stage_into(ns3d_ctx* c, const zd* const w[3], const zd* const u0[3], double 
     }
     ea.a0 = a0;
     ea.a1 = a1;
-    return fused<EPI_STAGE>(c, w, 1, ea);
+    return fused<EPI_STAGE>(c, w, 1, ea, has_a, chain);
 }
 
-int rk3_one(ns3d_ctx* c, zd* const u[3], const zd* const f[3]) {
+// Stages after the first of a call find their P1 output in A, left there by the x-forward
+// pass of the stage before (first: this step opens the call; last: no step follows in it).
+int rk3_one(ns3d_ctx* c, zd* const u[3], const zd* const f[3], bool first, bool last) {
     int st = ensure_fp64(c, &c->stage, 9);
     if (st) return st;
     // u1, u2 are the library's own: rows padded to M8 (128-B aligned), fields nc8 apart
@@ -658,9 +370,9 @@ int rk3_one(ns3d_ctx* c, zd* const u[3], const zd* const f[3]) {
     const int mz = c->Mz;
     // RK3_SSP (Source/RK_time_step.cu:310-327):
     //   u1 = E(u); u1 = E(u1); u2 = 3/4 u + 1/4 u1; u2 = E(u2); u = 1/3 u + 2/3 u2
-    if ((st = stage_into(c, uc, nullptr, 0.0, 1.0, u1, f, mz, mz, m8))) return st;
-    if ((st = stage_into(c, u1c, uc, 3.0 / 4.0, 1.0 / 4.0, u2, f, m8, mz, m8))) return st;
-    if ((st = stage_into(c, u2c, uc, 1.0 / 3.0, 2.0 / 3.0, u, f, m8, mz, mz))) return st;
+    if ((st = stage_into(c, uc, nullptr, 0.0, 1.0, u1, f, mz, mz, m8, 0, 0, 0, !first, true))) return st;
+    if ((st = stage_into(c, u1c, uc, 3.0 / 4.0, 1.0 / 4.0, u2, f, m8, mz, m8, 0, 0, 0, true, true))) return st;
+    if ((st = stage_into(c, u2c, uc, 1.0 / 3.0, 2.0 / 3.0, u, f, m8, mz, mz, 0, 0, 0, true, !last))) return st;
     return NS3D_OK;
 }
 
@@ -670,7 +382,7 @@ int rk3_one(ns3d_ctx* c, zd* const u[3], const zd* const f[3]) {
 using cf = cplx<float>;
 
 int stage_into32(ns3d_ctx* c, const cf* const w[3], const cf* const u0[3], double a0, double a1, cf* const out[3],
-                 const zd* const f[3]) {
+                 const zd* const f[3], bool has_a, bool chain) {
     EpiArgs ea = make_epi(c);
     for (int b = 0; b < 3; b++) {
         ea.w[b] = (zd*)w[b];
@@ -681,14 +393,14 @@ int stage_into32(ns3d_ctx* c, const cf* const w[3], const cf* const u0[3], doubl
     ea.a0 = a0;
     ea.a1 = a1;
     ea.mw = ea.mu0 = ea.mo = c->m16;  // the FP32 state and stages use rows padded to m16
-    int st = run_nonlinear_passes<float, float>(c, w, 1, c->m16);
+    int st = run_nonlinear_passes<float, float>(c, w, 1, c->m16, 0, has_a);
     if (st) return st;
-    st = run_x_forward_epilogue<float, EPI_STAGE32>(c, ea);
+    st = run_x_forward_epilogue<float, EPI_STAGE32>(c, ea, 1, chain);
     if (st) return st;
     return hipGetLastError() == hipSuccess ? NS3D_OK : NS3D_ERR_HIP;
 }
 
-int rk3_one32(ns3d_ctx* c, const zd* const f[3]) {
+int rk3_one32(ns3d_ctx* c, const zd* const f[3], bool first, bool last) {
     const long nc = c->nc16;
     cf* u[3] = {c->s32, c->s32 + nc, c->s32 + 2 * nc};
     cf* u1[3] = {c->s32 + 3 * nc, c->s32 + 4 * nc, c->s32 + 5 * nc};
@@ -697,9 +409,9 @@ int rk3_one32(ns3d_ctx* c, const zd* const f[3]) {
     const cf* u1c[3] = {u1[0], u1[1], u1[2]};
     const cf* u2c[3] = {u2[0], u2[1], u2[2]};
     int st;
-    if ((st = stage_into32(c, uc, nullptr, 0.0, 1.0, u1, f))) return st;
-    if ((st = stage_into32(c, u1c, uc, 3.0 / 4.0, 1.0 / 4.0, u2, f))) return st;
-    if ((st = stage_into32(c, u2c, uc, 1.0 / 3.0, 2.0 / 3.0, u, f))) return st;
+    if ((st = stage_into32(c, uc, nullptr, 0.0, 1.0, u1, f, !first, true))) return st;
+    if ((st = stage_into32(c, u1c, uc, 3.0 / 4.0, 1.0 / 4.0, u2, f, true, true))) return st;
+    if ((st = stage_into32(c, u2c, uc, 1.0 / 3.0, 2.0 / 3.0, u, f, true, !last))) return st;
     return NS3D_OK;
 }
 
@@ -714,10 +426,11 @@ int ensure_state32(ns3d_ctx* c) {
 // fields (converted from and to the caller's FP64 field once per call) and
 // the SSP stages are FP32 increments d over it (u1 = u^n + d1, u2 = u^n + d2;
 // EPI_INC / EPI_INC_FINAL), so a stage value is rounded to eps32*|d|, not
-// eps32*|u|.  The transforms and the stages' diffusion read hi alone; the
-// last stage reads hi + lo and writes the new pair.  d2 overwrites d1 in place.
+// eps32*|u|.  The transforms (of hi, and of hi + d summed in FP64 by the x-forward
+// pass that writes d) and the stages' diffusion read hi alone; the last stage reads
+// hi + lo and writes the new pair.  d2 overwrites d1 in place.
 // s32 (rows m16): hi [3], lo [3], d [3].
-int stage_incr(ns3d_ctx* c, bool first, double a1, bool last, const zd* const f[3]) {
+int stage_incr(ns3d_ctx* c, bool first, double a1, bool last, const zd* const f[3], bool has_a, bool chain) {
     const long nc = c->nc16;
     cf* hi[3] = {c->s32, c->s32 + nc, c->s32 + 2 * nc};
     cf* lo[3] = {c->s32 + 3 * nc, c->s32 + 4 * nc, c->s32 + 5 * nc};
@@ -734,18 +447,19 @@ int stage_incr(ns3d_ctx* c, bool first, double a1, bool last, const zd* const f[
     }
     ea.a1 = a1;
     ea.mw = ea.mo = ea.mu0 = c->m16;
-    int st = run_nonlinear_passes<float, float>(c, hic, 1, c->m16, 0, first ? nullptr : dc);
+    int st = run_nonlinear_passes<float, float>(c, hic, 1, c->m16, 0, has_a, first ? nullptr : dc);
     if (st) return st;
-    st = last ? run_x_forward_epilogue<float, EPI_INC_FINAL>(c, ea) : run_x_forward_epilogue<float, EPI_INC>(c, ea);
+    st = last ? run_x_forward_epilogue<float, EPI_INC_FINAL>(c, ea, 1, chain)
+              : run_x_forward_epilogue<float, EPI_INC>(c, ea, 1, chain);
     if (st) return st;
     return hipGetLastError() == hipSuccess ? NS3D_OK : NS3D_ERR_HIP;
 }
 
-int rk3_one_incr(ns3d_ctx* c, const zd* const f[3]) {
+int rk3_one_incr(ns3d_ctx* c, const zd* const f[3], bool first, bool last) {
     int st;
-    if ((st = stage_incr(c, true, 1.0, false, f))) return st;
-    if ((st = stage_incr(c, false, 1.0 / 4.0, false, f))) return st;
-    return stage_incr(c, false, 2.0 / 3.0, true, f);
+    if ((st = stage_incr(c, true, 1.0, false, f, !first, true))) return st;
+    if ((st = stage_incr(c, false, 1.0 / 4.0, false, f, true, true))) return st;
+    return stage_incr(c, false, 2.0 / 3.0, true, f, true, !last);
 }
 
 // the RK3 loops of NS3D_FP32_STATE and NS3D_FP32_INCR keep 9 FP32 fields (s32)
@@ -772,7 +486,7 @@ int ensure_batch(ns3d_ctx* c, int nb) {
     return ensure_scratch(c, 15 * nb);
 }
 
-int rk3_one_batch(ns3d_ctx* c, int nb, zd* u, const zd* const f[3]) {
+int rk3_one_batch(ns3d_ctx* c, int nb, zd* u, const zd* const f[3], bool first, bool last) {
     const long n8 = c->nc8, nc = c->nc;
     int st = ensure_batch(c, nb);
     if (st) return st;
@@ -786,9 +500,9 @@ int rk3_one_batch(ns3d_ctx* c, int nb, zd* u, const zd* const f[3]) {
     const long bs = 3 * nc, bst = 6 * n8;
     c->batch = nb;
     c->bsc = 15 * c->nci;
-    if (!(st = stage_into(c, uc, nullptr, 0.0, 1.0, u1, f, mz, mz, m8, bs, 0, bst)))
-        if (!(st = stage_into(c, u1c, uc, 3.0 / 4.0, 1.0 / 4.0, u2, f, m8, mz, m8, bst, bs, bst)))
-            st = stage_into(c, u2c, uc, 1.0 / 3.0, 2.0 / 3.0, uu, f, m8, mz, mz, bst, bs, bs);
+    if (!(st = stage_into(c, uc, nullptr, 0.0, 1.0, u1, f, mz, mz, m8, bs, 0, bst, !first, true)))
+        if (!(st = stage_into(c, u1c, uc, 3.0 / 4.0, 1.0 / 4.0, u2, f, m8, mz, m8, bst, bs, bst, true, true)))
+            st = stage_into(c, u2c, uc, 1.0 / 3.0, 2.0 / 3.0, uu, f, m8, mz, mz, bst, bs, bs, true, !last);
     c->batch = 1;
     c->bsc = 0;
     return st;
@@ -804,7 +518,7 @@ int rk3_batch_members(ns3d_ctx* c, int nb, int nsteps, zd* u, const zd* const f[
     int st = NS3D_OK;
     for (int i = 0; i < nsteps && !st; i++) {
         c->mm.step = i;
-        st = rk3_one_batch(c, nb, u, f);
+        st = rk3_one_batch(c, nb, u, f, i == 0, i == nsteps - 1);
     }
     c->mm.left = nullptr;
     c->mm.step = 0;
@@ -824,7 +538,7 @@ int rk3_steps(ns3d_ctx* c, int nsteps, zd* const u[3], const zd* const f[3]) {
                                c->s32 + (3 + b) * n16, c->nc, c->Mz, c->m16);
         HIPCHK(hipGetLastError());
         for (int i = 0; i < nsteps; i++)
-            if ((st = rk3_one_incr(c, f))) return st;
+            if ((st = rk3_one_incr(c, f, i == 0, i == nsteps - 1))) return st;
         for (int b = 0; b < 3; b++)
             hipLaunchKernelGGL(k_join_rows, dim3(nblk(c->nc, 256)), dim3(256), 0, c->stream, c->s32 + b * n16,
                                c->s32 + (3 + b) * n16, u[b], c->nc, c->Mz, c->m16);
@@ -833,7 +547,7 @@ int rk3_steps(ns3d_ctx* c, int nsteps, zd* const u[3], const zd* const f[3]) {
     }
     if (c->precision != NS3D_FP32_STATE) {
         for (int i = 0; i < nsteps; i++) {
-            int st = rk3_one(c, u, f);
+            int st = rk3_one(c, u, f, i == 0, i == nsteps - 1);
             if (st) return st;
         }
         return NS3D_OK;
@@ -847,7 +561,7 @@ int rk3_steps(ns3d_ctx* c, int nsteps, zd* const u[3], const zd* const f[3]) {
         hipLaunchKernelGGL(k_d2f_rows, dim3(nblk(nc, 256)), dim3(256), 0, c->stream, u[b], c->s32 + b * n16, nc, c->Mz,
                            c->m16);
     for (int i = 0; i < nsteps; i++) {
-        st = rk3_one32(c, f);
+        st = rk3_one32(c, f, i == 0, i == nsteps - 1);
         if (st) return st;
     }
     for (int b = 0; b < 3; b++)
@@ -860,73 +574,18 @@ int rk3_steps(ns3d_ctx* c, int nsteps, zd* const u[3], const zd* const f[3]) {
 // ---------------------------------------------------------------- standalone 3D transforms
 template <typename TB>
 int c2r_3d(ns3d_ctx* c, const cplx<TB>* in, TB* out, cplx<TB>* tmp, bool scale) {
-    hipStream_t s = c->stream;
-    const long nc = c->nc;
-    int st = with_size(c->Nx, [&](auto N) -> int {
-        constexpr int NX = decltype(N)::value;
-        constexpr int E = E_C2C<TB>;
-        constexpr int P = PXY<TB, NX, E>;
-        const int nlt = (c->Mz + P - 1) / P;
-        hipLaunchKernelGGL((k_axis_c2c<TB, NX, P, +1, 0, E>), xgrid(c->Ny * nlt), dim3(P * XYPlan<NX, E>::TPP), 0, s, in, tmp, 1, nc,
-                           c->Ny, c->Mz, c->Mz, nlt, c->Ny * nlt, twp<TB>(c, 0));
-        return NS3D_OK;
-    });
-    if (st) return st;
-    st = with_size(c->Ny, [&](auto N) -> int {
-        constexpr int NY = decltype(N)::value;
-        constexpr int E = E_C2C<TB>;
-        constexpr int P = PXY<TB, NY, E>;
-        const int nlt = (c->Mz + P - 1) / P;
-        hipLaunchKernelGGL((k_axis_c2c<TB, NY, P, +1, 1, E>), xgrid(c->Nx * nlt), dim3(P * XYPlan<NY, E>::TPP), 0, s, tmp, tmp, 1,
-                           nc, c->Ny, c->Mz, c->Mz, nlt, c->Nx * nlt, twp<TB>(c, 1));
-        return NS3D_OK;
-    });
-    if (st) return st;
-    return with_size(c->Nz, [&](auto N) -> int {
-        constexpr int NZ = decltype(N)::value;
-        constexpr int P = PZ<TB, NZ>;
-        const long npairs = c->npen / 2;
-        const TB sc = scale ? (TB)(1.0 / (1.0 * c->Nx * c->Ny * c->Nz)) : (TB)1;
-        const int nb = (int)nblk(npairs, P);
-        hipLaunchKernelGGL((k_z_c2r<TB, NZ, P>), xgrid(nb), dim3(P * ZPlanT<TB, NZ>::TPP), 0, s, tmp, out, npairs,
-                           c->Mz, nb, c->tab, twp<TB>(c, 2), sc);
-        return NS3D_OK;
-    });
+    int st = with_size(c->Nx, [&](auto N) { return launch_c2c<TB, decltype(N)::value>(c, +1, 0, in, tmp); });
+    if (!st) st = with_size(c->Ny, [&](auto N) { return launch_c2c<TB, decltype(N)::value>(c, +1, 1, tmp, tmp); });
+    if (!st) st = with_size(c->Nz, [&](auto N) { return launch_c2r<TB, decltype(N)::value>(c, tmp, out, scale); });
+    return st;
 }
 
 template <typename TB>
 int r2c_3d(ns3d_ctx* c, const TB* in, cplx<TB>* out) {
-    hipStream_t s = c->stream;
-    const long nc = c->nc;
-    int st = with_size(c->Nz, [&](auto N) -> int {
-        constexpr int NZ = decltype(N)::value;
-        constexpr int P = PZ<TB, NZ>;
-        const long npairs = c->npen / 2;
-        const int nb = (int)nblk(npairs, P);
-        hipLaunchKernelGGL((k_z_r2c<TB, NZ, P>), xgrid(nb), dim3(P * ZPlanT<TB, NZ>::TPP), 0, s, in, out, npairs,
-                           c->Mz, nb, twp<TB>(c, 2));
-        return NS3D_OK;
-    });
-    if (st) return st;
-    st = with_size(c->Ny, [&](auto N) -> int {
-        constexpr int NY = decltype(N)::value;
-        constexpr int E = E_C2C<TB>;
-        constexpr int P = PXY<TB, NY, E>;
-        const int nlt = (c->Mz + P - 1) / P;
-        hipLaunchKernelGGL((k_axis_c2c<TB, NY, P, -1, 1, E>), xgrid(c->Nx * nlt), dim3(P * XYPlan<NY, E>::TPP), 0, s, out, out, 1,
-                           nc, c->Ny, c->Mz, c->Mz, nlt, c->Nx * nlt, twp<TB>(c, 1));
-        return NS3D_OK;
-    });
-    if (st) return st;
-    return with_size(c->Nx, [&](auto N) -> int {
-        constexpr int NX = decltype(N)::value;
-        constexpr int E = E_C2C<TB>;
-        constexpr int P = PXY<TB, NX, E>;
-        const int nlt = (c->Mz + P - 1) / P;
-        hipLaunchKernelGGL((k_axis_c2c<TB, NX, P, -1, 0, E>), xgrid(c->Ny * nlt), dim3(P * XYPlan<NX, E>::TPP), 0, s, out, out, 1,
-                           nc, c->Ny, c->Mz, c->Mz, nlt, c->Ny * nlt, twp<TB>(c, 0));
-        return NS3D_OK;
-    });
+    int st = with_size(c->Nz, [&](auto N) { return launch_r2c<TB, decltype(N)::value>(c, in, out); });
+    if (!st) st = with_size(c->Ny, [&](auto N) { return launch_c2c<TB, decltype(N)::value>(c, -1, 1, out, out); });
+    if (!st) st = with_size(c->Nx, [&](auto N) { return launch_c2c<TB, decltype(N)::value>(c, -1, 0, out, out); });
+    return st;
 }
 
 // FP64-interface 3D transforms (FP32 bulk: convert, transform, convert back)
@@ -1022,7 +681,7 @@ int weno_stage(ns3d_ctx* c, int scheme, const double* xs, const double* xn, doub
     return hipGetLastError() == hipSuccess ? NS3D_OK : NS3D_ERR_HIP;
 }
 
-int rk3_scalar_one(ns3d_ctx* c, zd* const u[3], const zd* const f[3], double* th, int scheme) {
+int rk3_scalar_one(ns3d_ctx* c, zd* const u[3], const zd* const f[3], double* th, int scheme, bool first, bool last) {
     int st = ensure_fp64(c, &c->stage, 9);
     if (st) return st;
     if (!c->uphys && hipMalloc(&c->uphys, bulk_bytes(c) / 2 * (size_t)c->nr * 3) != hipSuccess) return NS3D_ERR_ALLOC;
@@ -1037,10 +696,10 @@ int rk3_scalar_one(ns3d_ctx* c, zd* const u[3], const zd* const f[3], double* th
     double* th2 = c->theta_stage + c->nr;
     c->uphys_out = c->uphys;
     // the velocity stages write their physical flow; the scalar stage follows with the same SSP weights
-    if (!(st = stage_into(c, uc, nullptr, 0.0, 1.0, u1, f))) st = weno_stage(c, scheme, th, nullptr, th1, 0.0, 1.0);
-    if (!st && !(st = stage_into(c, u1c, uc, 3.0 / 4.0, 1.0 / 4.0, u2, f)))
+    if (!(st = stage_into(c, uc, nullptr, 0.0, 1.0, u1, f, 0, 0, 0, 0, 0, 0, !first, true))) st = weno_stage(c, scheme, th, nullptr, th1, 0.0, 1.0);
+    if (!st && !(st = stage_into(c, u1c, uc, 3.0 / 4.0, 1.0 / 4.0, u2, f, 0, 0, 0, 0, 0, 0, true, true)))
         st = weno_stage(c, scheme, th1, th, th2, 3.0 / 4.0, 1.0 / 4.0);
-    if (!st && !(st = stage_into(c, u2c, uc, 1.0 / 3.0, 2.0 / 3.0, u, f)))
+    if (!st && !(st = stage_into(c, u2c, uc, 1.0 / 3.0, 2.0 / 3.0, u, f, 0, 0, 0, 0, 0, 0, true, !last)))
         st = weno_stage(c, scheme, th2, th, th, 1.0 / 3.0, 2.0 / 3.0);
     c->uphys_out = nullptr;
     return st;
@@ -1489,7 +1148,7 @@ int ns3d_rk3_ssp_batch(ns3d_ctx* c, int nbatch, int nsteps, ns3d_cplx* u, const 
         return checked(c, NS3D_OK);
     }
     for (int i = 0; i < nsteps; i++) {
-        int st = rk3_one_batch(c, nbatch, ub, f);
+        int st = rk3_one_batch(c, nbatch, ub, f, i == 0, i == nsteps - 1);
         if (st) return st;
     }
     return checked(c, NS3D_OK);
@@ -1544,7 +1203,7 @@ int ns3d_rk3_ssp_scalar(ns3d_ctx* c, int nsteps, ns3d_cplx* ux, ns3d_cplx* uy, n
     zd* u[3] = {(zd*)ux, (zd*)uy, (zd*)uz};
     const zd* f[3] = {(const zd*)fx, (const zd*)fy, (const zd*)fz};
     for (int i = 0; i < nsteps; i++) {
-        int st = rk3_scalar_one(c, u, f, theta, scheme);
+        int st = rk3_scalar_one(c, u, f, theta, scheme, i == 0, i == nsteps - 1);
         if (st) return st;
     }
     return checked(c, NS3D_OK);

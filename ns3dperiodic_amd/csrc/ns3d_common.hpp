@@ -7,6 +7,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace ns3d {
 
 template <typename T>
@@ -17,7 +19,20 @@ struct alignas(2 * sizeof(T)) cplx {
 template <typename T> __device__ __forceinline__ cplx<T> mk(T a, T b) { cplx<T> r; r.x = a; r.y = b; return r; }
 template <typename T> __device__ __forceinline__ cplx<T> operator+(cplx<T> a, cplx<T> b) { return mk<T>(a.x + b.x, a.y + b.y); }
 template <typename T> __device__ __forceinline__ cplx<T> operator-(cplx<T> a, cplx<T> b) { return mk<T>(a.x - b.x, a.y - b.y); }
-template <typename T> __device__ __forceinline__ cplx<T> cmul(cplx<T> a, cplx<T> b) { return mk<T>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
+// FP64: the fused multiply-adds are spelled out, so that every kernel rounds a product alike
+// (a transform fused into one kernel is bitwise the one another kernel makes); FP32 leaves
+// the choice to the compiler.
+template <typename T> __device__ __forceinline__ cplx<T> cmul(cplx<T> a, cplx<T> b) {
+    if constexpr (sizeof(T) == 8)
+        return mk<T>(__builtin_fma(a.x, b.x, -(a.y * b.y)), __builtin_fma(a.x, b.y, a.y * b.x));
+    else
+        return mk<T>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+}
+// A product rounded by itself, never contracted into a following addition.
+template <typename T> __device__ __forceinline__ T mul_rounded(T a, T b) {
+#pragma clang fp contract(off)
+    return a * b;
+}
 template <typename T> __device__ __forceinline__ cplx<T> cscale(cplx<T> a, T s) { return mk<T>(a.x * s, a.y * s); }
 template <typename T> __device__ __forceinline__ cplx<T> conjg(cplx<T> a) { return mk<T>(a.x, -a.y); }
 // multiply by (sgn * i)
@@ -37,18 +52,53 @@ constexpr int BUF_OOB = (int)0x80000000u;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void* base, int bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, bytes, 0x00020000);
 }
-template <typename T> __device__ __forceinline__ cplx<T> buf_load(__amdgpu_buffer_rsrc_t r, int off);
-template <> __device__ __forceinline__ cplx<double> buf_load<double>(__amdgpu_buffer_rsrc_t r, int off) {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+// off: per-lane byte offset (range-checked); so: byte offset uniform over the wave, in
+// the instruction's scalar operand, so a strided run of elements shares one lane offset.
+template <typename T> __device__ __forceinline__ cplx<T> buf_load(__amdgpu_buffer_rsrc_t r, int off, int so = 0);
+template <> __device__ __forceinline__ cplx<double> buf_load<double>(__amdgpu_buffer_rsrc_t r, int off, int so) {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, off, so, 0);
     cplx<double> a;
     __builtin_memcpy(&a, &v, sizeof(a));
     return a;
 }
-template <> __device__ __forceinline__ cplx<float> buf_load<float>(__amdgpu_buffer_rsrc_t r, int off) {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
+template <> __device__ __forceinline__ cplx<float> buf_load<float>(__amdgpu_buffer_rsrc_t r, int off, int so) {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, off, so, 0);
     cplx<float> a;
     __builtin_memcpy(&a, &v, sizeof(a));
     return a;
+}
+typedef unsigned int buf_u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int buf_u32x2 __attribute__((ext_vector_type(2)));
+// Stores out of range are dropped.  NT: nontemporal (streaming) store.
+template <typename T, bool NT = false>
+__device__ __forceinline__ void buf_store(__amdgpu_buffer_rsrc_t r, cplx<T> a, int off, int so = 0) {
+    if constexpr (sizeof(T) == 8) {
+        buf_u32x4 v;
+        __builtin_memcpy(&v, &a, sizeof(a));
+        __builtin_amdgcn_raw_buffer_store_b128(v, r, off, so, NT ? 2 : 0);
+    } else {
+        buf_u32x2 v;
+        __builtin_memcpy(&v, &a, sizeof(a));
+        __builtin_amdgcn_raw_buffer_store_b64(v, r, off, so, NT ? 2 : 0);
+    }
+}
+
+template <bool NT, typename T> __device__ __forceinline__ void st_cplx(cplx<T>* p, cplx<T> a) {
+    if constexpr (NT) {
+        typedef T v2 __attribute__((ext_vector_type(2)));
+        v2 v = {a.x, a.y};
+        __builtin_nontemporal_store(v, (v2*)p);
+    } else {
+        *p = a;
+    }
+}
+
+// f(integral_constant<int, I>) for I = B .. E-1
+template <int B, int E, class F> __device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (B < E) {
+        f(std::integral_constant<int, B>{});
+        static_for<B + 1, E>(f);
+    }
 }
 
 // Per-context spectral constants.  Per-axis tables are built on the host with
@@ -71,6 +121,7 @@ struct SpecTables {
     const double* mx;       // [Nx]  kx^2/kxMax^2  (build_mask_matrix :471-519, with Nz := Mz)
     const double* my;       // [Ny]
     const double* mz;       // [Mz]
+    double kb1;             // 2*pi/Lx: kx[j] = kb1*m
     double k1k2, k1k3, k2k3;  // products of the base wavenumbers 2*pi/L
     double mask_smax;       // largest s with sqrt(s) < 2/3 (host libm sqrt)
     int lmax;               // largest l whose z-plane keeps any mode (mz[l] <= mask_smax)
