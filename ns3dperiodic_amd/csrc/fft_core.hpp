@@ -221,6 +221,22 @@ template <typename TB, int N> struct ZSel {
     using type = typename std::conditional<(sizeof(TB) == 4 && NS3D_ZPLAN32 == 8), Plan<N>, ZPlan<N>>::type;
 };
 template <typename TB, int N> using ZPlanT = typename ZSel<TB, N>::type;
+// Threads per pencil in the z pass: the plan's, or for radix-3 lengths rounded up to a power
+// of two that divides the wavefront (48: 16, 96: 32, 192: 64).  A quarter of the lanes then
+// idle in the radix-4 passes, but every exchange is ordered within one wave instead of by a
+// block barrier, and the radix-3 pass takes one butterfly a thread instead of two, which
+// saves its registers: 192^3 FP64 z pass 0.239 -> 0.193 ms, 0.178 with two transforms in
+// step, for which there is room now; FP32 0.134 -> 0.110.  Radix-5 lengths lose (160^3 FP64
+// 0.121 -> 0.155 ms: 24 of 64 lanes idle), and FP32 takes it at 192 and 384 only: at 48 and
+// 96 the compiler contracts the partly idle radix-4 passes differently.
+constexpr int pow2_up(int n) {
+    int p = 1;
+    while (p < n) p *= 2;
+    return p;
+}
+template <typename TB, int N>
+constexpr int ZTPP = N % 3 == 0 && pow2_up(ZPlanT<TB, N>::TPP) <= 64 && (sizeof(TB) == 8 || N >= 192)
+                         ? pow2_up(ZPlanT<TB, N>::TPP) : ZPlanT<TB, N>::TPP;
 
 // Registers per thread for a plan: max over passes of ceil((N/R)/TPP)*R.
 template <int N, int TPP, typename S> struct PlanRegs;

@@ -363,7 +363,7 @@ k_y_inv_grad(const cplx<TB>* __restrict__ A, cplx<TB>* __restrict__ B, long nc, 
 // C2R convention: x,y passes already done; only Re of l=0 and l=Nz/2 is used.
 template <typename TB, int NZ, int P, bool TRUNC = false>
 struct ZPencil {
-    static constexpr int TPP = ZPlanT<TB, NZ>::TPP;
+    static constexpr int TPP = ZTPP<TB, NZ>;
     static constexpr int PAD = (sizeof(TB) == 8) ? 1 : 2;
 #ifndef NS3D_ZSWZ
 #define NS3D_ZSWZ 8
@@ -651,7 +651,7 @@ template <typename TB, int NZ, int P, int NF>
 #endif
 __global__ void __attribute__((amdgpu_waves_per_eu(NF == 1 ? (sizeof(TB) == 4 ? NS3D_WAVES_Z32 : NS3D_WAVES_Z)
                                                           : (sizeof(TB) == 4 ? NS3D_WAVES_Z2_32 : NS3D_WAVES_Z2), 8)))
-__launch_bounds__((P * ZPlanT<TB, NZ>::TPP))
+__launch_bounds__((P * ZTPP<TB, NZ>))
 k_z_product(const cplx<TB>* __restrict__ Bf, cplx<TB>* __restrict__ C, long nc, long npen, int Mz, int nb,
             SpecTables tab, const cplx<TB>* __restrict__ twg, TB scale, TB* __restrict__ uphys, long nr, int nt, long bsc,
             MemberMask mm) {
@@ -665,9 +665,9 @@ k_z_product(const cplx<TB>* __restrict__ Bf, cplx<TB>* __restrict__ C, long nc, 
 #define NS3D_ZILP32 0
 #endif
     // Two paired transforms at once (two exchange buffers): FP64 at power-of-two
-    // lengths (256^3: z pass 0.458 -> 0.406 ms).  Measured no gain in FP32, and
-    // register spills at the radix-3 lengths.
-    constexpr bool ILP = NF == 1 && (NZ & (NZ - 1)) == 0 && (sizeof(TB) == 8 ? NS3D_ZILP != 0 : NS3D_ZILP32 != 0);
+    // lengths (256^3: z pass 0.458 -> 0.406 ms) and at the radix-3 lengths whose pencils
+    // lie within a wave (192^3: 0.193 -> 0.178 ms; the others spill).  Measured no gain in FP32.
+    constexpr bool ILP = NF == 1 && ((NZ & (NZ - 1)) == 0 || (NZ % 3 == 0 && Z::WAVE)) && (sizeof(TB) == 8 ? NS3D_ZILP != 0 : NS3D_ZILP32 != 0);
 #ifndef NS3D_ZTWREG
 #define NS3D_ZTWREG 1
 #endif
@@ -758,6 +758,7 @@ k_z_product(const cplx<TB>* __restrict__ Bf, cplx<TB>* __restrict__ C, long nc, 
         if (uphys && valid) {
 #pragma unroll
             for (int e = 0; e < NPT; e++) {
+                if (!Z::FI::out_active(t, e / Z::FI::RL)) continue;
                 const long g = pen * NZ + Z::FI::out_index(t, e / Z::FI::RL, e % Z::FI::RL);
                 uphys[g] = w[0][e];
                 uphys[nr + g] = w[1][e];
@@ -802,6 +803,7 @@ k_z_product(const cplx<TB>* __restrict__ Bf, cplx<TB>* __restrict__ C, long nc, 
         if (uphys && valid) {
 #pragma unroll
             for (int e = 0; e < NPT; e++) {
+                if (!Z::FI::out_active(t, e / Z::FI::RL)) continue;
                 const long g = pen * NZ + Z::FI::out_index(t, e / Z::FI::RL, e % Z::FI::RL);
                 uphys[g] = w[0][e];
                 uphys[nr + g] = w[1][e];
@@ -1469,7 +1471,7 @@ k_update(const cplx<double>* __restrict__ Qx, const cplx<double>* __restrict__ Q
 // ---------------------------------------------------------------- z C2R / R2C (single fields)
 // Two neighbouring (x,y) pencils share one complex FFT: Y = X_p0 + i X_p1.
 template <typename TB, int NZ, int P>
-__global__ void __launch_bounds__((P * ZPlanT<TB, NZ>::TPP))
+__global__ void __launch_bounds__((P * ZTPP<TB, NZ>))
 k_z_c2r(const cplx<TB>* __restrict__ in, TB* __restrict__ out, long npairs, int Mz, int nb, SpecTables tab,
         const cplx<TB>* __restrict__ twg, TB scale) {
     using Z = ZPencil<TB, NZ, P>;
@@ -1488,6 +1490,7 @@ k_z_c2r(const cplx<TB>* __restrict__ in, TB* __restrict__ out, long npairs, int 
     if (!valid) return;
 #pragma unroll
     for (int q = 0; q < Z::FI::BL; q++) {
+        if (!Z::FI::out_active(t, q)) continue;
 #pragma unroll
         for (int r = 0; r < Z::FI::RL; r++) {
             const int n = Z::FI::out_index(t, q, r);
@@ -1498,7 +1501,7 @@ k_z_c2r(const cplx<TB>* __restrict__ in, TB* __restrict__ out, long npairs, int 
 }
 
 template <typename TB, int NZ, int P>
-__global__ void __launch_bounds__((P * ZPlanT<TB, NZ>::TPP))
+__global__ void __launch_bounds__((P * ZTPP<TB, NZ>))
 k_z_r2c(const TB* __restrict__ in, cplx<TB>* __restrict__ out, long npairs, int Mz, int nb,
         const cplx<TB>* __restrict__ twg) {
     using Z = ZPencil<TB, NZ, P>;
@@ -1518,8 +1521,9 @@ k_z_r2c(const TB* __restrict__ in, cplx<TB>* __restrict__ out, long npairs, int 
 #pragma unroll
         for (int r = 0; r < Z::FF::R0; r++) {
             const int n = Z::FF::in_index(t, q, r);
-            q1[q * Z::FF::R0 + r] = valid ? in[p0 * NZ + n] : (TB)0;
-            q2[q * Z::FF::R0 + r] = valid ? in[p1 * NZ + n] : (TB)0;
+            const bool on = valid && Z::FF::in_active(t, q);
+            q1[q * Z::FF::R0 + r] = on ? in[p0 * NZ + n] : (TB)0;
+            q2[q * Z::FF::R0 + r] = on ? in[p1 * NZ + n] : (TB)0;
         }
     }
     Z::r2c_pair(q1, q2, out + p0 * Mz, out + p1 * Mz, valid, lds, tw, t, p);

@@ -72,7 +72,7 @@ int launch_z(ns3d_ctx* c, int nf) {
     hipStream_t s = c->stream;
     constexpr int P = PZ<TB, NZ>;
     const int nb = (int)nblk(c->npen, P);
-    dim3 grid = xgrid(nb, 1, nz), blk(P * ZPlanT<TB, NZ>::TPP);
+    dim3 grid = xgrid(nb, 1, nz), blk(P * ZTPP<TB, NZ>);
     const TB scale = (TB)(1.0 / (1.0 * c->Nx * c->Ny * c->Nz));
     TB* up = nf == 1 ? (TB*)c->uphys_out : nullptr;
     if (nf == 1)
@@ -148,7 +148,7 @@ int launch_c2r(ns3d_ctx* c, const cplx<TB>* in, TB* out, bool scale) {
     const long npairs = c->npen / 2;
     const TB sc = scale ? (TB)(1.0 / (1.0 * c->Nx * c->Ny * c->Nz)) : (TB)1;
     const int nb = (int)nblk(npairs, P);
-    hipLaunchKernelGGL((k_z_c2r<TB, NZ, P>), xgrid(nb), dim3(P * ZPlanT<TB, NZ>::TPP), 0, c->stream, in, out, npairs, c->Mz, nb,
+    hipLaunchKernelGGL((k_z_c2r<TB, NZ, P>), xgrid(nb), dim3(P * ZTPP<TB, NZ>), 0, c->stream, in, out, npairs, c->Mz, nb,
                        c->tab, twp<TB>(c, 2), sc);
     return NS3D_OK;
 }
@@ -158,7 +158,7 @@ int launch_r2c(ns3d_ctx* c, const TB* in, cplx<TB>* out) {
     constexpr int P = PZ<TB, NZ>;
     const long npairs = c->npen / 2;
     const int nb = (int)nblk(npairs, P);
-    hipLaunchKernelGGL((k_z_r2c<TB, NZ, P>), xgrid(nb), dim3(P * ZPlanT<TB, NZ>::TPP), 0, c->stream, in, out, npairs, c->Mz, nb,
+    hipLaunchKernelGGL((k_z_r2c<TB, NZ, P>), xgrid(nb), dim3(P * ZTPP<TB, NZ>), 0, c->stream, in, out, npairs, c->Mz, nb,
                        twp<TB>(c, 2));
     return NS3D_OK;
 }
