@@ -50,7 +50,7 @@ template <> struct Radix<3> {
 //   X2,3 = a0 + c2 t1 + c1 t2 +- DIR i (s2 t3 - s1 t4)
 // (c_k = cos(2 pi k/5), s_k = sin(2 pi k/5)).
 template <> struct Radix<5> {
-    template <int DIR, typename T> __device__ __forceinline__ static void dft(cplx<T>* v) {
+    template <int DIR, bool PIN = false, typename T> __device__ __forceinline__ static void dft(cplx<T>* v) {
         const T c1 = (T)0.30901699437494742410229341718281906;   // cos(2 pi/5)
         const T c2 = (T)-0.80901699437494742410229341718281906;  // cos(4 pi/5)
         const T s1 = (T)0.95105651629515357211643933337938214;   // sin(2 pi/5)
@@ -59,7 +59,7 @@ template <> struct Radix<5> {
         const cplx<T> t1 = v[1] + v[4], t2 = v[2] + v[3];
         const cplx<T> t3 = v[1] - v[4], t4 = v[2] - v[3];
         cplx<T> m1, m2, n1, n2;
-        if constexpr (sizeof(T) == 8) {  // contraction spelled out, as in cmul
+        if constexpr (PIN) {  // contraction spelled out, as in cmul_pinned
             m1 = mk<T>(__builtin_fma(c2, t2.x, __builtin_fma(c1, t1.x, a0.x)), __builtin_fma(c2, t2.y, __builtin_fma(c1, t1.y, a0.y)));
             m2 = mk<T>(__builtin_fma(c1, t2.x, __builtin_fma(c2, t1.x, a0.x)), __builtin_fma(c1, t2.y, __builtin_fma(c2, t1.y, a0.y)));
             n1 = mul_i<DIR>(mk<T>(__builtin_fma(s1, t3.x, s2 * t4.x), __builtin_fma(s1, t3.y, s2 * t4.y)));
@@ -295,7 +295,8 @@ template <typename T, int K> struct TwRegs {
     cplx<T> w[K];
 };
 
-template <typename T, int N, int TPP, int DIR, typename S, typename Addr, bool WAVE = false>
+// PIN: every product's contraction spelled out (cmul_pinned).
+template <typename T, int N, int TPP, int DIR, typename S, typename Addr, bool WAVE = false, bool PIN = false>
 struct PencilFFT {
     using Info = SeqInfo<S>;
     static constexpr int NP = Info::n;
@@ -366,10 +367,13 @@ struct PencilFFT {
                     for (int r = 1; r < R; r++) {
                         cplx<T> w = tr ? tr->w[tw_off(I) + q * (R - 1) + r - 1] : tw[r * jm * (N / (Ns * R))];
                         if (DIR > 0) w.y = -w.y;
-                        v[q * R + r] = cmul(v[q * R + r], w);
+                        v[q * R + r] = PIN ? cmul_pinned(v[q * R + r], w) : cmul(v[q * R + r], w);
                     }
                 }
-                Radix<R>::template dft<DIR>(v + q * R);
+                if constexpr (R == 5 && PIN)
+                    Radix<R>::template dft<DIR, true>(v + q * R);
+                else
+                    Radix<R>::template dft<DIR>(v + q * R);
             }
         }
     }

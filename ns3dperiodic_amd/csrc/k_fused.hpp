@@ -132,6 +132,8 @@ __device__ __forceinline__ bool member_idle(const MemberMask& m) { return m.left
 // grid.y enumerates the fields; with OS = 1 each block produces one output
 // (w_b or dx w_b) and the input is read by two blocks.
 // TS: scalar type of the state w (double, or float for the FP32-state RK3 loop).
+// VEC = 1 (NF = 2): the second vector field comes from a reduced Krylov vector, vec[c*(N-1)
+// + i-1] = Im v^_c[i] over the N modes of the reference layout (k_unpack_reduced's rule).
 // ADD = 1: the transformed field is w + w2 (w2 of the same type and layout; the
 // FP32-increment RK3 loop's stage value base + increment where no x-forward pass
 // leaves P1's output), summed in FP64.
@@ -145,13 +147,13 @@ using XInvPlan = typename std::conditional<MIRROR_P1<TB, NX>, typename SeqRev<ty
 template <typename TB> __device__ __forceinline__ cplx<TB> ikx(cplx<double> s, double kx) {
     return mk<TB>((TB)mul_rounded(-s.y, kx), (TB)mul_rounded(s.x, kx));
 }
-template <typename TB, int NX, int P, int NF, int E, int OS, typename TS = double, int ADD = 0>
+template <typename TB, int NX, int P, int NF, int E, int OS, typename TS = double, int ADD = 0, int VEC = 0>
 __global__ void __attribute__((amdgpu_waves_per_eu(NS3D_WAVES_XY, 8))) __launch_bounds__((P * XYPlan<NX, E>::TPP))
 k_x_inv_grad(PtrArr<const cplx<TS>, 3 * NF> w, cplx<TB>* __restrict__ A, long nc, int Ny, int Mz, int Mw, int Ms,
              int nlt, int nb, SpecTables tab, const cplx<TB>* __restrict__ twg, int nt, long bwi, long bsc,
-             MemberMask mm, PtrArr<const cplx<TS>, 3> w2 = {}) {
+             MemberMask mm, PtrArr<const cplx<TS>, 3> w2 = {}, const double* __restrict__ vec = nullptr) {
     constexpr int TPP = XYPlan<NX, E>::TPP;
-    using F = PencilFFT<TB, NX, TPP, +1, XInvPlan<TB, NX, E>, IndexMajor<P>>;
+    using F = PencilFFT<TB, NX, TPP, +1, XInvPlan<TB, NX, E>, IndexMajor<P>, false, sizeof(TB) == 8>;
     __shared__ cplx<TB> lds[NX * P];
     __shared__ cplx<TB> tw[NX];
     const int bid0 = xcd_tile();
@@ -186,7 +188,10 @@ k_x_inv_grad(PtrArr<const cplx<TS>, 3 * NF> w, cplx<TB>* __restrict__ A, long nc
             raw[i] = mk<TS>(0, 0);
             if constexpr (ADD != 0) raw2[i] = mk<TS>(0, 0);
             if (F::in_active(t, q) && keep && mask_keep(tab, j, k, l)) {
-                raw[i] = src[base + j * S];
+                if (VEC && f >= 3)   // (mode 0 is masked)
+                    raw[i].y = (TS)vec[(f - 3) * ((long)NX * Ny * Mz - 1) + base + j * S - 1];
+                else
+                    raw[i] = src[base + j * S];
                 if constexpr (ADD != 0) raw2[i] = src2[base + j * S];
             }
         }
@@ -640,9 +645,8 @@ struct ZPencil {
 template <typename TB, int NZ, int P, int NF>
 // The bilinear z pass (24 real fields per point): with its inputs through
 // buffer loads the FP32 pass fits 2 waves/SIMD in 240 VGPRs whatever the
-// bound; in FP64 2 waves/SIMD cost 92 B/lane of scratch spills at 256^3 and
-// still beat 1 wave with the overflow in AGPRs (256^3 tangent-map step
-// 10.13 -> 9.46 ms, 128^3 1.35 -> 1.31 ms).
+// bound; FP64 fits 2 waves/SIMD in 252, or spills there at the lengths that
+// run one pair at a time, which still beats 1 wave with the overflow in AGPRs.
 #ifndef NS3D_WAVES_Z2
 #define NS3D_WAVES_Z2 2
 #endif
@@ -682,7 +686,11 @@ k_z_product(const cplx<TB>* __restrict__ Bf, cplx<TB>* __restrict__ C, long nc, 
 #ifndef NS3D_ZTWFWD
 #define NS3D_ZTWFWD 1
 #endif
-    __shared__ cplx<TB> lds[(ILP ? 2 : 1) * P * (NZ + Z::PAD)];
+    // The bilinear pass in FP64 at the same lengths, its pairs two at a time as well: 128^3
+    // 0.119 -> 0.096 ms, 256^3 0.95 -> 0.71 (where one pair at a time spilled 92 B a lane and
+    // waited for its loads); at the other lengths two pairs spill more (160^3 0.49 -> 0.64).
+    constexpr bool ILP2 = NF == 2 && sizeof(TB) == 8 && ((NZ & (NZ - 1)) == 0 || (NZ % 3 == 0 && Z::WAVE));
+    __shared__ cplx<TB> lds[(ILP || ILP2 ? 2 : 1) * P * (NZ + Z::PAD)];
     __shared__ cplx<TB> tw[NZ];
     const int bid0 = xcd_tile();
     if (bid0 >= nb || member_idle(mm)) return;
@@ -820,6 +828,61 @@ k_z_product(const cplx<TB>* __restrict__ Bf, cplx<TB>* __restrict__ C, long nc, 
         run_pair(a, b, false, true, -1, -1);        // dy w_z, dz w_z
 #pragma unroll
         for (int e = 0; e < NPT; e++) Q[2][e] = w[0][e] * Q[2][e] + w[1][e] * a[e] + w[2][e] * b[e];
+    } else if constexpr (ILP2) {
+        // As the last branch below, two paired transforms at a time with the inputs of the
+        // next two in flight (one u-derived, one v-derived pair).
+        cplx<TB>* lb = lds + P * (NZ + Z::PAD);
+        TB u[3][NPT], vv[3][NPT], a[NPT], b[NPT], c[NPT], d[NPT];
+        TB kz[Z::NIN];
+        cplx<TB> r1[Z::NIN], r2[Z::NIN], r3[Z::NIN], r4[Z::NIN];
+        Z::kz_regs(kz, tab, t);
+        fetch(r1, r2, 0, 1);
+        fetch(r3, r4, 9, 10);
+        auto run_two = [&](TB* x1, TB* x2, bool d1, bool d2, TB* x3, TB* x4, int n1, int n2, int n3, int n4) {
+            cplx<TB> va[Z::E], vb[Z::E];
+            Z::finish_pair(va, r1, d1, r2, d2, kz, t);
+            Z::finish_pair(vb, r3, d1, r4, d2, kz, t);
+            if (n1 >= 0) {
+                fetch(r1, r2, n1, n2);
+                fetch(r3, r4, n3, n4);
+            }
+            Z::FI::run2(va, vb, lds, lb, tw, t, p);
+#pragma unroll
+            for (int e = 0; e < NPT; e++) {
+                x1[e] = va[e].x * scale;
+                x2[e] = va[e].y * scale;
+                x3[e] = vb[e].x * scale;
+                x4[e] = vb[e].y * scale;
+            }
+        };
+        run_two(u[0], u[1], false, false, vv[0], vv[1], 2, 3, 11, 12);
+        run_two(u[2], a, false, false, vv[2], c, 6, 0, 15, 9);        // u_z, dx u_x; v_z, dx v_x
+#pragma unroll
+        for (int e = 0; e < NPT; e++) Q[0][e] = vv[0][e] * a[e] + u[0][e] * c[e];
+        run_two(a, b, false, true, c, d, 4, 7, 13, 16);               // dy, dz of u_x; of v_x
+#pragma unroll
+        for (int e = 0; e < NPT; e++) {
+            Q[0][e] += vv[1][e] * a[e] + vv[2][e] * b[e];
+            Q[0][e] += u[1][e] * c[e] + u[2][e] * d[e];
+        }
+        run_two(a, b, false, false, c, d, 1, 5, 10, 14);              // dx, dy of u_y; of v_y
+#pragma unroll
+        for (int e = 0; e < NPT; e++) {
+            Q[1][e] = vv[0][e] * a[e] + vv[1][e] * b[e];
+            Q[1][e] += u[0][e] * c[e] + u[1][e] * d[e];
+        }
+        run_two(a, b, true, false, c, d, 8, 2, 17, 11);               // dz u_y, dx u_z; dz v_y, dx v_z
+#pragma unroll
+        for (int e = 0; e < NPT; e++) {
+            Q[1][e] += vv[2][e] * a[e] + u[2][e] * c[e];
+            Q[2][e] = vv[0][e] * b[e] + u[0][e] * d[e];
+        }
+        run_two(a, b, false, true, c, d, -1, -1, -1, -1);             // dy, dz of u_z; of v_z
+#pragma unroll
+        for (int e = 0; e < NPT; e++) {
+            Q[2][e] += vv[1][e] * a[e] + vv[2][e] * b[e];
+            Q[2][e] += u[1][e] * c[e] + u[2][e] * d[e];
+        }
     } else {
         // Q_c = (v.grad) u_c + (u.grad) v_c  (convolute_2p3_UV, Source/advection_2_3.cu:401-475).
         // Each paired transform holds two u-derived or two v-derived fields,
@@ -930,6 +993,8 @@ k_axis_c2c(const cplx<TB>* in, cplx<TB>* out, int nf, long nc, int Ny, int Mz, i
 // ---------------------------------------------------------------- P5 epilogues
 // EPI_STAGE32: EPI_STAGE with w, u0 and out in FP32 (the FP32-state RK3 loop);
 // the arithmetic and the forcing stay FP64.
+// EPI_UV_VEC: EPI_UV_RHS with v read from a reduced Krylov vector (vin, k_unpack_reduced's
+// rule) and Im(r) - shift*Im(v) written to another (vout, k_pack_reduced's rule).
 // EPI_INC / EPI_INC_FINAL: the SSP stages in increment form over a base state
 // u^n held as a pair of FP32 fields, u^n = hi + lo (the FP32-increment RK3
 // loop).  With w = base + d (d: the previous stage's FP32 increment, u0; null
@@ -943,7 +1008,7 @@ k_axis_c2c(const cplx<TB>* in, cplx<TB>* out, int nf, long nc, int Ny, int Mz, i
 // by one thread).
 enum EpiMode {
     EPI_Q = 0, EPI_STAGE = 1, EPI_RHS = 2, EPI_UV = 3, EPI_UV_RHS = 4, EPI_IUV = 5, EPI_STAGE32 = 6,
-    EPI_INC = 7, EPI_INC_FINAL = 8
+    EPI_INC = 7, EPI_INC_FINAL = 8, EPI_UV_VEC = 9
 };
 
 struct EpiArgs {
@@ -966,6 +1031,10 @@ struct EpiArgs {
     int* nf;
     // EPI_INC_FINAL: the lo half of the state (read and written), rows of stride mw
     cplx<float>* out32[3];
+    // EPI_UV_VEC (may be one vector)
+    const double* vin;
+    double* vout;
+    double shift;
 };
 
 // Non-finite flag of the fused epilogues and the scalar stage: every lane that
@@ -1215,16 +1284,23 @@ k_x_fwd_epi(const cplx<TB>* D, cplx<TB>* A, long nc, int Ny, int Mz, int Ms, int
     auto voff = [&](int m, int esz, int q) __attribute__((always_inline)) {
         return lv && F::out_active(t, q) ? ((t * Ny + k) * m + l) * esz : BUF_OOB;
     };
+    // reduced vectors: element i of component b at (vec - 1 + b*(N-1))[i], none for i = 0
+    auto rsrc_vec = [&](const double* vec, int b) __attribute__((always_inline)) {
+        return buf_rsrc(vec - 1 + (long)b * (nrow * Mz - 1), (int)(nrow * Mz * 8));
+    };
+    auto voff_vec = [&](int j, int q) __attribute__((always_inline)) { return (j | k | l) == 0 ? BUF_OOB : voff(Mz, 8, q); };
     auto load_unit = [&](auto UC) __attribute__((always_inline)) {
         constexpr int u = decltype(UC)::value, b = u / UPC, e0 = (u % UPC) * UM;
         EpiUnit<MODE, UM>& U = un[u % RING];
         constexpr int es = (int)sizeof(cplx<TS>);
-        const auto rw = rsrc_of(ea.w[b], z * ea.bw, ea.mw, es);
+        const auto rw = MODE == EPI_UV_VEC ? rsrc_vec(ea.vin, b) : rsrc_of(ea.w[b], z * ea.bw, ea.mw, es);
 #pragma unroll
         for (int i = 0; i < UM; i++) {
             const int e = e0 + i;
             const int q = e / F::RL, so = F::out_index(0, q, e % F::RL) * Ny;
-            if constexpr (MODE != EPI_Q) U.w[i] = buf_load<TS>(rw, voff(ea.mw, es, q), so * ea.mw * es);
+            if constexpr (MODE == EPI_UV_VEC)
+                U.w[i] = mk<TS>(0, (TS)buf_load_f64(rw, voff_vec(F::out_index(t, q, e % F::RL), q), so * Mz * 8));
+            else if constexpr (MODE != EPI_Q) U.w[i] = buf_load<TS>(rw, voff(ea.mw, es, q), so * ea.mw * es);
         }
         if constexpr (HAS_U0) {
             if (ea.u0[b]) {
@@ -1273,7 +1349,7 @@ k_x_fwd_epi(const cplx<TB>* D, cplx<TB>* A, long nc, int Ny, int Mz, int Ms, int
     // projection: AM Q - Q with AM Q = kv (kv.Q)/|k|^2.  FP64: R replaces Q;
     // FP32: Q stays in FP32 and kd = (kv.Q)/|k|^2 is kept in FP64.
     cplx<double> kd[(F64 || MODE == EPI_Q) ? 1 : NO];
-    const double qs = MODE == EPI_RHS || MODE == EPI_UV_RHS ? 1.0 : ea.dt;   // weight of (AM Q - Q)
+    const double qs = MODE == EPI_RHS || MODE == EPI_UV_RHS || MODE == EPI_UV_VEC ? 1.0 : ea.dt;   // weight of (AM Q - Q)
 #pragma unroll
     for (int e = 0; e < NO; e++) {
         const int j = F::out_index(t, e / F::RL, e % F::RL);
@@ -1319,7 +1395,7 @@ k_x_fwd_epi(const cplx<TB>* D, cplx<TB>* A, long nc, int Ny, int Mz, int Ms, int
         if constexpr (F64) {
             // the mirror-image plan: its first pass reads what the last forward pass holds
             static_assert(!CHAIN || MIRROR_P1<TB, NX>, "the standalone P1 runs the same plan");
-            using FI = PencilFFT<TB, NX, TPP, +1, XInvPlan<TB, NX, E>, IndexMajor<P>>;
+            using FI = PencilFFT<TB, NX, TPP, +1, XInvPlan<TB, NX, E>, IndexMajor<P>, false, true>;
             FI::run2(v, d, lds, lds + NX * P, tw, t, p);
             put(FI{}, v, b, t);
             put(FI{}, d, 3 + b, t);
@@ -1368,7 +1444,7 @@ k_x_fwd_epi(const cplx<TB>* D, cplx<TB>* A, long nc, int Ny, int Mz, int Ms, int
         constexpr int es = (int)sizeof(cplx<TS>);
         // UV, UV_RHS and IUV update w in place
         constexpr bool INPLACE = MODE == EPI_UV || MODE == EPI_UV_RHS || MODE == EPI_IUV || MODE == EPI_INC_FINAL;
-        const int mo = INPLACE ? ea.mw : ea.mo;
+        const int mo = INPLACE ? ea.mw : ea.mo;   // (EPI_UV_VEC stores through its own resource)
         const auto ro = rsrc_of(INPLACE ? ea.w[b] : ea.out[b], INPLACE ? z * ea.bw : z * ea.bo, mo, es);
 #pragma unroll
         for (int i = 0; i < UM; i++) {
@@ -1427,6 +1503,12 @@ k_x_fwd_epi(const cplx<TB>* D, cplx<TB>* A, long nc, int Ny, int Mz, int Ms, int
                     r.y = R.y + G * w.y;
                     if constexpr (MODE == EPI_RHS) r = r + U.f[i];
                     buf_store<double>(ro, r, vo, so);
+                    bad |= vo >= 0 && !finite2(r);
+                } else if constexpr (MODE == EPI_UV_VEC) {
+                    const double G = -k2 * ea.nu;
+                    r = mk<double>(R.x + G * w.x, R.y + G * w.y);
+                    const int vv = voff_vec(j, q);
+                    buf_store_f64(rsrc_vec(ea.vout, b), ea.shift != 0.0 ? r.y - ea.shift * w.y : r.y, vv, jo * Ny * Mz * 8);
                     bad |= vo >= 0 && !finite2(r);
                 } else if constexpr (MODE == EPI_UV) {
                     const double G = 1.0 - k2 * ea.dtnu;

@@ -125,16 +125,6 @@ k_pack_full(PtrArr<const cplx<double>, 3> v, double* __restrict__ vec, long N) {
 #pragma unroll
     for (int c = 0; c < 3; c++) vec[c * N + i] = v.p[c][i].y;
 }
-// A_vector_add_diagonal_kernel (:296-310) and the shifted pack (:253-270).
-__global__ void __launch_bounds__(256)
-k_pack_reduced_shifted(PtrArr<const cplx<double>, 3> v, const double* __restrict__ vin, double shift,
-                       double* __restrict__ vec, long N) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N - 1) return;
-#pragma unroll
-    for (int c = 0; c < 3; c++) vec[c * (N - 1) + i] = v.p[c][i + 1].y - shift * vin[c * (N - 1) + i];
-}
-
 // ------------------------------------------------------- a9: WENO advection
 // Reference: Source/advection_WENO.cu:47-101 (weno5/weno3), :105-301 (faces), :304-360 (flux).
 // The nonlinear weights alpha_k = c_k / (eps + beta_k)^2 normalised by their

@@ -253,9 +253,11 @@ template <typename TB> int nt_for(const ns3d_ctx* c, int P, double fields) {
 constexpr double FIELDS_P1 = 3.6, FIELDS_P2 = 6.0, FIELDS_P34 = 3.0;
 
 // ---------------------------------------------------------------- launches by length
-// P1 of nf fields (in2: nf = 1 only, may be null: added to in before the transforms)
+// P1 of nf fields (in2: nf = 1 only, may be null: added to in before the transforms;
+// vec: nf = 2 only, may be null: the second vector field as a reduced Krylov vector)
 template <typename TB, typename TS, int NX>
-int launch_x_inv(ns3d_ctx* c, const cplx<TS>* const* in, const cplx<TS>* const* in2, int nf, int mw, long bin);
+int launch_x_inv(ns3d_ctx* c, const cplx<TS>* const* in, const cplx<TS>* const* in2, int nf, int mw, long bin,
+                 const double* vec);
 template <typename TB, int NY> int launch_y_inv(ns3d_ctx* c, int nf);
 template <typename TB, int NZ> int launch_z(ns3d_ctx* c, int nf);
 template <typename TB, int NY> int launch_y_fwd(ns3d_ctx* c, int nf);

@@ -5,7 +5,8 @@
 #include "launch.hpp"
 
 template <typename TB, typename TS, int NX>
-int launch_x_inv(ns3d_ctx* c, const cplx<TS>* const* in, const cplx<TS>* const* in2, int nf, int mw, long bin) {
+int launch_x_inv(ns3d_ctx* c, const cplx<TS>* const* in, const cplx<TS>* const* in2, int nf, int mw, long bin,
+                 const double* vec) {
     const int nz = c->batch, Mi = mi_of(c);
     const long nc = c->nci, bsc = c->bsc;
     cplx<TB>* A = (cplx<TB>*)c->scratch;
@@ -31,8 +32,13 @@ int launch_x_inv(ns3d_ctx* c, const cplx<TS>* const* in, const cplx<TS>* const* 
                            twp<TB>(c, 0), nt_for<TB>(c, P, FIELDS_P1 * nf), bin, bsc, c->mm);
     } else if constexpr (std::is_same<TS, double>::value) {
         PtrArr<const zd, 6> w{{in[0], in[1], in[2], in[3], in[4], in[5]}};
-        hipLaunchKernelGGL((k_x_inv_grad<TB, NX, P, 2, E, OS>), grid, blk, 0, s, w, A, nc, c->Ny, c->Mz, mw, Mi, nlt, nb, c->tab,
-                           twp<TB>(c, 0), nt_for<TB>(c, P, FIELDS_P1 * nf), bin, bsc, c->mm);
+        if (vec)
+            hipLaunchKernelGGL((k_x_inv_grad<TB, NX, P, 2, E, OS, double, 0, 1>), grid, blk, 0, s, w, A, nc, c->Ny, c->Mz, c->Mz, Mi,
+                               nlt, nb, c->tab, twp<TB>(c, 0), nt_for<TB>(c, P, FIELDS_P1 * nf), 0L, bsc, c->mm,
+                               PtrArr<const zd, 3>{}, vec);
+        else
+            hipLaunchKernelGGL((k_x_inv_grad<TB, NX, P, 2, E, OS>), grid, blk, 0, s, w, A, nc, c->Ny, c->Mz, mw, Mi, nlt, nb, c->tab,
+                               twp<TB>(c, 0), nt_for<TB>(c, P, FIELDS_P1 * nf), bin, bsc, c->mm);
     } else {
         return NS3D_ERR_ARG;
     }

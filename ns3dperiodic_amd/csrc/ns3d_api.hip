@@ -258,16 +258,17 @@ bool can_chain(const ns3d_ctx* c) {
 // has_a: the previous stage's x-forward pass left P1's output in A (CHAIN), in is not read.
 // in2 (nf = 1 only, may be null): a second field of in's type and layout added
 // to the input before the transforms (the FP32-increment loop's base + increment).
+// vec (nf = 2 only, may be null): the second vector field as a reduced Krylov vector.
 template <typename TB, typename TS = double>
 int run_nonlinear_passes(ns3d_ctx* c, const cplx<TS>* const* in, int nf, int mw = 0, long bin = 0, bool has_a = false,
-                         const cplx<TS>* const* in2 = nullptr) {
+                         const cplx<TS>* const* in2 = nullptr, const double* vec = nullptr) {
     has_a = has_a && can_chain(c);
     if (mw == 0) mw = c->Mz;
     int st = ensure_scratch(c, 15 * nf * c->batch);
     if (st) return st;
     if (!has_a) {
         prof_begin(c, 0);
-        st = with_size(c->Nx, [&](auto N) { return launch_x_inv<TB, TS, decltype(N)::value>(c, in, in2, nf, mw, bin); });
+        st = with_size(c->Nx, [&](auto N) { return launch_x_inv<TB, TS, decltype(N)::value>(c, in, in2, nf, mw, bin, vec); });
         prof_end(c);
         if (st) return st;
     }
@@ -319,11 +320,11 @@ template <int MODE>
 int fused(ns3d_ctx* c, const zd* const* in, int nf, const EpiArgs& ea, bool has_a = false, bool chain = false) {
     int st;
     if (c->precision == NS3D_FP64) {
-        st = run_nonlinear_passes<double>(c, in, nf, ea.mw, ea.bw, has_a);
+        st = run_nonlinear_passes<double, double>(c, in, nf, ea.mw, ea.bw, has_a, (const zd* const*)nullptr, ea.vin);
         if (st) return st;
         st = run_x_forward_epilogue<double, MODE>(c, ea, nf, chain);
     } else {
-        st = run_nonlinear_passes<float>(c, in, nf, ea.mw, ea.bw, has_a);
+        st = run_nonlinear_passes<float, double>(c, in, nf, ea.mw, ea.bw, has_a, (const zd* const*)nullptr, ea.vin);
         if (st) return st;
         st = run_x_forward_epilogue<float, MODE>(c, ea, nf, chain);
     }
@@ -1345,12 +1346,26 @@ int ns3d_rk3_ssp_uv(ns3d_ctx* c, ns3d_cplx* ux, ns3d_cplx* uy, ns3d_cplx* uz, ns
     int st = ensure_fp64(c, &c->extra, 6);
     if (st) return st;
     zd* v1[3] = {c->extra, c->extra + c->nc, c->extra + 2 * c->nc};
-    // RK3_SSP_UV (Source/RK_time_step.cu:342-355)
-    if ((st = ns3d_copy3(c, vx, vy, vz, (ns3d_cplx*)v1[0], (ns3d_cplx*)v1[1], (ns3d_cplx*)v1[2]))) return st;
-    if ((st = ns3d_stage_uv(c, ux, uy, uz, (ns3d_cplx*)v1[0], (ns3d_cplx*)v1[1], (ns3d_cplx*)v1[2]))) return st;
+    // RK3_SSP_UV (Source/RK_time_step.cu:342-355): v1 = E(v) about u, u one step on,
+    // v = v/2 + E(v1)/2 about the new u; the copy and the combination are in the epilogues
+    const zd* uu[3] = {(const zd*)ux, (const zd*)uy, (const zd*)uz};
+    const zd* vv[3] = {(const zd*)vx, (const zd*)vy, (const zd*)vz};
+    auto stage = [&](const zd* const w[3], const zd* const u0[3], zd* const out[3]) -> int {
+        const zd* in[6] = {uu[0], uu[1], uu[2], w[0], w[1], w[2]};
+        EpiArgs ea = make_epi(c);
+        for (int b = 0; b < 3; b++) {
+            ea.w[b] = (zd*)w[b];
+            ea.u0[b] = u0 ? u0[b] : nullptr;
+            ea.out[b] = out[b];
+        }
+        if (u0) ea.a0 = ea.a1 = 0.5;
+        return fused<EPI_STAGE>(c, in, 2, ea);
+    };
+    const zd* v1c[3] = {v1[0], v1[1], v1[2]};
+    zd* vo[3] = {(zd*)vx, (zd*)vy, (zd*)vz};
+    if ((st = stage(vv, nullptr, v1))) return st;
     if ((st = ns3d_rk3_ssp(c, ux, uy, uz, fx, fy, fz))) return st;
-    if ((st = ns3d_stage_uv(c, ux, uy, uz, (ns3d_cplx*)v1[0], (ns3d_cplx*)v1[1], (ns3d_cplx*)v1[2]))) return st;
-    return ns3d_axpby3(c, vx, vy, vz, 0.5, (ns3d_cplx*)v1[0], (ns3d_cplx*)v1[1], (ns3d_cplx*)v1[2], 0.5, vx, vy, vz);
+    return stage(v1c, vv, vo);
 }
 
 int ns3d_unpack_reduced(ns3d_ctx* c, const double* vec, ns3d_cplx* vx, ns3d_cplx* vy, ns3d_cplx* vz) {
@@ -1401,19 +1416,15 @@ int ns3d_set_base_state(ns3d_ctx* c, ns3d_cplx* ux, ns3d_cplx* uy, ns3d_cplx* uz
 namespace {
 int jv_reduced_impl(ns3d_ctx* c, const double* in, double* out, bool newton) {
     if (!c || !in || !out || !c->base[0] || !c->kry) return NS3D_ERR_ARG;
-    ns3d_cplx* v[3] = {(ns3d_cplx*)c->kry, (ns3d_cplx*)(c->kry + c->nc), (ns3d_cplx*)(c->kry + 2 * c->nc)};
-    ns3d_cplx* u[3] = {(ns3d_cplx*)c->base[0], (ns3d_cplx*)c->base[1], (ns3d_cplx*)c->base[2]};
-    int st;
-    // NSCallMatrixVector_reduced (Source/NS3D_periodic.cu:340-361)
-    if ((st = ns3d_unpack_reduced(c, in, v[0], v[1], v[2]))) return st;
-    if ((st = ns3d_rk3_ssp_uv_rhs(c, u[0], u[1], u[2], v[0], v[1], v[2]))) return st;
-    if (!newton) return ns3d_pack_reduced(c, v[0], v[1], v[2], out);
-    // ..._Newton_Globalization (:364-389): out = pack(J v) - v/tau
-    PtrArr<const zd, 3> vv{{(const zd*)v[0], (const zd*)v[1], (const zd*)v[2]}};
-    hipLaunchKernelGGL(k_pack_reduced_shifted, dim3(nblk(c->nc, 256)), dim3(256), 0, c->stream, vv, in, 1.0 / c->tau,
-                       out, c->nc);
-    HIPCHK(hipGetLastError());
-    return NS3D_OK;
+    // NSCallMatrixVector_reduced (Source/NS3D_periodic.cu:340-361) and
+    // ..._Newton_Globalization (:364-389: out = pack(J v) - v/tau); the passes at both
+    // ends read and write the vectors themselves
+    const zd* in6[6] = {c->base[0], c->base[1], c->base[2], nullptr, nullptr, nullptr};
+    EpiArgs ea = make_epi(c);
+    ea.vin = in;
+    ea.vout = out;
+    ea.shift = newton ? 1.0 / c->tau : 0.0;
+    return fused<EPI_UV_VEC>(c, in6, 2, ea);
 }
 }  // namespace
 

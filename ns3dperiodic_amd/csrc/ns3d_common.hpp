@@ -19,14 +19,11 @@ struct alignas(2 * sizeof(T)) cplx {
 template <typename T> __device__ __forceinline__ cplx<T> mk(T a, T b) { cplx<T> r; r.x = a; r.y = b; return r; }
 template <typename T> __device__ __forceinline__ cplx<T> operator+(cplx<T> a, cplx<T> b) { return mk<T>(a.x + b.x, a.y + b.y); }
 template <typename T> __device__ __forceinline__ cplx<T> operator-(cplx<T> a, cplx<T> b) { return mk<T>(a.x - b.x, a.y - b.y); }
-// FP64: the fused multiply-adds are spelled out, so that every kernel rounds a product alike
-// (a transform fused into one kernel is bitwise the one another kernel makes); FP32 leaves
-// the choice to the compiler.
-template <typename T> __device__ __forceinline__ cplx<T> cmul(cplx<T> a, cplx<T> b) {
-    if constexpr (sizeof(T) == 8)
-        return mk<T>(__builtin_fma(a.x, b.x, -(a.y * b.y)), __builtin_fma(a.x, b.y, a.y * b.x));
-    else
-        return mk<T>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+template <typename T> __device__ __forceinline__ cplx<T> cmul(cplx<T> a, cplx<T> b) { return mk<T>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
+// The same with the fused multiply-adds spelled out, for transforms that two kernels have to
+// round alike (elsewhere the compiler's own choice gives shorter schedules).
+template <typename T> __device__ __forceinline__ cplx<T> cmul_pinned(cplx<T> a, cplx<T> b) {
+    return mk<T>(__builtin_fma(a.x, b.x, -(a.y * b.y)), __builtin_fma(a.x, b.y, a.y * b.x));
 }
 // A product rounded by itself, never contracted into a following addition.
 template <typename T> __device__ __forceinline__ T mul_rounded(T a, T b) {
@@ -83,6 +80,17 @@ __device__ __forceinline__ void buf_store(__amdgpu_buffer_rsrc_t r, cplx<T> a, i
     }
 }
 
+__device__ __forceinline__ double buf_load_f64(__amdgpu_buffer_rsrc_t r, int off, int so) {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, off, so, 0);
+    double a;
+    __builtin_memcpy(&a, &v, sizeof(a));
+    return a;
+}
+__device__ __forceinline__ void buf_store_f64(__amdgpu_buffer_rsrc_t r, double a, int off, int so) {
+    buf_u32x2 v;
+    __builtin_memcpy(&v, &a, sizeof(a));
+    __builtin_amdgcn_raw_buffer_store_b64(v, r, off, so, 0);
+}
 template <bool NT, typename T> __device__ __forceinline__ void st_cplx(cplx<T>* p, cplx<T> a) {
     if constexpr (NT) {
         typedef T v2 __attribute__((ext_vector_type(2)));

@@ -6,7 +6,7 @@
     template int launch_x_fwd<double, MODE, N>(ns3d_ctx*, const EpiArgs&, int, bool); \
     template int launch_x_fwd<float, MODE, N>(ns3d_ctx*, const EpiArgs&, int, bool);
 #define PASSES(T, N)                                                             \
-    template int launch_x_inv<T, double, N>(ns3d_ctx*, const zd* const*, const zd* const*, int, int, long); \
+    template int launch_x_inv<T, double, N>(ns3d_ctx*, const zd* const*, const zd* const*, int, int, long, const double*); \
     template int launch_y_inv<T, N>(ns3d_ctx*, int);                             \
     template int launch_z<T, N>(ns3d_ctx*, int);                                 \
     template int launch_y_fwd<T, N>(ns3d_ctx*, int);                             \
@@ -16,12 +16,13 @@
 #define L(N)                                                                     \
     PASSES(double, N)                                                            \
     PASSES(float, N)                                                             \
-    template int launch_x_inv<float, float, N>(ns3d_ctx*, const cplx<float>* const*, const cplx<float>* const*, int, int, long); \
+    template int launch_x_inv<float, float, N>(ns3d_ctx*, const cplx<float>* const*, const cplx<float>* const*, int, int, long, const double*); \
     EPI_BOTH(N, EPI_Q)                                                           \
     EPI_BOTH(N, EPI_STAGE)                                                       \
     EPI_BOTH(N, EPI_RHS)                                                         \
     EPI_BOTH(N, EPI_UV)                                                          \
     EPI_BOTH(N, EPI_UV_RHS)                                                      \
+    EPI_BOTH(N, EPI_UV_VEC)                                                      \
     EPI_BOTH(N, EPI_IUV)                                                         \
     template int launch_x_fwd<float, EPI_STAGE32, N>(ns3d_ctx*, const EpiArgs&, int, bool); \
     template int launch_x_fwd<float, EPI_INC, N>(ns3d_ctx*, const EpiArgs&, int, bool);    \
