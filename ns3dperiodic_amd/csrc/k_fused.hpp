@@ -1239,20 +1239,6 @@ k_x_fwd_epi(const cplx<TB>* D, cplx<TB>* A, long nc, int Ny, int Mz, int Ms, int
     const long z = blockIdx.z;           // batch member
     D += z * bsc;
     A += z * bsc;
-    // chain: the masked modes of this thread's column, and whether any lane has some
-    unsigned kept = 0;
-    bool chained = false;
-    if constexpr (CHAIN) {
-        const bool col = lv && column_kept(tab, k, l);
-        chained = __syncthreads_or(col);
-        if (col) {
-#pragma unroll
-            for (int e = 0; e < NO; e++) {
-                const int q = e / F::RL, j = F::out_index(t, q, e % F::RL);
-                if (F::out_active(t, q) && mask_keep(tab, j, k, l)) kept |= 1u << e;
-            }
-        }
-    }
     // D: this thread's elements, plane stride Ny*Ms
     const int strD = Ny * Ms * (int)sizeof(cplx<TB>);
     const int offD = lv ? (k * Ms + l) * (int)sizeof(cplx<TB>) : BUF_OOB;
@@ -1340,11 +1326,28 @@ k_x_fwd_epi(const cplx<TB>* D, cplx<TB>* A, long nc, int Ny, int Mz, int Ms, int
             }
         }
     };
-    // the first RING - 1 units are in flight while the transforms run
+    // chain: the masked modes of this thread's column, and whether any lane has some
+    unsigned kept = 0;
+    bool chained = false;
+    bool col = false;
+    if constexpr (CHAIN) {
+        col = lv && column_kept(tab, k, l);
+        if (col) {
+#pragma unroll
+            for (int e = 0; e < NO; e++) {
+                const int q = e / F::RL, j = F::out_index(t, q, e % F::RL);
+                if (F::out_active(t, q) && mask_keep(tab, j, k, l)) kept |= 1u << e;
+            }
+        }
+    }
+    const double ky = tab.ky[k], kz = lv ? tab.kz[l] : 0.0;
+    // the first RING - 1 units are in flight while the transforms run; the block-wide vote
+    // waits for the mask, so it comes after them (before D's loads: 32^3 step 80.9 us, here
+    // 79.6; 256^3 3.88 ms, here 3.85)
     if constexpr (MODE != EPI_Q) static_for<0, RING - 1>([&](auto UC) __attribute__((always_inline)) { load_unit(UC); });
+    if constexpr (CHAIN) chained = __syncthreads_or(col);
     F::run2(qv[0], qv[1], lds, lds + NX * P, tw, t, p);
     F::run(qv[2], lds, tw, t, p);
-    const double ky = tab.ky[k], kz = lv ? tab.kz[l] : 0.0;
     const double kyz2 = ky * ky + kz * kz;
     // projection: AM Q - Q with AM Q = kv (kv.Q)/|k|^2.  FP64: R replaces Q;
     // FP32: Q stays in FP32 and kd = (kv.Q)/|k|^2 is kept in FP64.
@@ -1378,7 +1381,6 @@ k_x_fwd_epi(const cplx<TB>* D, cplx<TB>* A, long nc, int Ny, int Mz, int Ms, int
     }
     // chain: inverse transforms of one component's w and dx w, stored to A
     auto chain = [&](int b, cplx<TB>* v, cplx<TB>* d) __attribute__((always_inline)) {
-        const bool col = lv && column_kept(tab, k, l);
         auto put = [&](auto FC, cplx<TB>* x, int field, int ti) __attribute__((always_inline)) {
             using FX = decltype(FC);
             const auto ra = buf_rsrc(A + (long)field * nc, bytesD);
