@@ -237,13 +237,14 @@ k_x_inv_grad(PtrArr<const cplx<TS>, 3 * NF> w, cplx<TB>* __restrict__ A, long nc
 // ---------------------------------------------------------------- P2
 // y-inverse: B(w_b) , B(dx w_b) , B(i ky w_b).  Block: one x index j and P z
 // indices.  grid.y enumerates components; with OS = 1 each block produces one
-// of the three outputs (A_b is then read by two blocks).
+// of the three outputs (A_b is then read by two blocks): a third of the serial
+// chain of a block, for grids whose blocks all fit the chip at once (launch_y_inv).
 template <typename TB, int NY, int P, int NF, int E, int OS>
 __global__ void __attribute__((amdgpu_waves_per_eu(NS3D_WAVES_XY, 8))) __launch_bounds__((P * XYPlan<NY, E>::TPP))
 k_y_inv_grad(const cplx<TB>* __restrict__ A, cplx<TB>* __restrict__ B, long nc, int Ny, int Mz, int Ms, int nlt,
              int nb, SpecTables tab, const cplx<TB>* __restrict__ twg, int nt, long bsc, MemberMask mm) {
     constexpr int TPP = XYPlan<NY, E>::TPP;
-    using F = PencilFFT<TB, NY, TPP, +1, typename XYPlan<NY, E>::R, IndexMajor<P>>;
+    using F = PencilFFT<TB, NY, TPP, +1, typename XYPlan<NY, E>::R, IndexMajor<P>, false, sizeof(TB) == 8>;
     __shared__ cplx<TB> lds[NY * P];
     __shared__ cplx<TB> tw[NY];
     const int bid0 = xcd_tile();
@@ -302,7 +303,8 @@ k_y_inv_grad(const cplx<TB>* __restrict__ A, cplx<TB>* __restrict__ B, long nc, 
                 const int kk = F::in_index(t, q, r);
                 const cplx<TB> s = v[q * F::R0 + r];
                 const TB ky = F::in_active(t, q) ? (TB)tab.ky[kk] : (TB)0;
-                const cplx<TB> dv = mk<TB>(-s.y * ky, s.x * ky);
+                // (FP64: rounded products and pinned transforms, both forms of the pass give the same bits)
+                const cplx<TB> dv = sizeof(TB) == 8 ? mk<TB>(mul_rounded(-s.y, ky), mul_rounded(s.x, ky)) : mk<TB>(-s.y * ky, s.x * ky);
                 if constexpr (OS) {
                     v[q * F::R0 + r] = which ? dv : s;
                 } else {

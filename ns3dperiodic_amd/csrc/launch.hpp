@@ -80,9 +80,6 @@ template <typename TB, int N> constexpr int E_XFWD = sizeof(TB) == 8 ? (N > 256 
 #ifndef NS3D_OS_XINV
 #define NS3D_OS_XINV 0
 #endif
-#ifndef NS3D_OS_YINV
-#define NS3D_OS_YINV 0
-#endif
 // pencils per block in the z pass: ~128 threads (FP32: NS3D_PZT32)
 #ifndef NS3D_PZT32
 #define NS3D_PZT32 128

@@ -57,14 +57,29 @@ int launch_y_inv(ns3d_ctx* c, int nf) {
                             NS3D_BY_RADIX(NY, NS3D_PYINV64, NS3D_R3_PYINV64)>;
     const int nlt = (c->Mz + P - 1) / P;
     const int nb = c->Nx * nlt;
-    constexpr int OS = NS3D_OS_YINV;
-    dim3 grid = xgrid(nb, 3 * nf * (OS ? 3 : 1), nz), blk(P * XYPlan<NY, E>::TPP);
-    if (nf == 1)
-        hipLaunchKernelGGL((k_y_inv_grad<TB, NY, P, 1, E, OS>), grid, blk, 0, s, A, B, nc, c->Ny, c->Mz, Mi, nlt, nb, c->tab,
-                           twp<TB>(c, 1), nt_for<TB>(c, P, FIELDS_P2 * nf), bsc, c->mm);
-    else
-        hipLaunchKernelGGL((k_y_inv_grad<TB, NY, P, 2, E, OS>), grid, blk, 0, s, A, B, nc, c->Ny, c->Mz, Mi, nlt, nb, c->tab,
-                           twp<TB>(c, 1), nt_for<TB>(c, P, FIELDS_P2 * nf), bsc, c->mm);
+    // One output per block (OS) where even three times the blocks leave every wave resident
+    // at once, so that a block's latency is the pass's time: FP64 32^3 step 79.6 -> 73.9 us,
+    // 48x64x32 111.6 -> 105.9, 96^3 281 -> 267; 128^3 (two rounds) 493 -> 500.  FP32 rounds
+    // differently in the two forms and keeps one.
+    constexpr int T = P * XYPlan<NY, E>::TPP;
+    constexpr long RESIDENT = 5 * 1024;   // waves at 5 to a SIMD
+    const long tiles = (long)c->Nx * (c->tab.lmax / P + 1) * c->batch;
+    const bool os = sizeof(TB) == 8 && nf == 1 && 9 * tiles * ((T + 63) / 64) <= RESIDENT;
+    const dim3 grid = xgrid(nb, 3 * nf, nz), blk(T);
+    const int nt = nt_for<TB>(c, P, FIELDS_P2 * nf);
+    auto launch = [&](auto kernel, dim3 g) {
+        hipLaunchKernelGGL(kernel, g, blk, 0, s, A, B, nc, c->Ny, c->Mz, Mi, nlt, nb, c->tab, twp<TB>(c, 1), nt, bsc, c->mm);
+    };
+    if (nf == 2) {
+        launch(k_y_inv_grad<TB, NY, P, 2, E, 0>, grid);
+    } else if constexpr (sizeof(TB) == 8) {
+        if (os)
+            launch(k_y_inv_grad<TB, NY, P, 1, E, 1>, xgrid(nb, 9, nz));
+        else
+            launch(k_y_inv_grad<TB, NY, P, 1, E, 0>, grid);
+    } else {
+        launch(k_y_inv_grad<TB, NY, P, 1, E, 0>, grid);
+    }
     return NS3D_OK;
 }
 
