@@ -127,41 +127,47 @@ k_pack_full(PtrArr<const cplx<double>, 3> v, double* __restrict__ vec, long N) {
 }
 // ------------------------------------------------------- a9: WENO advection
 // Reference: Source/advection_WENO.cu:47-101 (weno5/weno3), :105-301 (faces), :304-360 (flux).
-// The nonlinear weights alpha_k = c_k / (eps + beta_k)^2 normalised by their
-// sum are formed over the common denominator prod_k (eps + beta_k)^2, so a
-// face costs one FP64 division instead of six; if those products leave the
-// FP64 range (smoothness indicators beyond ~1e70) the per-weight form is used.
-__device__ __forceinline__ double weno_combine3(double c0, double c1, double c2, double d0, double d1, double d2,
-                                                double q0, double q1, double q2) {
-    const double a0 = c0 * (d1 * d2), a1 = c1 * (d0 * d2), a2 = c2 * (d0 * d1);
-    const double s = a0 + a1 + a2;
-    if (s < 1.0e300 && s > 1.0e-300) return (a0 * q0 + a1 * q1 + a2 * q2) / s;
-    const double b0 = c0 / d0, b1 = c1 / d1, b2 = c2 / d2, t = b0 + b1 + b2;
-    return b0 / t * q0 + b1 / t * q1 + b2 / t * q2;
+// A face is one reconstruction, its stencil mirrored to the upwind side, from the
+// differences of the scalar along the axis: with f3 the upwind cell's value and e_1..e_4
+// the differences outwards, the candidate values are f3 + p_k / 6 and the smoothness
+// indicators 13/12 (t_k^2 + 3/13 u_k^2), t and u sums of the e's.  The nonlinear weights
+// alpha_k = c_k / (eps + beta_k)^2, here with the common factors taken out, are formed over
+// the common denominator prod_k (eps + beta_k)^2, so a face costs one FP64 division
+// instead of six; if those products leave the FP64 range (smoothness indicators beyond
+// ~1e70) the per-weight form is used.
+// Numerators and denominator of one face; FAST: the quotient over the common denominator
+// (ok: it is in range), else the per-weight form.
+template <bool FAST>
+__device__ __forceinline__ double weno_increment5(double e1, double e2, double e3, double e4, bool& ok) {
+    constexpr double eps = 1.0E-22 * 12.0 / 13.0, g = 3.0 / 13.0;
+    const double t0 = e2 - e1, t1 = e3 - e2, t2 = e4 - e3;
+    const double u0 = 3.0 * e2 - e1, u1 = e2 + e3, u2 = e4 - 3.0 * e3;
+    const double b0 = (t0 * t0 + eps) + g * u0 * u0;
+    const double b1 = (t1 * t1 + eps) + g * u1 * u1;
+    const double b2 = (t2 * t2 + eps) + g * u2 * u2;
+    const double d0 = b0 * b0, d1 = b1 * b1, d2 = b2 * b2;
+    const double p0 = 5.0 * e2 - 2.0 * e1, p1 = e2 + 2.0 * e3, p2 = 4.0 * e3 - e4;
+    if constexpr (FAST) {
+        const double a0 = d1 * d2, a1 = 6.0 * (d0 * d2), a2 = 3.0 * (d0 * d1);
+        const double s = a0 + a1 + a2;
+        ok = s < 1.0e300 && s > 1.0e-299;
+        return (a0 * p0 + a1 * p1 + a2 * p2) / (6.0 * s);
+    }
+    const double w0 = 1.0 / d0, w1 = 6.0 / d1, w2 = 3.0 / d2, t = 6.0 * (w0 + w1 + w2);
+    return w0 / t * p0 + w1 / t * p1 + w2 / t * p2;
 }
-__device__ __forceinline__ double weno5(double f1, double f2, double f3, double f4, double f5) {
-    const double eps = 1.0E-22;
-    const double q0 = 1.0 / 3.0 * f1 - 7.0 / 6.0 * f2 + 11.0 / 6.0 * f3;
-    const double q1 = -1.0 / 6.0 * f2 + 5.0 / 6.0 * f3 + 1.0 / 3.0 * f4;
-    const double q2 = 1.0 / 3.0 * f3 + 5.0 / 6.0 * f4 - 1.0 / 6.0 * f5;
-    const double t0 = f1 - 2.0 * f2 + f3, u0 = f1 - 4.0 * f2 + 3.0 * f3;
-    const double t1 = f2 - 2.0 * f3 + f4, u1 = f2 - f4;
-    const double t2 = f3 - 2.0 * f4 + f5, u2 = 3.0 * f3 - 4.0 * f4 + f5;
-    const double b0 = 13.0 / 12.0 * t0 * t0 + 0.25 * u0 * u0;
-    const double b1 = 13.0 / 12.0 * t1 * t1 + 0.25 * u1 * u1;
-    const double b2 = 13.0 / 12.0 * t2 * t2 + 0.25 * u2 * u2;
-    return weno_combine3(0.1, 0.6, 0.3, (eps + b0) * (eps + b0), (eps + b1) * (eps + b1), (eps + b2) * (eps + b2),
-                         q0, q1, q2);
-}
-__device__ __forceinline__ double weno3(double f1, double f2, double f3) {
-    const double eps = 1.0E-22;
-    const double q0 = -0.5 * f1 + 1.5 * f2, q1 = 0.5 * f2 + 0.5 * f3;
-    const double b0 = (f2 - f1) * (f2 - f1), b1 = (f3 - f2) * (f3 - f2);
-    const double d0 = (eps + b0) * (eps + b0), d1 = (eps + b1) * (eps + b1);
-    const double a0 = (1.0 / 3.0) * d1, a1 = (2.0 / 3.0) * d0, s = a0 + a1;
-    if (s < 1.0e300 && s > 1.0e-300) return (a0 * q0 + a1 * q1) / s;
-    const double c0 = (1.0 / 3.0) / d0, c1 = (2.0 / 3.0) / d1, t = c0 + c1;
-    return c0 / t * q0 + c1 / t * q1;
+template <bool FAST>
+__device__ __forceinline__ double weno_increment3(double e1, double e2, bool& ok) {
+    constexpr double eps = 1.0E-22;
+    const double b0 = e1 * e1 + eps, b1 = e2 * e2 + eps;
+    const double d0 = b0 * b0, d1 = b1 * b1;
+    if constexpr (FAST) {
+        const double a0 = d1, a1 = 2.0 * d0, s = a0 + a1;
+        ok = s < 1.0e300 && s > 1.0e-299;
+        return (a0 * e1 + a1 * e2) / (2.0 * s);
+    }
+    const double w0 = 1.0 / d0, w1 = 2.0 / d1, t = 2.0 * (w0 + w1);
+    return w0 / t * e1 + w1 / t * e2;
 }
 
 struct Grid3 {
@@ -174,106 +180,183 @@ struct Grid3 {
     }
 };
 
-// The two faces of a cell along one axis, upwinded by the face velocities
-// Um (face -1/2) and Up (face +1/2): flux_{x,y,z}_weno_{L,R}
-// (Source/advection_WENO.cu:105-301).  w[o] is the scalar at offset o along
-// the axis (|o| <= 3 for WENO5, 2 for WENO3, 1 for the first-order scheme).
-// Each face takes one reconstruction, its stencil selected by the upwind
-// side, so diverging lanes run no second branch.  q9: the z right-biased
-// reconstruction reads offset -1 where -2 belongs (Source/advection_WENO.cu:288).
-template <int SCHEME>
-__device__ __forceinline__ void weno_faces(const double* w, double Um, double Up, bool q9, double& sm, double& sp) {
-    const bool lm = Um >= 0.0, lp = Up >= 0.0;
-    if constexpr (SCHEME == 5) {
-        sm = weno5(lm ? w[-3] : w[2], lm ? w[-2] : w[1], lm ? w[-1] : w[0], lm ? w[0] : w[-1],
-                   lm ? w[1] : (q9 ? w[-1] : w[-2]));
-        sp = weno5(lp ? w[-2] : w[3], lp ? w[-1] : w[2], lp ? w[0] : w[1], lp ? w[1] : w[0],
-                   lp ? w[2] : (q9 ? w[0] : w[-1]));
-    } else if constexpr (SCHEME == 3) {
-        sm = weno3(lm ? w[-2] : w[1], lm ? w[-1] : w[0], lm ? w[0] : w[-1]);
-        sp = weno3(lp ? w[-1] : w[2], lp ? w[0] : w[1], lp ? w[1] : w[0]);
-    } else {
-        sm = lm ? w[-1] : w[0];
-        sp = lp ? w[0] : w[1];
-    }
-}
-
 __device__ __forceinline__ int wrap_add(int i, int o, int n) {
     const int v = i + o;
     return v < 0 ? v + n : (v >= n ? v - n : v);
 }
 
-// (u.grad) x at (j,k,l) with upwind WENO faces chosen by the sign of the
-// face-averaged velocity: flux_device + advection (Source/advection_WENO.cu:304-392).
-template <int SCHEME, typename TU>
-__device__ __forceinline__ double weno_point(const TU* __restrict__ ux, const TU* __restrict__ uy,
-                                             const TU* __restrict__ uz, const double* __restrict__ x, const Grid3& G,
-                                             long id, int j, int k, int l, double rdx, double rdy, double rdz, int zfix) {
-    constexpr int R = SCHEME == 5 ? 3 : (SCHEME == 3 ? 2 : 1);
-    const long sx = (long)G.Ny * G.Nz, sy = G.Nz;
-    const long bx = id - (long)j * sx, by = id - (long)k * sy, bz = id - l;   // id with j, k or l removed
-    long ox[2 * R + 1], oy[2 * R + 1], oz[2 * R + 1];
-#pragma unroll
-    for (int o = -R; o <= R; o++) {
-        ox[o + R] = bx + wrap_add(j, o, G.Nx) * sx;
-        oy[o + R] = by + (long)wrap_add(k, o, G.Ny) * sy;
-        oz[o + R] = bz + wrap_add(l, o, G.Nz);
+// The face between two cells along one axis, upwinded by the face velocity U:
+// flux_{x,y,z}_weno_{L,R} (Source/advection_WENO.cu:105-301).  w[o], o = 1-R..R, is the
+// scalar around the lower cell (R = 3 for WENO5, 2 for WENO3, 1 for the first-order
+// scheme).  The upper cell's lower face is this same expression, so a face is evaluated
+// once.  q9: the z right-biased reconstruction reads offset -1 where -2 belongs
+// (Source/advection_WENO.cu:288), i.e. its last difference is zero.
+template <int SCHEME, bool FAST>
+__device__ __forceinline__ double weno_face(const double* w, double U, bool q9, bool& ok) {
+    const bool lo = U >= 0.0;
+    const double f = lo ? w[0] : w[1];
+    if constexpr (SCHEME == 5) {
+        const double m1 = w[0] - w[-1], p1 = w[2] - w[1];
+        const double r = weno_increment5<FAST>(lo ? w[-1] - w[-2] : w[3] - w[2], lo ? m1 : p1, w[1] - w[0],
+                                               lo ? p1 : (q9 ? 0.0 : m1), ok);
+        return lo ? f + r : f - r;
+    } else if constexpr (SCHEME == 3) {
+        const double r = weno_increment3<FAST>(lo ? w[0] - w[-1] : w[2] - w[1], w[1] - w[0], ok);
+        return lo ? f + r : f - r;
     }
-    const double uc = (double)ux[id], vc = (double)uy[id], wc = (double)uz[id];
-    const double Uw = 0.5 * ((double)ux[ox[R - 1]] + uc), Ue = 0.5 * (uc + (double)ux[ox[R + 1]]);
-    const double Un = 0.5 * ((double)uy[oy[R - 1]] + vc), Us = 0.5 * (vc + (double)uy[oy[R + 1]]);
-    const double Ur = 0.5 * ((double)uz[oz[R - 1]] + wc), Uf = 0.5 * (wc + (double)uz[oz[R + 1]]);
-    double wx[2 * R + 1], wy[2 * R + 1], wz[2 * R + 1];
-    const double xc = x[id];
+    ok = true;
+    return f;
+}
+// N faces, face n of window w + n * stride: the quotients of all of them are independent
+// chains, with one branch behind them for those out of range.
+template <int SCHEME, int N>
+__device__ __forceinline__ void weno_faces(const double* w, int stride, const double* U, bool q9, double* f) {
+    bool ok[N], all = true;
 #pragma unroll
-    for (int o = 0; o <= 2 * R; o++) {
-        wx[o] = o == R ? xc : x[ox[o]];
-        wy[o] = o == R ? xc : x[oy[o]];
-        wz[o] = o == R ? xc : x[oz[o]];
+    for (int n = 0; n < N; n++) {
+        f[n] = weno_face<SCHEME, true>(w + n * stride, U[n], q9, ok[n]);
+        all = all && ok[n];
     }
-    double sw, se, sn, ss, sr, sf;
-    weno_faces<SCHEME>(wx + R, Uw, Ue, false, sw, se);
-    weno_faces<SCHEME>(wy + R, Un, Us, false, sn, ss);
-    weno_faces<SCHEME>(wz + R, Ur, Uf, !zfix, sr, sf);
-    return uc * (se - sw) * rdx + vc * (ss - sn) * rdy + wc * (sf - sr) * rdz;
+    if (SCHEME && !all) {
+#pragma unroll
+        for (int n = 0; n < N; n++) {
+            bool o;
+            if (!ok[n]) f[n] = weno_face<SCHEME, false>(w + n * stride, U[n], q9, o);
+        }
+    }
 }
 
-// Point index of this thread: blocks are remapped so that each XCD (block b
-// runs on XCD b mod 8) sweeps one contiguous run of x-planes, keeping the
-// +-3-plane stencil reuse inside one L2.  The grid is a multiple of 8 blocks.
-__device__ __forceinline__ long weno_index() { return (long)xcd_tile() * blockDim.x + threadIdx.x; }
+// (u.grad) x with upwind WENO faces chosen by the sign of the face-averaged velocity:
+// flux_device + advection (Source/advection_WENO.cu:304-392); out(id, x, adv) per cell.
+// VALU bound in WENO5, so each face is evaluated once: a block covers whole z rows and
+// marches over `march` x planes; the x face of the step before stays in registers with the
+// x window, a thread's YC cells share their y faces, and the z face goes to the upper
+// neighbour through LDS (the row is in the block, so no face is left over), as does the
+// next plane's row, which is in the x window already.  Six faces a cell, each thread one
+// point: WENO5 at 256^3 426 us, 128^3 52.6; this form 225 and 33.5 (y faces evaluated per
+// thread, rows read from memory: 246 and 37); first order 235 and 168 us at 256^3.
+constexpr int WENO_THREADS = 512;   // a block: whole rows, at most one of the longest
+template <int SCHEME, int YC, typename TU, class OUT>
+__device__ __forceinline__ void weno_march(const TU* __restrict__ ux, const TU* __restrict__ uy,
+                                           const TU* __restrict__ uz, const double* __restrict__ x, const Grid3& G,
+                                           int march, double rdx, double rdy, double rdz, bool q9, OUT&& out) {
+    constexpr int R = SCHEME == 5 ? 3 : (SCHEME == 3 ? 2 : 1);
+    constexpr int W = 2 * R;
+    __shared__ double zf[2][YC][WENO_THREADS];
+    __shared__ double zx[2][YC][WENO_THREADS];
+    const int rows = blockDim.x / G.Nz, nyb = (G.Ny + rows * YC - 1) / (rows * YC);
+    const int tile = xcd_tile();
+    const int jb = tile / nyb, j0 = jb * march;
+    if (j0 >= G.Nx) return;
+    const int j1 = min(j0 + march, G.Nx);
+    const int t = threadIdx.x, r = t / G.Nz, l = t - r * G.Nz;
+    const int k0 = ((tile - jb * nyb) * rows + r) * YC;
+    const bool row = r < rows && k0 < G.Ny;
+    const int below = l == 0 ? t + G.Nz - 1 : t - 1;
+    const long sx = (long)G.Ny * G.Nz;
+    // in-plane offsets: the y rows k0-R .. k0+YC-1+R and the z window
+    int oy[YC + W], oz[W];
+#pragma unroll
+    for (int o = 0; o < YC + W; o++) oy[o] = row ? wrap_add(k0, o - R, G.Ny) * G.Nz : 0;
+#pragma unroll
+    for (int o = 0; o < W; o++) oz[o] = row ? wrap_add(l, o + 1 - R, G.Nz) : 0;
+    const int lc = row ? l : 0;
+    auto plane = [&](int j) __attribute__((always_inline)) { return x + (long)wrap_add(j, 0, G.Nx) * sx; };
+    double wx[YC][W], fx[YC], uc[YC];
+#pragma unroll
+    for (int c = 0; c < YC; c++) {
+        const int oc = oy[c + R] + lc;
+#pragma unroll
+        for (int o = 0; o < W; o++) wx[c][o] = plane(j0 - R + o)[oc];
+        const double ub = (double)ux[(long)wrap_add(j0, -1, G.Nx) * sx + oc];
+        uc[c] = (double)ux[(long)j0 * sx + oc];
+        const double Ux = 0.5 * (ub + uc[c]);
+        weno_faces<SCHEME, 1>(wx[c] + R - 1, 0, &Ux, false, fx + c);
+        zx[j0 & 1][c][t] = wx[c][R];
+    }
+    __syncthreads();
+    for (int j = j0; j < j1; j++) {
+        const long base = (long)j * sx;
+        const double* xj = x + base;
+        const double* xr = plane(j + R);
+        const TU* un = ux + (long)wrap_add(j, 1, G.Nx) * sx;
+        double fe[YC], ue[YC], wc[YC], xc[YC], adv[YC], wy[YC + W], vy[YC + 2];
+        // every load of the step first
+#pragma unroll
+        for (int c = 0; c < YC; c++) {
+            const int oc = oy[c + R] + lc;
+#pragma unroll
+            for (int o = 0; o < W - 1; o++) wx[c][o] = wx[c][o + 1];
+            wx[c][W - 1] = xr[oc];
+            ue[c] = (double)un[oc];
+            xc[c] = wx[c][R - 1];
+        }
+#pragma unroll
+        for (int o = 0; o < YC + W; o++) wy[o] = o >= R && o < R + YC ? xc[o - R] : xj[oy[o] + lc];
+#pragma unroll
+        for (int o = 0; o < YC + 2; o++) vy[o] = (double)uy[base + oy[o + R - 1] + lc];
+        double wz[YC][W], wn[YC];
+#pragma unroll
+        for (int c = 0; c < YC; c++) {
+#pragma unroll
+            for (int o = 0; o < W; o++) wz[c][o] = o == R - 1 ? xc[c] : zx[j & 1][c][t - lc + oz[o]];
+            wc[c] = (double)uz[base + oy[c + R] + lc];
+            wn[c] = (double)uz[base + oy[c + R] + oz[R]];
+        }
+        double fz[YC], fy[YC + 1], Ux[YC], Uy[YC + 1], Uz[YC];
+#pragma unroll
+        for (int c = 0; c < YC; c++) {
+            Uz[c] = 0.5 * (wc[c] + wn[c]);
+            Ux[c] = 0.5 * (uc[c] + ue[c]);
+        }
+#pragma unroll
+        for (int c = 0; c <= YC; c++) Uy[c] = 0.5 * (vy[c] + vy[c + 1]);
+        weno_faces<SCHEME, YC>(wz[0] + R - 1, W, Uz, q9, fz);
+#pragma unroll
+        for (int c = 0; c < YC; c++) {
+            zf[j & 1][c][t] = fz[c];
+            zx[(j + 1) & 1][c][t] = wx[c][R];
+        }
+        weno_faces<SCHEME, YC + 1>(wy + R - 1, 1, Uy, false, fy);
+        weno_faces<SCHEME, YC>(wx[0] + R - 1, W, Ux, false, fe);
+#pragma unroll
+        for (int c = 0; c < YC; c++) {
+            adv[c] = uc[c] * (fe[c] - fx[c]) * rdx + vy[c + 1] * (fy[c + 1] - fy[c]) * rdy;
+            fx[c] = fe[c];
+            uc[c] = ue[c];
+        }
+        __syncthreads();   // two buffers: the next step's writes need no second barrier
+#pragma unroll
+        for (int c = 0; c < YC; c++) {
+            if (row && k0 + c < G.Ny)
+                out(base + oy[c + R] + lc, xc[c], adv[c] + wc[c] * (fz[c] - zf[j & 1][c][below]) * rdz);
+        }
+    }
+}
 
 // advection kernel + flux_device (Source/advection_WENO.cu:304-392), generalised to any advected scalar x.
-template <int SCHEME>
-__global__ void __launch_bounds__(256)
+template <int SCHEME, int YC>
+__global__ void __attribute__((amdgpu_waves_per_eu(YC == 1 ? 4 : 3, 8))) __launch_bounds__(WENO_THREADS)
 k_weno(const double* __restrict__ ux, const double* __restrict__ uy, const double* __restrict__ uz,
-       const double* __restrict__ x, double* __restrict__ out, Grid3 G, double rdx, double rdy, double rdz, int zfix) {
-    const long id = weno_index();
-    const long n = (long)G.Nx * G.Ny * G.Nz;
-    if (id >= n) return;
-    const int l = (int)(id % G.Nz);
-    const long t1 = id / G.Nz;
-    const int k = (int)(t1 % G.Ny), j = (int)(t1 / G.Ny);
-    out[id] = weno_point<SCHEME>(ux, uy, uz, x, G, id, j, k, l, rdx, rdy, rdz, zfix);
+       const double* __restrict__ x, double* __restrict__ out, Grid3 G, int march, double rdx, double rdy, double rdz,
+       int zfix) {
+    weno_march<SCHEME, YC>(ux, uy, uz, x, G, march, rdx, rdy, rdz, !zfix,
+                       [&](long id, double, double adv) __attribute__((always_inline)) { out[id] = adv; });
 }
 
 // SSP stage of a passive scalar: out = a0*th_n + a1*(th_s - dt * (u.grad)_WENO th_s),
 // u being the masked physical velocity of the same stage (TU = bulk precision).
-template <int SCHEME, typename TU>
-__global__ void __launch_bounds__(256)
-k_weno_stage(const TU* __restrict__ u, long nr, const double* __restrict__ x, const double* __restrict__ xn,
-             double* __restrict__ out, Grid3 G, double rdx, double rdy, double rdz, int zfix, double dt,
-             double a0, double a1, int* nf) {
-    const long id = weno_index();
-    if (id >= nr) return;
-    const int l = (int)(id % G.Nz);
-    const long t1 = id / G.Nz;
-    const int k = (int)(t1 % G.Ny), j = (int)(t1 / G.Ny);
-    const double adv = weno_point<SCHEME>(u, u + nr, u + 2 * nr, x, G, id, j, k, l, rdx, rdy, rdz, zfix);
-    const double e = x[id] - dt * adv;
-    const double o = xn ? a0 * xn[id] + a1 * e : a1 * e;
-    out[id] = o;
-    flag_nonfinite(nf, !isfinite(o));
+template <int SCHEME, int YC, typename TU>
+__global__ void __attribute__((amdgpu_waves_per_eu(YC == 1 ? 4 : 3, 8))) __launch_bounds__(WENO_THREADS)
+k_weno_stage(const TU* __restrict__ u, long nr, const double* __restrict__ x, const double* xn, double* out, Grid3 G,
+             int march, double rdx, double rdy, double rdz, int zfix, double dt, double a0, double a1, int* nf) {
+    weno_march<SCHEME, YC>(u, u + nr, u + 2 * nr, x, G, march, rdx, rdy, rdz, !zfix,
+                       [&](long id, double xc, double adv) __attribute__((always_inline)) {
+                           const double e = xc - dt * adv;
+                           const double o = xn ? a0 * xn[id] + a1 * e : a1 * e;
+                           out[id] = o;
+                           flag_nonfinite(nf, !isfinite(o));
+                       });
 }
 
 __global__ void k_set_int(int* __restrict__ p, int v) {
