@@ -288,6 +288,40 @@ template <bool WAVE> __device__ __forceinline__ void exch_sync() {
     }
 }
 
+// a of the lanes with bit B set and b of those without, B below, change places
+// (one instruction swaps a register pair between the halves of each row pair or wave).
+template <int B> __device__ __forceinline__ void swap_lanes(unsigned& a, unsigned& b) {
+    const auto r = B == 32 ? __builtin_amdgcn_permlane32_swap(a, b, false, false) : __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+template <int B, typename T> __device__ __forceinline__ void swap_lanes(cplx<T>& a, cplx<T>& b) {
+    constexpr int W = sizeof(cplx<T>) / 4;
+    unsigned x[W], y[W];
+    __builtin_memcpy(x, &a, sizeof(a));
+    __builtin_memcpy(y, &b, sizeof(b));
+#pragma unroll
+    for (int i = 0; i < W; i++) swap_lanes<B>(x[i], y[i]);
+    __builtin_memcpy(&a, x, sizeof(a));
+    __builtin_memcpy(&b, y, sizeof(b));
+}
+// Thread of a pencil (t) and pencil of the block (p) such that the top two bits of t are
+// lane bits 5 and 4; contiguous quarter rows (at least 64 B in FP64) stay with adjacent lanes.
+template <int TPP> struct SwapLanes {
+    __device__ __forceinline__ static void map(int tid, int& t, int& p) {
+        const int lane = tid & 63, wave = tid >> 6;
+        if constexpr (TPP <= 64) {
+            constexpr int L = TPP / 4;   // lanes of a quarter row
+            t = (lane >> 4) * L + (lane & (L - 1));
+            p = wave * (64 / TPP) + (lane & 15) / L;
+        } else {
+            constexpr int WP = TPP / 64;
+            t = (lane >> 4) * (TPP / 4) + (wave % WP) * 16 + (lane & 15);
+            p = wave / WP;
+        }
+    }
+};
+
 // Per-thread register twiddles of a plan (PencilFFT::load_tw); plans with the
 // same radix sequence share the slot layout, and then one set serves both
 // transform directions.
@@ -296,13 +330,21 @@ template <typename T, int K> struct TwRegs {
 };
 
 // PIN: every product's contraction spelled out (cmul_pinned).
-template <typename T, int N, int TPP, int DIR, typename S, typename Addr, bool WAVE = false, bool PIN = false>
+template <typename T, int N, int TPP, int DIR, typename S, typename Addr, bool WAVE = false, bool PIN = false, bool SWAP = false>
 struct PencilFFT {
     using Info = SeqInfo<S>;
     static constexpr int NP = Info::n;
     static constexpr int E = PlanRegs<N, TPP, S>::value();
     static constexpr int R0 = Info::rad[0];
     static constexpr int RL = Info::rad[NP - 1];
+    // SWAP: the exchange after the first pass by lane swaps (lane_swap): a thread's logical index in
+    // the second pass is then swapped(t).
+    static constexpr int SB = R0 == 4 ? 2 : 1;   // index bits that change places
+    __device__ __forceinline__ static int swapped(int t) {
+        if constexpr (!SWAP) return t;
+        constexpr int b = __builtin_ctz(TPP);
+        return ((t << SB) & (TPP - 1)) | (t >> (b - SB));
+    }
     // first-pass input pattern: v[q*R0 + r] <-> x[t + q*TPP + r*N/R0]
     static constexpr int B0 = (N / R0 + TPP - 1) / TPP;
     // last-pass output pattern: v[q*RL + r] <-> y[t + q*TPP + r*N/RL]
@@ -335,7 +377,7 @@ struct PencilFFT {
         if constexpr (Ns > 1) {
 #pragma unroll
             for (int q = 0; q < B; q++) {
-                const int jj = t + q * TPP;
+                const int jj = (I == 1 ? swapped(t) : t) + q * TPP;
                 const int jm = (NB % TPP == 0 || jj < NB) ? jj % Ns : 0;
 #pragma unroll
                 for (int r = 1; r < R; r++) tr.w[tw_off(I) + q * (R - 1) + r - 1] = tw[r * jm * (N / (Ns * R))];
@@ -377,6 +419,13 @@ struct PencilFFT {
             }
         }
     }
+    // LDS address of element idx in the exchange after pass I.  After lane_swap the second
+    // pass writes with neighbouring lanes Ns*R elements apart: the low bits are XOR-ed with
+    // those bits of the index (reads stay contiguous within aligned groups).
+    template <int I> __device__ __forceinline__ static int addr(int p, int idx) {
+        if constexpr (SWAP && I == 1) idx ^= (idx / (Info::prod_before(1) * Info::rad[1])) & 15;
+        return Addr::template at<(SWAP && I == 1) ? 0 : Info::prod_before(I)>(p, idx);
+    }
     // Stockham exchange after pass I: store in the order pass I+1 reads.
     template <int I>
     __device__ __forceinline__ static void exch_write(const cplx<T>* v, cplx<T>* lds, int t, int p) {
@@ -390,7 +439,7 @@ struct PencilFFT {
             if (NB % TPP == 0 || jj < NB) {
                 const int base = (jj / Ns) * Ns * R + (jj % Ns);
 #pragma unroll
-                for (int r = 0; r < R; r++) lds[Addr::template at<Ns>(p, base + r * Ns)] = v[q * R + r];
+                for (int r = 0; r < R; r++) lds[addr<I>(p, base + r * Ns)] = v[q * R + r];
             }
         }
     }
@@ -405,7 +454,7 @@ struct PencilFFT {
             const int jj = t + q * TPP;
             if (NB2 % TPP == 0 || jj < NB2) {
 #pragma unroll
-                for (int r = 0; r < R2; r++) v[q * R2 + r] = lds[Addr::template at<Ns>(p, jj + r * NB2)];
+                for (int r = 0; r < R2; r++) v[q * R2 + r] = lds[addr<I>(p, jj + r * NB2)];
             }
         }
     }
@@ -413,9 +462,13 @@ struct PencilFFT {
     template <int I>
     __device__ __forceinline__ static void pass(cplx<T>* v, cplx<T>* lds, const cplx<T>* __restrict__ tw, int t, int p,
                                                 const TwReg* tr) {
-        butterflies<I>(v, tw, t, tr);
-        if constexpr (I + 1 < NP) {
-            exch_write<I>(v, lds, t, p);
+        const int tl = I == 1 ? swapped(t) : t;
+        butterflies<I>(v, tw, tl, tr);
+        if constexpr (SWAP && I == 0) {
+            lane_swap(v);
+            pass<1>(v, lds, tw, t, p, tr);
+        } else if constexpr (I + 1 < NP) {
+            exch_write<I>(v, lds, tl, p);
             exch_sync<WAVE>();
             exch_read<I>(v, lds, t, p);
             exch_sync<WAVE>();
@@ -427,16 +480,37 @@ struct PencilFFT {
     template <int I>
     __device__ __forceinline__ static void pass2(cplx<T>* va, cplx<T>* vb, cplx<T>* la, cplx<T>* lb,
                                                  const cplx<T>* __restrict__ tw, int t, int p, const TwReg* tr) {
-        butterflies<I>(va, tw, t, tr);
-        butterflies<I>(vb, tw, t, tr);
-        if constexpr (I + 1 < NP) {
-            exch_write<I>(va, la, t, p);
-            exch_write<I>(vb, lb, t, p);
+        const int tl = I == 1 ? swapped(t) : t;
+        butterflies<I>(va, tw, tl, tr);
+        butterflies<I>(vb, tw, tl, tr);
+        if constexpr (SWAP && I == 0) {
+            lane_swap(va);
+            lane_swap(vb);
+            pass2<1>(va, vb, la, lb, tw, t, p, tr);
+        } else if constexpr (I + 1 < NP) {
+            exch_write<I>(va, la, tl, p);
+            exch_write<I>(vb, lb, tl, p);
             exch_sync<WAVE>();
             exch_read<I>(va, la, t, p);
             exch_read<I>(vb, lb, t, p);
             exch_sync<WAVE>();
             pass2<I + 1>(va, vb, la, lb, tw, t, p, tr);
+        }
+    }
+    // The first exchange without LDS: an LDS store of 16 B a lane takes the CU 13.7 cycles (a
+    // load 5.0), 75 a radix-4 exchange; the swaps are 16 VALU instructions.  After a radix-4 first pass the register index (2 bits)
+    // changes places with the top two bits of t, which SwapLanes puts at lane bits 5 and 4;
+    // after a radix-2 one (two butterflies a thread, v[2q + r]) r with lane bit 5.
+    __device__ __forceinline__ static void lane_swap(cplx<T>* v) {
+        static_assert(!SWAP || (E == 4 && (R0 == 4 || R0 == 2) && (TPP & (TPP - 1)) == 0 && TPP >= 16), "plan of lane_swap");
+        if constexpr (R0 == 4) {
+            swap_lanes<32>(v[0], v[2]);
+            swap_lanes<32>(v[1], v[3]);
+            swap_lanes<16>(v[0], v[1]);
+            swap_lanes<16>(v[2], v[3]);
+        } else {
+            swap_lanes<32>(v[0], v[1]);
+            swap_lanes<32>(v[2], v[3]);
         }
     }
 

@@ -368,7 +368,7 @@ k_y_inv_grad(const cplx<TB>* __restrict__ A, cplx<TB>* __restrict__ B, long nc, 
 // z pass on one (x,y) pencil: paired C2R transforms (two real fields per
 // complex FFT), the advective product, and paired R2C transforms.
 // C2R convention: x,y passes already done; only Re of l=0 and l=Nz/2 is used.
-template <typename TB, int NZ, int P, bool TRUNC = false>
+template <typename TB, int NZ, int P, bool TRUNC = false, int NF = 1>
 struct ZPencil {
     static constexpr int TPP = ZTPP<TB, NZ>;
     static constexpr int PAD = (sizeof(TB) == 8) ? 1 : 2;
@@ -392,8 +392,21 @@ struct ZPencil {
 #define NS3D_ZWAVE 1
 #endif
     static constexpr bool WAVE = NS3D_ZWAVE != 0 && TPP <= 64 && 64 % TPP == 0;
-    using FI = PencilFFT<TB, NZ, TPP, +1, typename ZPlanT<TB, NZ>::R, LA, WAVE>;
-    using FF = PencilFFT<TB, NZ, TPP, -1, typename SeqRev<typename ZPlanT<TB, NZ>::R>::type, LA, WAVE>;
+    // The first exchange by lane swaps, FP64 at power-of-two lengths: z pass at 512^3 3.40 ->
+    // 3.10 ms, 256^3 0.324 -> 0.309, 128^3 49.3 -> 47.6 us, bilinear 86.6 -> 80.4; at 64 the
+    // bilinear step gains (J.v 48.0 -> 47.3 us), the other does not (65 fields 280 -> 282 us).
+    static constexpr bool SWAP = sizeof(TB) == 8 && (NZ & (NZ - 1)) == 0 && NZ >= (NF == 2 ? 64 : 128);
+    static_assert(!SWAP || P * TPP % 64 == 0, "whole waves");
+    using FI = PencilFFT<TB, NZ, TPP, +1, typename ZPlanT<TB, NZ>::R, LA, WAVE, false, SWAP>;
+    using FF = PencilFFT<TB, NZ, TPP, -1, typename SeqRev<typename ZPlanT<TB, NZ>::R>::type, LA, WAVE, false, SWAP>;
+    __device__ __forceinline__ static void lanes(int tid, int& t, int& p) {
+        if constexpr (SWAP) {
+            SwapLanes<TPP>::map(tid, t, p);
+        } else {
+            t = tid % TPP;
+            p = tid / TPP;
+        }
+    }
     static_assert(FI::RL == FF::R0 && FI::BL == FF::B0, "mirror plans must share the product layout");
     static constexpr int E = FI::E > FF::E ? FI::E : FF::E;
     static constexpr int NPT = FI::BL * FI::RL;  // physical points per thread
@@ -662,7 +675,7 @@ k_z_product(const cplx<TB>* __restrict__ Bf, cplx<TB>* __restrict__ C, long nc, 
             SpecTables tab, const cplx<TB>* __restrict__ twg, TB scale, TB* __restrict__ uphys, long nr, int nt, long bsc,
             MemberMask mm) {
     // B is zero on z-planes l > lmax (never written by the y pass): TRUNC skips them
-    using Z = ZPencil<TB, NZ, P, true>;
+    using Z = ZPencil<TB, NZ, P, true, NF>;
     constexpr int TPP = Z::TPP, NPT = Z::NPT;
 #ifndef NS3D_ZILP
 #define NS3D_ZILP 1
@@ -698,7 +711,9 @@ k_z_product(const cplx<TB>* __restrict__ Bf, cplx<TB>* __restrict__ C, long nc, 
     if (bid0 >= nb || member_idle(mm)) return;
     const int bid = tile_order<NS3D_REV_Z>(bid0, nb);
     stage_twiddles<TB, NZ>(tw, twg);
-    const int tid = threadIdx.x, t = tid % TPP, p = tid / TPP;
+    const int tid = threadIdx.x;
+    int t, p;
+    Z::lanes(tid, t, p);
     const long pen = (long)bid * P + p;
     const bool valid = pen < npen;
     const long off = valid ? pen * Mz : 0;
@@ -1567,7 +1582,9 @@ k_z_c2r(const cplx<TB>* __restrict__ in, TB* __restrict__ out, long npairs, int 
     const int bid = xcd_tile();
     if (bid >= nb) return;
     stage_twiddles<TB, NZ>(tw, twg);
-    const int tid = threadIdx.x, t = tid % TPP, p = tid / TPP;
+    const int tid = threadIdx.x;
+    int t, p;
+    Z::lanes(tid, t, p);
     const long pair = (long)bid * P + p;
     const bool valid = pair < npairs;
     const long p0 = valid ? 2 * pair : 0, p1 = p0 + 1;
@@ -1597,7 +1614,9 @@ k_z_r2c(const TB* __restrict__ in, cplx<TB>* __restrict__ out, long npairs, int 
     const int bid = xcd_tile();
     if (bid >= nb) return;
     stage_twiddles<TB, NZ>(tw, twg);
-    const int tid = threadIdx.x, t = tid % TPP, p = tid / TPP;
+    const int tid = threadIdx.x;
+    int t, p;
+    Z::lanes(tid, t, p);
     const long pair = (long)bid * P + p;
     const bool valid = pair < npairs;
     const long p0 = valid ? 2 * pair : 0, p1 = p0 + 1;
