@@ -63,18 +63,21 @@ def pass_bytes_incr(nc):
 
 def profiled_traffic(precision, kernel_prefix):
     """HBM bytes per dispatch (rocprofv3 FETCH_SIZE + WRITE_SIZE, copy-calibrated)
-    of a kernel at 256^3, from the committed profile summary; None if absent."""
+    of a kernel at 256^3, from the committed profile summary, averaged over the
+    launches of its instances; None if absent."""
     path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", "rk3_256_passes_traffic.md")
     if not os.path.exists(path):
         return None
+    total = n = 0
     for line in open(path):
         line = line.strip()
         if not line.startswith("{"):
             continue
         d = json.loads(line)
         if d["precision"] == precision and d["kernel"].startswith(kernel_prefix + "<"):
-            return d["fetch_bytes"] + d["write_bytes"]
-    return None
+            total += d.get("calls", 1) * (d["fetch_bytes"] + d["write_bytes"])
+            n += d.get("calls", 1)
+    return total / n if n else None
 
 
 def run_gpu(N, precision, steps, warmup, u0, Re, dt):
@@ -112,6 +115,10 @@ def run_gpu(N, precision, steps, warmup, u0, Re, dt):
     state = 8 if precision == "fp32s" else 16
     nc = N * N * (N // 2 + 1)
     pb = pass_bytes_incr(nc) if precision == "fp32i" else pass_bytes(nc, bulk, state)
+    sb = 3 * sum(pb) if precision == "fp32i" else step_bytes(nc, bulk, state)
+    # an x-forward launch that no P1 launch follows writes the next stage's P1 output (6 bulk fields) itself
+    if calls[4]:
+        pb[4] += 6 * bulk * nc * max(0, calls[4] - calls[0]) / calls[4]
     passes = []
     for i in range(5):
         avg = ms[i] / calls[i] if calls[i] else float("nan")
@@ -119,7 +126,6 @@ def run_gpu(N, precision, steps, warmup, u0, Re, dt):
         passes.append({"pass": PASS_NAMES[i], "kernel": PASS_KERNELS[i], "calls": calls[i], "avg_ms": avg,
                        "total_ms": ms[i], "alg_bytes": pb[i], "GBps": gbs})
     ms_step = total_ms / steps
-    sb = 3 * sum(pb) if precision == "fp32i" else step_bytes(nc, bulk, state)
     return {
         "precision": precision,
         "steps_per_s": steps / (total_ms * 1e-3),
