@@ -241,7 +241,9 @@ template <typename TB, int NX> constexpr bool CHAINS = sizeof(TB) == 8 ? MIRROR_
 // them next is 4-9% faster (step 4.10 -> 3.87 ms); smaller outputs are read back from the
 // cache and lose by it (192^3 y-inverse 0.175 -> 0.195 ms, 128^3 pencil copies 0.022 -> 0.029),
 // and so do partial lines (512^3 y-inverse, 64-B segments, 2.56 -> 2.91 ms; 320^3 FP32
-// y-forward, 96-B segments, 0.155 -> 0.276 ms).
+// y-forward, 96-B segments, 0.155 -> 0.276 ms); 128-B segments that start in the
+// middle of a line, as FP32 rows of 136 modes have every other time, still gain: 256^3 FP32
+// step 2.71 -> 2.66 ms.
 template <typename TB> int nt_for(const ns3d_ctx* c, int P, double fields) {
     return P * sizeof(cplx<TB>) >= 128 &&
            fields * (double)c->nci * c->batch * sizeof(cplx<TB>) > (sizeof(TB) == 8 ? 256.0 : 128.0) * (1 << 20);
