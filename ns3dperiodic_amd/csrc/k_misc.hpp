@@ -133,10 +133,14 @@ k_pack_full(PtrArr<const cplx<double>, 3> v, double* __restrict__ vec, long N) {
 // indicators 13/12 (t_k^2 + 3/13 u_k^2), t and u sums of the e's.  The nonlinear weights
 // alpha_k = c_k / (eps + beta_k)^2, here with the common factors taken out, are formed over
 // the common denominator prod_k (eps + beta_k)^2, so a face costs one FP64 division
-// instead of six; if those products leave the FP64 range (smoothness indicators beyond
-// ~1e70) the per-weight form is used.
+// instead of six; where those products could leave the FP64 range (differences of the
+// scalar beyond ~1e33, WENO3 ~1e60) the per-weight form is used.
 // Numerators and denominator of one face; FAST: the quotient over the common denominator
-// (ok: it is in range), else the per-weight form.
+// (ok: it and every product of the numerator are in range), else the per-weight form.
+// The test of the denominator s covers the numerator: p_k = t_k / 2 +- 3 u_k / 2, so
+// |p_k| <= 3.2 sqrt(b_k), and d1 d2 <= s, d0 d2 <= s / 6, d0 d1 <= s / 3 give
+// |a_k p_k| <= 4 s^(9/8): under 1e299 for s < 1e265.  WENO3: |a_k e_k| <= s^(5/4), under
+// 1e300 for s < 1e240.
 template <bool FAST>
 __device__ __forceinline__ double weno_increment5(double e1, double e2, double e3, double e4, bool& ok) {
     constexpr double eps = 1.0E-22 * 12.0 / 13.0, g = 3.0 / 13.0;
@@ -150,7 +154,7 @@ __device__ __forceinline__ double weno_increment5(double e1, double e2, double e
     if constexpr (FAST) {
         const double a0 = d1 * d2, a1 = 6.0 * (d0 * d2), a2 = 3.0 * (d0 * d1);
         const double s = a0 + a1 + a2;
-        ok = s < 1.0e300 && s > 1.0e-299;
+        ok = s < 1.0e265 && s > 1.0e-299;
         return (a0 * p0 + a1 * p1 + a2 * p2) / (6.0 * s);
     }
     const double w0 = 1.0 / d0, w1 = 6.0 / d1, w2 = 3.0 / d2, t = 6.0 * (w0 + w1 + w2);
@@ -163,7 +167,7 @@ __device__ __forceinline__ double weno_increment3(double e1, double e2, bool& ok
     const double d0 = b0 * b0, d1 = b1 * b1;
     if constexpr (FAST) {
         const double a0 = d1, a1 = 2.0 * d0, s = a0 + a1;
-        ok = s < 1.0e300 && s > 1.0e-299;
+        ok = s < 1.0e240 && s > 1.0e-299;
         return (a0 * e1 + a1 * e2) / (2.0 * s);
     }
     const double w0 = 1.0 / d0, w1 = 2.0 / d1, t = 2.0 * (w0 + w1);
