@@ -1439,6 +1439,13 @@ int jv_reduced_impl(ns3d_ctx* c, const double* in, double* out, bool newton) {
     // NSCallMatrixVector_reduced (Source/NS3D_periodic.cu:340-361) and
     // ..._Newton_Globalization (:364-389: out = pack(J v) - v/tau); the passes at both
     // ends read and write the vectors themselves
+    // (one vector may be both: each element is read and written by one thread; vectors that
+    // overlap otherwise are read from a copy, as blocks write while others still read)
+    const size_t len = 3 * (size_t)(c->nc - 1);
+    if (in != out && in < out + len && out < in + len) {
+        HIPCHK(hipMemcpyAsync(c->kry, in, len * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+        in = (const double*)c->kry;
+    }
     const zd* in6[6] = {c->base[0], c->base[1], c->base[2], nullptr, nullptr, nullptr};
     EpiArgs ea = make_epi(c);
     ea.vin = in;
