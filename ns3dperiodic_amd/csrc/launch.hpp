@@ -236,6 +236,15 @@ inline dim3 xgrid(long nb, int nfy = 1, int nz = 1) {
 // two kernels and the chained results are not bitwise those of the standalone P1.
 template <typename TB, int NX> constexpr bool CHAINS = sizeof(TB) == 8 ? MIRROR_P1<TB, NX> : NX % 5 != 0;
 
+// D of nf fields.  Where the x-forward pass writes the next stage's P1 output over A
+// (chain), D is at the head of region B; else behind C in A, on memory the z pass has not
+// just read.  One stage or right-hand side in FP32, D in B against D in A: 96x192x48 80.1
+// and 77.8 us, 64x512x64 145.6 and 141.0, 512x64x64 159.1 and 153.0, 128^3 125.1 and 120.6;
+// in FP64 and at 192^3 and above within 1%.
+template <typename TB> cplx<TB>* d_at(const ns3d_ctx* c, int nf, bool chain) {
+    return (cplx<TB>*)c->scratch + (chain ? 6 * nf : 3) * c->nci;
+}
+
 // Nontemporal stores of a pass's output: for outputs beyond the 256 MiB Infinity Cache,
 // written in full 128-B lines (P modes to a row segment).  At 256^3 FP64 the pass that reads
 // them next is 4-9% faster (step 4.10 -> 3.87 ms); smaller outputs are read back from the
@@ -259,7 +268,8 @@ int launch_x_inv(ns3d_ctx* c, const cplx<TS>* const* in, const cplx<TS>* const* 
                  const double* vec);
 template <typename TB, int NY> int launch_y_inv(ns3d_ctx* c, int nf);
 template <typename TB, int NZ> int launch_z(ns3d_ctx* c, int nf);
-template <typename TB, int NY> int launch_y_fwd(ns3d_ctx* c, int nf);
+// P4: C (at A) -> D (d_at)
+template <typename TB, int NY> int launch_y_fwd(ns3d_ctx* c, int nf, bool chain);
 // P5; chain: with the P1 of the next stage (the RK3 loops' modes)
 template <typename TB, int MODE, int NX> int launch_x_fwd(ns3d_ctx* c, const EpiArgs& ea, int nf, bool chain);
 // standalone transforms of one field in the reference layout

@@ -105,20 +105,18 @@ int launch_z(ns3d_ctx* c, int nf) {
     return NS3D_OK;
 }
 
-// C -> D at the head of region B
 template <typename TB, int NY>
-int launch_y_fwd(ns3d_ctx* c, int nf) {
+int launch_y_fwd(ns3d_ctx* c, int nf, bool chain) {
     const int nz = c->batch, Mi = mi_of(c);
     const long nc = c->nci, bsc = c->bsc;
     cplx<TB>* A = (cplx<TB>*)c->scratch;
-    cplx<TB>* B = A + (long)6 * nf * nc;
     hipStream_t s = c->stream;
     constexpr int E = E_C2C<TB>;
     constexpr int P = PXY_T<TB, NY, E, NS3D_PYFWD32, 8>;
     const int nlt = (c->Mz + P - 1) / P;
     const int nb = c->Nx * nlt;
     dim3 grid = xgrid(nb, 3, nz), blk(P * XYPlan<NY, E>::TPP);
-    hipLaunchKernelGGL((k_axis_c2c<TB, NY, P, -1, 1, E>), grid, blk, 0, s, A, B, 3, nc, c->Ny, c->Mz, Mi, nlt, nb,
+    hipLaunchKernelGGL((k_axis_c2c<TB, NY, P, -1, 1, E>), grid, blk, 0, s, A, d_at<TB>(c, nf, chain), 3, nc, c->Ny, c->Mz, Mi, nlt, nb,
                        twp<TB>(c, 1), nt_for<TB>(c, P, FIELDS_P34), bsc, c->mm);
     return NS3D_OK;
 }
@@ -126,7 +124,7 @@ int launch_y_fwd(ns3d_ctx* c, int nf) {
 template <typename TB, int MODE, int NX>
 int launch_x_fwd(ns3d_ctx* c, const EpiArgs& ea, int nf, bool chain) {
     cplx<TB>* A = (cplx<TB>*)c->scratch;
-    const cplx<TB>* D = A + (long)6 * nf * c->nci;
+    const cplx<TB>* D = d_at<TB>(c, nf, chain);
     constexpr int E = E_XFWD<TB, NX>;
     constexpr int P0 = sizeof(TB) == 8 ? 8 : NS3D_BY_RADIX(NX, NS3D_PXFWD32, NS3D_R3_PXFWD32);
     constexpr int P = PXY_T<TB, NX, E, P0, P0>;

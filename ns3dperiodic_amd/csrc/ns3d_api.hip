@@ -251,18 +251,17 @@ bool can_chain(const ns3d_ctx* c) {
 }
 
 // ---------------------------------------------------------------- fused pipeline
-// Runs P1..P4 for NF vector fields and leaves D (3 fields) at the head of region B
-// (scratch + 6*nf*nci), so that A is free for the P1 output of the next stage.
+// Runs P1..P4 for NF vector fields and leaves D (3 fields) at d_at(c, nf, chain).
 // mw: row stride of the input fields (0: Mz, the reference layout)
 // bin: batch member stride of the inputs (c->batch members, scratch c->bsc apart).
-// has_a: the previous stage's x-forward pass left P1's output in A (CHAIN), in is not read.
+// has_a: the previous stage's x-forward pass left P1's output in A (CHAIN), in is not read;
+// chain: this stage's will (both only where can_chain(c)).
 // in2 (nf = 1 only, may be null): a second field of in's type and layout added
 // to the input before the transforms (the FP32-increment loop's base + increment).
 // vec (nf = 2 only, may be null): the second vector field as a reduced Krylov vector.
 template <typename TB, typename TS = double>
-int run_nonlinear_passes(ns3d_ctx* c, const cplx<TS>* const* in, int nf, int mw = 0, long bin = 0, bool has_a = false,
+int run_nonlinear_passes(ns3d_ctx* c, const cplx<TS>* const* in, int nf, int mw, long bin, bool has_a, bool chain,
                          const cplx<TS>* const* in2 = nullptr, const double* vec = nullptr) {
-    has_a = has_a && can_chain(c);
     if (mw == 0) mw = c->Mz;
     int st = ensure_scratch(c, 15 * nf * c->batch);
     if (st) return st;
@@ -281,15 +280,14 @@ int run_nonlinear_passes(ns3d_ctx* c, const cplx<TS>* const* in, int nf, int mw 
     prof_end(c);
     if (st) return st;
     prof_begin(c, 3);
-    st = with_size(c->Ny, [&](auto N) { return launch_y_fwd<TB, decltype(N)::value>(c, nf); });
+    st = with_size(c->Ny, [&](auto N) { return launch_y_fwd<TB, decltype(N)::value>(c, nf, chain); });
     prof_end(c);
     return st;
 }
 
 // P5 for nf fields' D; chain: with the P1 of the next stage (the RK3 loops' modes).
 template <typename TB, int MODE>
-int run_x_forward_epilogue(ns3d_ctx* c, const EpiArgs& ea, int nf = 1, bool chain = false) {
-    chain = chain && can_chain(c);
+int run_x_forward_epilogue(ns3d_ctx* c, const EpiArgs& ea, int nf, bool chain) {
     prof_begin(c, 4);
     int st = with_size(c->Nx, [&](auto N) { return launch_x_fwd<TB, MODE, decltype(N)::value>(c, ea, nf, chain); });
     prof_end(c);
@@ -319,12 +317,14 @@ EpiArgs make_epi(const ns3d_ctx* c) {
 template <int MODE>
 int fused(ns3d_ctx* c, const zd* const* in, int nf, const EpiArgs& ea, bool has_a = false, bool chain = false) {
     int st;
+    has_a = has_a && can_chain(c);
+    chain = chain && can_chain(c);
     if (c->precision == NS3D_FP64) {
-        st = run_nonlinear_passes<double, double>(c, in, nf, ea.mw, ea.bw, has_a, (const zd* const*)nullptr, ea.vin);
+        st = run_nonlinear_passes<double, double>(c, in, nf, ea.mw, ea.bw, has_a, chain, (const zd* const*)nullptr, ea.vin);
         if (st) return st;
         st = run_x_forward_epilogue<double, MODE>(c, ea, nf, chain);
     } else {
-        st = run_nonlinear_passes<float, double>(c, in, nf, ea.mw, ea.bw, has_a, (const zd* const*)nullptr, ea.vin);
+        st = run_nonlinear_passes<float, double>(c, in, nf, ea.mw, ea.bw, has_a, chain, (const zd* const*)nullptr, ea.vin);
         if (st) return st;
         st = run_x_forward_epilogue<float, MODE>(c, ea, nf, chain);
     }
@@ -394,7 +394,9 @@ int stage_into32(ns3d_ctx* c, const cf* const w[3], const cf* const u0[3], doubl
     ea.a0 = a0;
     ea.a1 = a1;
     ea.mw = ea.mu0 = ea.mo = c->m16;  // the FP32 state and stages use rows padded to m16
-    int st = run_nonlinear_passes<float, float>(c, w, 1, c->m16, 0, has_a);
+    has_a = has_a && can_chain(c);
+    chain = chain && can_chain(c);
+    int st = run_nonlinear_passes<float, float>(c, w, 1, c->m16, 0, has_a, chain);
     if (st) return st;
     st = run_x_forward_epilogue<float, EPI_STAGE32>(c, ea, 1, chain);
     if (st) return st;
@@ -448,7 +450,9 @@ int stage_incr(ns3d_ctx* c, bool first, double a1, bool last, const zd* const f[
     }
     ea.a1 = a1;
     ea.mw = ea.mo = ea.mu0 = c->m16;
-    int st = run_nonlinear_passes<float, float>(c, hic, 1, c->m16, 0, has_a, first ? nullptr : dc);
+    has_a = has_a && can_chain(c);
+    chain = chain && can_chain(c);
+    int st = run_nonlinear_passes<float, float>(c, hic, 1, c->m16, 0, has_a, chain, first ? nullptr : dc);
     if (st) return st;
     st = last ? run_x_forward_epilogue<float, EPI_INC_FINAL>(c, ea, 1, chain)
               : run_x_forward_epilogue<float, EPI_INC>(c, ea, 1, chain);

@@ -9,7 +9,7 @@
     template int launch_x_inv<T, double, N>(ns3d_ctx*, const zd* const*, const zd* const*, int, int, long, const double*); \
     template int launch_y_inv<T, N>(ns3d_ctx*, int);                             \
     template int launch_z<T, N>(ns3d_ctx*, int);                                 \
-    template int launch_y_fwd<T, N>(ns3d_ctx*, int);                             \
+    template int launch_y_fwd<T, N>(ns3d_ctx*, int, bool);                       \
     template int launch_c2c<T, N>(ns3d_ctx*, int, int, const cplx<T>*, cplx<T>*); \
     template int launch_c2r<T, N>(ns3d_ctx*, const cplx<T>*, T*, bool);          \
     template int launch_r2c<T, N>(ns3d_ctx*, const T*, cplx<T>*);
