@@ -18,7 +18,7 @@ int launch_x_inv(ns3d_ctx* c, const cplx<TS>* const* in, const cplx<TS>* const* 
     constexpr int OS = NS3D_OS_XINV;
     dim3 grid = xgrid(nb, 3 * nf * (OS ? 2 : 1), nz), blk(P * XYPlan<NX, E>::TPP);
     if (nf == 1 && in2) {
-        if constexpr (std::is_same<TS, float>::value && !CHAINS<TB, NX>) {
+        if constexpr (std::is_same<TS, float>::value && !CHAINS<TB, NX, EPI_INC>) {
             PtrArr<const cplx<TS>, 3> w{{in[0], in[1], in[2]}};
             PtrArr<const cplx<TS>, 3> w2{{in2[0], in2[1], in2[2]}};
             hipLaunchKernelGGL((k_x_inv_grad<TB, NX, P, 1, E, OS, TS, 1>), grid, blk, 0, s, w, A, nc, c->Ny, c->Mz, mw, Mi, nlt, nb, c->tab,
@@ -135,7 +135,7 @@ int launch_x_fwd(ns3d_ctx* c, const EpiArgs& ea, int nf, bool chain) {
         hipLaunchKernelGGL((k_x_fwd_epi<TB, NX, P, MODE, E, decltype(CH)::value, E_XINV<TB, NX>>), grid, blk, 0, c->stream, D, A,
                            c->nci, c->Ny, c->Mz, mi_of(c), nlt, nb, c->tab, twp<TB>(c, 0), ea, nt_for<TB>(c, P, FIELDS_P1 * nf), c->bsc, c->mm);
     };
-    constexpr bool CAN = CHAINS<TB, NX> && (MODE == EPI_STAGE || MODE == EPI_STAGE32 || MODE == EPI_INC || MODE == EPI_INC_FINAL);
+    constexpr bool CAN = CHAINS<TB, NX, MODE> && (MODE == EPI_STAGE || MODE == EPI_STAGE32 || MODE == EPI_INC || MODE == EPI_INC_FINAL);
     if constexpr (CAN) {
         if (chain) launch(std::integral_constant<int, 1>{});
         else launch(std::integral_constant<int, 0>{});

@@ -239,12 +239,13 @@ int ensure_fp64(ns3d_ctx* c, zd** p, int fields) {
     return NS3D_OK;
 }
 
-// Whether this grid's x-forward pass carries the next stage's P1 (CHAINS).
+// Whether this grid's x-forward pass with the MODE epilogue carries the next stage's P1 (CHAINS).
+template <int MODE>
 bool can_chain(const ns3d_ctx* c) {
     bool r = false;
     with_size(c->Nx, [&](auto NXc) -> int {
         constexpr int NX = decltype(NXc)::value;
-        r = c->precision == NS3D_FP64 ? CHAINS<double, NX> : CHAINS<float, NX>;
+        r = c->precision == NS3D_FP64 ? CHAINS<double, NX, MODE> : CHAINS<float, NX, MODE>;
         return 0;
     });
     return r;
@@ -255,7 +256,7 @@ bool can_chain(const ns3d_ctx* c) {
 // mw: row stride of the input fields (0: Mz, the reference layout)
 // bin: batch member stride of the inputs (c->batch members, scratch c->bsc apart).
 // has_a: the previous stage's x-forward pass left P1's output in A (CHAIN), in is not read;
-// chain: this stage's will (both only where can_chain(c)).
+// chain: this stage's will (both only where can_chain).
 // in2 (nf = 1 only, may be null): a second field of in's type and layout added
 // to the input before the transforms (the FP32-increment loop's base + increment).
 // vec (nf = 2 only, may be null): the second vector field as a reduced Krylov vector.
@@ -317,8 +318,8 @@ EpiArgs make_epi(const ns3d_ctx* c) {
 template <int MODE>
 int fused(ns3d_ctx* c, const zd* const* in, int nf, const EpiArgs& ea, bool has_a = false, bool chain = false) {
     int st;
-    has_a = has_a && can_chain(c);
-    chain = chain && can_chain(c);
+    has_a = has_a && can_chain<MODE>(c);
+    chain = chain && can_chain<MODE>(c);
     if (c->precision == NS3D_FP64) {
         st = run_nonlinear_passes<double, double>(c, in, nf, ea.mw, ea.bw, has_a, chain, (const zd* const*)nullptr, ea.vin);
         if (st) return st;
@@ -394,8 +395,8 @@ int stage_into32(ns3d_ctx* c, const cf* const w[3], const cf* const u0[3], doubl
     ea.a0 = a0;
     ea.a1 = a1;
     ea.mw = ea.mu0 = ea.mo = c->m16;  // the FP32 state and stages use rows padded to m16
-    has_a = has_a && can_chain(c);
-    chain = chain && can_chain(c);
+    has_a = has_a && can_chain<EPI_STAGE32>(c);
+    chain = chain && can_chain<EPI_STAGE32>(c);
     int st = run_nonlinear_passes<float, float>(c, w, 1, c->m16, 0, has_a, chain);
     if (st) return st;
     st = run_x_forward_epilogue<float, EPI_STAGE32>(c, ea, 1, chain);
@@ -450,8 +451,8 @@ int stage_incr(ns3d_ctx* c, bool first, double a1, bool last, const zd* const f[
     }
     ea.a1 = a1;
     ea.mw = ea.mo = ea.mu0 = c->m16;
-    has_a = has_a && can_chain(c);
-    chain = chain && can_chain(c);
+    has_a = has_a && can_chain<EPI_INC>(c);
+    chain = chain && can_chain<EPI_INC>(c);
     int st = run_nonlinear_passes<float, float>(c, hic, 1, c->m16, 0, has_a, chain, first ? nullptr : dc);
     if (st) return st;
     st = last ? run_x_forward_epilogue<float, EPI_INC_FINAL>(c, ea, 1, chain)
