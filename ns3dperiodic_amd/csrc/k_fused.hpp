@@ -235,6 +235,15 @@ k_x_inv_grad(PtrArr<const cplx<TS>, 3 * NF> w, cplx<TB>* __restrict__ A, long nc
 }
 
 // ---------------------------------------------------------------- P2
+// How P2 loads a thread's elements, of which some are masked.  Range
+// checked: all at once.  Behind branches: at the lengths with a radix-3 or radix-5 pass, where
+// a thread's last elements may not exist, most of the loads wait for the one before, and it is
+// the compiler's choice how many.  P2 behind branches and range checked, FP64: 384^3 1.69 and
+// 1.18 ms, 192^3 190 and 161 us, 160^3 115 and 81; FP32: 192^3 115 and 102, 320x384x320 735 and
+// 518, 128^3 in an RK3 step 29.3 and 27.0.  The branches stay for FP64 powers of two (64^3 in a
+// step 10.2 and 10.5 us), FP32 at 512 (512^3 1.65 and 1.82 ms) and at radix 5 (320^3 458 and 493 us).
+template <typename TB, int NY>
+constexpr bool Y_RANGE_LOADS = sizeof(TB) == 4 ? NY % 5 != 0 && NY < 512 : (NY & (NY - 1)) != 0;
 // y-inverse: B(w_b) , B(dx w_b) , B(i ky w_b).  Block: one x index j and P z
 // indices.  grid.y enumerates components; with OS = 1 each block produces one
 // of the three outputs (A_b is then read by two blocks): a third of the serial
@@ -266,35 +275,46 @@ k_y_inv_grad(const cplx<TB>* __restrict__ A, cplx<TB>* __restrict__ B, long nc, 
 #ifndef NS3D_HOIST
 #define NS3D_HOIST 1
 #endif
-    // x-derivative input, loaded before the first transforms when both are done here
-    cplx<TB> v2[(!OS && NS3D_HOIST) ? F::E : 1];
-    if constexpr (!OS && NS3D_HOIST) {
-        const cplx<TB>* __restrict__ src = A + (long)(s_ * 6 + 3 + b) * nc;
+    // A masked element is zero: RANGE: its load is out of a buffer's range, else it is not loaded.
+    constexpr bool RANGE = Y_RANGE_LOADS<TB, NY>;
+    int off[RANGE ? F::E : 1];   // byte offsets of this thread's elements in a field
+    if constexpr (RANGE) {
 #pragma unroll
         for (int q = 0; q < F::B0; q++) {
 #pragma unroll
             for (int r = 0; r < F::R0; r++) {
-                const int kk = F::in_index(t, q, r);
-                cplx<TB> s = mk<TB>(0, 0);
-                if (F::in_active(t, q) && lv && column_kept(tab, kk, l)) s = src[base + kk * S];
-                v2[q * F::R0 + r] = s;
+                const int kk = F::in_active(t, q) ? F::in_index(t, q, r) : 0;
+                const bool on = F::in_active(t, q) && lv && column_kept(tab, kk, lv ? l : 0);
+                off[q * F::R0 + r] = on ? (int)((base + kk * S) * (long)sizeof(cplx<TB>)) : BUF_OOB;
             }
         }
     }
-    // velocity component: produce w_b and dy w_b
-    if (!OS || which < 2) {
-        const cplx<TB>* __restrict__ src = A + (long)(s_ * 6 + b) * nc;
-        cplx<TB> v[F::E], d[OS ? 1 : F::E];
+    auto load = [&](cplx<TB>* x, int field) __attribute__((always_inline)) {
+        const cplx<TB>* __restrict__ src = A + (long)field * nc;
+        if constexpr (RANGE) {
+            const auto rs = buf_rsrc(src, (int)(nc * (long)sizeof(cplx<TB>)));
 #pragma unroll
-        for (int q = 0; q < F::B0; q++) {
+            for (int e = 0; e < F::B0 * F::R0; e++) x[e] = buf_load<TB>(rs, off[e]);
+        } else {
 #pragma unroll
-            for (int r = 0; r < F::R0; r++) {
-                const int kk = F::in_index(t, q, r);
-                cplx<TB> s = mk<TB>(0, 0);
-                if (F::in_active(t, q) && lv && column_kept(tab, kk, l)) s = src[base + kk * S];
-                v[q * F::R0 + r] = s;
+            for (int q = 0; q < F::B0; q++) {
+#pragma unroll
+                for (int r = 0; r < F::R0; r++) {
+                    const int kk = F::in_index(t, q, r);
+                    cplx<TB> s = mk<TB>(0, 0);
+                    if (F::in_active(t, q) && lv && column_kept(tab, kk, l)) s = src[base + kk * S];
+                    x[q * F::R0 + r] = s;
+                }
             }
         }
+    };
+    // x-derivative input, loaded before the first transforms when both are done here
+    cplx<TB> v2[(!OS && NS3D_HOIST) ? F::E : 1];
+    if constexpr (!OS && NS3D_HOIST) load(v2, s_ * 6 + 3 + b);
+    // velocity component: produce w_b and dy w_b
+    if (!OS || which < 2) {
+        cplx<TB> v[F::E], d[OS ? 1 : F::E];
+        load(v, s_ * 6 + b);
         if (NS3D_TW_LATE) stage_twiddles<TB, NY>(tw, twg);
 #pragma unroll
         for (int q = 0; q < F::B0; q++) {
@@ -337,17 +357,7 @@ k_y_inv_grad(const cplx<TB>* __restrict__ A, cplx<TB>* __restrict__ B, long nc, 
 #pragma unroll
             for (int e = 0; e < F::E; e++) v[e] = v2[e];
         } else {
-            const cplx<TB>* __restrict__ src = A + (long)(s_ * 6 + 3 + b) * nc;
-#pragma unroll
-            for (int q = 0; q < F::B0; q++) {
-#pragma unroll
-                for (int r = 0; r < F::R0; r++) {
-                    const int kk = F::in_index(t, q, r);
-                    cplx<TB> s = mk<TB>(0, 0);
-                    if (F::in_active(t, q) && lv && column_kept(tab, kk, l)) s = src[base + kk * S];
-                    v[q * F::R0 + r] = s;
-                }
-            }
+            load(v, s_ * 6 + 3 + b);
         }
         // with OS these blocks skip the velocity branch, where the table is staged otherwise
         if (NS3D_TW_LATE && OS) stage_twiddles<TB, NY>(tw, twg);
