@@ -338,29 +338,65 @@ __device__ __forceinline__ void weno_march(const TU* __restrict__ ux, const TU* 
     }
 }
 
+// The same, one cell a thread with its six faces and no barrier: for grids that marching
+// blocks do not fill the chip with, where latency is the kernel's time (weno_launch).
+template <int SCHEME, typename TU, class OUT>
+__device__ __forceinline__ void weno_cells(const TU* __restrict__ ux, const TU* __restrict__ uy,
+                                           const TU* __restrict__ uz, const double* __restrict__ x, const Grid3& G,
+                                           double rdx, double rdy, double rdz, bool q9, OUT&& out) {
+    constexpr int R = SCHEME == 5 ? 3 : (SCHEME == 3 ? 2 : 1);
+    const int id = xcd_tile() * blockDim.x + threadIdx.x;
+    if (id >= G.Nx * G.Ny * G.Nz) return;
+    const int l = id % G.Nz, jk = id / G.Nz, k = jk % G.Ny, j = jk / G.Ny;
+    const int n[3] = {G.Nx, G.Ny, G.Nz}, c[3] = {j, k, l}, s[3] = {G.Ny * G.Nz, G.Nz, 1};
+    const TU* u[3] = {ux, uy, uz};
+    const double rd[3] = {rdx, rdy, rdz}, xc = x[id];
+    double w[3][2 * R + 1], uw[3][3], adv = 0.0;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+#pragma unroll
+        for (int o = -R; o <= R; o++) {
+            const int at = id + (wrap_add(c[a], o, n[a]) - c[a]) * s[a];
+            w[a][o + R] = o == 0 ? xc : x[at];
+            if (o >= -1 && o <= 1) uw[a][o + 1] = (double)u[a][at];
+        }
+    }
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        const double U[2] = {0.5 * (uw[a][0] + uw[a][1]), 0.5 * (uw[a][1] + uw[a][2])};
+        double f[2];
+        weno_faces<SCHEME, 2>(w[a] + R - 1, 1, U, a == 2 && q9, f);
+        adv += uw[a][1] * (f[1] - f[0]) * rd[a];
+    }
+    out((long)id, xc, adv);
+}
+
 // advection kernel + flux_device (Source/advection_WENO.cu:304-392), generalised to any advected scalar x.
+// YC = 0: weno_cells.
 template <int SCHEME, int YC>
-__global__ void __attribute__((amdgpu_waves_per_eu(YC == 1 ? 4 : 3, 8))) __launch_bounds__(WENO_THREADS)
+__global__ void __attribute__((amdgpu_waves_per_eu(YC <= 1 ? 4 : 3, 8))) __launch_bounds__(WENO_THREADS)
 k_weno(const double* __restrict__ ux, const double* __restrict__ uy, const double* __restrict__ uz,
        const double* __restrict__ x, double* __restrict__ out, Grid3 G, int march, double rdx, double rdy, double rdz,
        int zfix) {
-    weno_march<SCHEME, YC>(ux, uy, uz, x, G, march, rdx, rdy, rdz, !zfix,
-                       [&](long id, double, double adv) __attribute__((always_inline)) { out[id] = adv; });
+    auto put = [&](long id, double, double adv) __attribute__((always_inline)) { out[id] = adv; };
+    if constexpr (YC == 0) weno_cells<SCHEME>(ux, uy, uz, x, G, rdx, rdy, rdz, !zfix, put);
+    else weno_march<SCHEME, YC>(ux, uy, uz, x, G, march, rdx, rdy, rdz, !zfix, put);
 }
 
 // SSP stage of a passive scalar: out = a0*th_n + a1*(th_s - dt * (u.grad)_WENO th_s),
 // u being the masked physical velocity of the same stage (TU = bulk precision).
 template <int SCHEME, int YC, typename TU>
-__global__ void __attribute__((amdgpu_waves_per_eu(YC == 1 ? 4 : 3, 8))) __launch_bounds__(WENO_THREADS)
+__global__ void __attribute__((amdgpu_waves_per_eu(YC <= 1 ? 4 : 3, 8))) __launch_bounds__(WENO_THREADS)
 k_weno_stage(const TU* __restrict__ u, long nr, const double* __restrict__ x, const double* xn, double* out, Grid3 G,
              int march, double rdx, double rdy, double rdz, int zfix, double dt, double a0, double a1, int* nf) {
-    weno_march<SCHEME, YC>(u, u + nr, u + 2 * nr, x, G, march, rdx, rdy, rdz, !zfix,
-                       [&](long id, double xc, double adv) __attribute__((always_inline)) {
-                           const double e = xc - dt * adv;
-                           const double o = xn ? a0 * xn[id] + a1 * e : a1 * e;
-                           out[id] = o;
-                           flag_nonfinite(nf, !isfinite(o));
-                       });
+    auto put = [&](long id, double xc, double adv) __attribute__((always_inline)) {
+        const double e = xc - dt * adv;
+        const double o = xn ? a0 * xn[id] + a1 * e : a1 * e;
+        out[id] = o;
+        flag_nonfinite(nf, !isfinite(o));
+    };
+    if constexpr (YC == 0) weno_cells<SCHEME>(u, u + nr, u + 2 * nr, x, G, rdx, rdy, rdz, !zfix, put);
+    else weno_march<SCHEME, YC>(u, u + nr, u + 2 * nr, x, G, march, rdx, rdy, rdz, !zfix, put);
 }
 
 __global__ void k_set_int(int* __restrict__ p, int v) {

@@ -666,14 +666,20 @@ RedArgs red_args(const ns3d_ctx* c, const double* a, const double* b, const doub
 }
 
 // ---------------------------------------------------------------- passive scalar RK3
-// Launch shape of the WENO march.  A thread takes two y cells (3.5 faces a cell) where the
-// registers that costs (3 waves a SIMD against 4) pay: WENO5 at 256^3 225 us against 242, 128^3
+// Launch shape of the WENO kernels.  One cell a thread (0 y cells: weno_cells) up to 3/8 M points,
+// where marching blocks do not fill the chip and their steps follow one another: WENO5 at 8^3 to
+// 32^3 3.8 us against 6.8 to 7.1 marching, 48^3 5.0 and 7.3, 64^3 7.4 and 7.7, 128x64x48 10.2 and
+// 10.7 (96x80x64 12.5 and 10.7); and up to 1/2 M where the marching blocks leave lanes idle (80^3
+// 12.6 and 13.0, WENO3 8.4 and 9.6).  A marching thread takes two y cells (3.5 faces a cell) where
+// the registers that costs (3 waves a SIMD against 4) pay: WENO5 at 256^3 225 us against 242, 128^3
 // 33.5 against 34.0, 96^3 22.6 against 20.9.  A block marches 16 planes, fewer while the grid has
 // under 4096 waves (96^3 with 4 planes 20.3 us, with 8 24.5; below 4 the extra x faces cost as much).
 template <class F>
 void weno_launch(const ns3d_ctx* c, F&& f) {
     const int rows = c->Nz >= 256 ? 1 : 256 / c->Nz;
     const int threads = (rows * c->Nz + 63) / 64 * 64;
+    if (c->nr <= (rows * c->Nz < threads ? 1L << 19 : 3L << 17))
+        return f(std::integral_constant<int, 0>{}, xgrid(nblk(c->nr, 256)), dim3(256), 0);
     const int yc = c->nr >= (1L << 21) ? 2 : 1;
     const long nyb = nblk(c->Ny, rows * yc);
     int march = 16;
