@@ -60,6 +60,10 @@ typedef struct { double x, y; } ns3d_cplx;
                                        flag: NS3D_ERR_NONFINITE if any stage wrote a NaN or Inf.  The reference
                                        checks for NaN in its time loop (NS3D_periodic.cu:1357-1360) */
 
+#define NS3D_FLAG_NO_CHAIN 0x10u   /* every RK3 stage runs its own x-inverse pass, where the x-forward pass of the
+                                       stage before would have carried it: the same bits, more slowly (a check of
+                                       the chained passes).  No reference counterpart */
+
 typedef struct {
     int Nx, Ny, Nz;        /* physical grid, each in {8,16,32,48,64,80,96,128,160,192,256,320,384,512} */
     double Lx, Ly, Lz;     /* box lengths (reference: 2*pi/alpha, 2*pi, 2*pi/beta, NS3D_periodic.cu:969-979) */

@@ -18,6 +18,7 @@ NS3D_FLAG_NO_IPQ = 0x1
 NS3D_FLAG_WENO_ZFIX = 0x2
 NS3D_FLAG_MASK_NYQUIST = 0x4
 NS3D_FLAG_CHECK_FINITE = 0x8
+NS3D_FLAG_NO_CHAIN = 0x10
 NS3D_ERR_NONFINITE = -5
 NS3D_ERR_CAPACITY = -7
 UPD_STAGE, UPD_UV_RHS, UPD_UV, UPD_IUV, UPD_RHS = 0, 1, 2, 3, 4

@@ -20,10 +20,12 @@
 namespace ns3d {
 
 // ---------------------------------------------------------------- radix DFTs
+// PIN: the fused multiply-adds spelled out, as in cmul_pinned (radices 2 and 4 have none to
+// spell out, 16 is in no pinned plan).
 template <int R> struct Radix;
 
 template <> struct Radix<2> {
-    template <int DIR, typename T> __device__ __forceinline__ static void dft(cplx<T>* v) {
+    template <int DIR, bool PIN = false, typename T> __device__ __forceinline__ static void dft(cplx<T>* v) {
         cplx<T> a = v[0], b = v[1];
         v[0] = a + b;
         v[1] = a - b;
@@ -31,16 +33,23 @@ template <> struct Radix<2> {
 };
 
 template <> struct Radix<3> {
-    template <int DIR, typename T> __device__ __forceinline__ static void dft(cplx<T>* v) {
+    template <int DIR, bool PIN = false, typename T> __device__ __forceinline__ static void dft(cplx<T>* v) {
         const T h = (T)0.86602540378443864676372317075294;  // sqrt(3)/2
         cplx<T> a0 = v[0], a1 = v[1], a2 = v[2];
         cplx<T> s = a1 + a2;
         cplx<T> d = a1 - a2;
         cplx<T> m = mk<T>(a0.x - (T)0.5 * s.x, a0.y - (T)0.5 * s.y);
-        cplx<T> r = mul_i<DIR>(cscale(d, h));
         v[0] = a0 + s;
-        v[1] = m + r;
-        v[2] = m - r;
+        if constexpr (PIN) {
+            const cplx<T> e = mul_i<DIR>(d);
+            m = mk<T>(fma_t((T)-0.5, s.x, a0.x), fma_t((T)-0.5, s.y, a0.y));
+            v[1] = fma_c(e, h, m);
+            v[2] = fma_c(e, -h, m);
+        } else {
+            const cplx<T> r = mul_i<DIR>(cscale(d, h));
+            v[1] = m + r;
+            v[2] = m - r;
+        }
     }
 };
 
@@ -59,11 +68,11 @@ template <> struct Radix<5> {
         const cplx<T> t1 = v[1] + v[4], t2 = v[2] + v[3];
         const cplx<T> t3 = v[1] - v[4], t4 = v[2] - v[3];
         cplx<T> m1, m2, n1, n2;
-        if constexpr (PIN) {  // contraction spelled out, as in cmul_pinned
-            m1 = mk<T>(__builtin_fma(c2, t2.x, __builtin_fma(c1, t1.x, a0.x)), __builtin_fma(c2, t2.y, __builtin_fma(c1, t1.y, a0.y)));
-            m2 = mk<T>(__builtin_fma(c1, t2.x, __builtin_fma(c2, t1.x, a0.x)), __builtin_fma(c1, t2.y, __builtin_fma(c2, t1.y, a0.y)));
-            n1 = mul_i<DIR>(mk<T>(__builtin_fma(s1, t3.x, s2 * t4.x), __builtin_fma(s1, t3.y, s2 * t4.y)));
-            n2 = mul_i<DIR>(mk<T>(__builtin_fma(s2, t3.x, -(s1 * t4.x)), __builtin_fma(s2, t3.y, -(s1 * t4.y))));
+        if constexpr (PIN) {
+            m1 = mk<T>(fma_t(c2, t2.x, fma_t(c1, t1.x, a0.x)), fma_t(c2, t2.y, fma_t(c1, t1.y, a0.y)));
+            m2 = mk<T>(fma_t(c1, t2.x, fma_t(c2, t1.x, a0.x)), fma_t(c1, t2.y, fma_t(c2, t1.y, a0.y)));
+            n1 = mul_i<DIR>(mk<T>(fma_t(s1, t3.x, s2 * t4.x), fma_t(s1, t3.y, s2 * t4.y)));
+            n2 = mul_i<DIR>(mk<T>(fma_t(s2, t3.x, -(s1 * t4.x)), fma_t(s2, t3.y, -(s1 * t4.y))));
         } else {
             m1 = mk<T>(a0.x + c1 * t1.x + c2 * t2.x, a0.y + c1 * t1.y + c2 * t2.y);
             m2 = mk<T>(a0.x + c2 * t1.x + c1 * t2.x, a0.y + c2 * t1.y + c1 * t2.y);
@@ -79,7 +88,7 @@ template <> struct Radix<5> {
 };
 
 template <> struct Radix<4> {
-    template <int DIR, typename T> __device__ __forceinline__ static void dft(cplx<T>* v) {
+    template <int DIR, bool PIN = false, typename T> __device__ __forceinline__ static void dft(cplx<T>* v) {
         cplx<T> s02 = v[0] + v[2], d02 = v[0] - v[2];
         cplx<T> s13 = v[1] + v[3], d13 = mul_i<DIR>(v[1] - v[3]);
         v[0] = s02 + s13;
@@ -90,24 +99,31 @@ template <> struct Radix<4> {
 };
 
 template <> struct Radix<8> {
-    template <int DIR, typename T> __device__ __forceinline__ static void dft(cplx<T>* v) {
+    template <int DIR, bool PIN = false, typename T> __device__ __forceinline__ static void dft(cplx<T>* v) {
         const T c = (T)0.70710678118654752440084436210485;  // 1/sqrt(2)
         cplx<T> e[4] = {v[0], v[2], v[4], v[6]};
         cplx<T> o[4] = {v[1], v[3], v[5], v[7]};
         Radix<4>::dft<DIR>(e);
         Radix<4>::dft<DIR>(o);
         // W8^1 = (1 + DIR i)/sqrt2, W8^2 = DIR i, W8^3 = (-1 + DIR i)/sqrt2
-        cplx<T> o1 = cscale(o[1] + mul_i<DIR>(o[1]), c);
+        const cplx<T> s1 = o[1] + mul_i<DIR>(o[1]), s3 = mul_i<DIR>(o[3]) - o[3];
         cplx<T> o2 = mul_i<DIR>(o[2]);
-        cplx<T> o3 = cscale(mul_i<DIR>(o[3]) - o[3], c);
         v[0] = e[0] + o[0];
         v[4] = e[0] - o[0];
-        v[1] = e[1] + o1;
-        v[5] = e[1] - o1;
         v[2] = e[2] + o2;
         v[6] = e[2] - o2;
-        v[3] = e[3] + o3;
-        v[7] = e[3] - o3;
+        if constexpr (PIN) {
+            v[1] = fma_c(s1, c, e[1]);
+            v[5] = fma_c(s1, -c, e[1]);
+            v[3] = fma_c(s3, c, e[3]);
+            v[7] = fma_c(s3, -c, e[3]);
+        } else {
+            const cplx<T> o1 = cscale(s1, c), o3 = cscale(s3, c);
+            v[1] = e[1] + o1;
+            v[5] = e[1] - o1;
+            v[3] = e[3] + o3;
+            v[7] = e[3] - o3;
+        }
     }
 };
 
@@ -329,7 +345,7 @@ template <typename T, int K> struct TwRegs {
     cplx<T> w[K];
 };
 
-// PIN: every product's contraction spelled out (cmul_pinned).
+// PIN: every product's contraction spelled out (cmul_pinned, Radix).
 template <typename T, int N, int TPP, int DIR, typename S, typename Addr, bool WAVE = false, bool PIN = false, bool SWAP = false>
 struct PencilFFT {
     using Info = SeqInfo<S>;
@@ -412,7 +428,7 @@ struct PencilFFT {
                         v[q * R + r] = PIN ? cmul_pinned(v[q * R + r], w) : cmul(v[q * R + r], w);
                     }
                 }
-                if constexpr (R == 5 && PIN)
+                if constexpr (PIN)
                     Radix<R>::template dft<DIR, true>(v + q * R);
                 else
                     Radix<R>::template dft<DIR>(v + q * R);

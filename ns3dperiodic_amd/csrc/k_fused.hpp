@@ -143,6 +143,8 @@ template <typename TB, int NX> constexpr bool MIRROR_P1 = sizeof(TB) == 8 && NX 
 template <typename TB, int NX, int E>
 using XInvPlan = typename std::conditional<MIRROR_P1<TB, NX>, typename SeqRev<typename XYPlan<NX, E>::R>::type,
                                            typename XYPlan<NX, E>::R>::type;
+// P1's transforms are pinned (PencilFFT's PIN) wherever the x-forward pass may carry them.
+template <typename TB, int NX> constexpr bool PIN_P1 = sizeof(TB) == 8 || NX % 5 != 0;
 // i kx w: the products rounded by themselves (the transform's additions must not absorb them).
 template <typename TB> __device__ __forceinline__ cplx<TB> ikx(cplx<double> s, double kx) {
     return mk<TB>((TB)mul_rounded(-s.y, kx), (TB)mul_rounded(s.x, kx));
@@ -153,7 +155,7 @@ k_x_inv_grad(PtrArr<const cplx<TS>, 3 * NF> w, cplx<TB>* __restrict__ A, long nc
              int nlt, int nb, SpecTables tab, const cplx<TB>* __restrict__ twg, int nt, long bwi, long bsc,
              MemberMask mm, PtrArr<const cplx<TS>, 3> w2 = {}, const double* __restrict__ vec = nullptr) {
     constexpr int TPP = XYPlan<NX, E>::TPP;
-    using F = PencilFFT<TB, NX, TPP, +1, XInvPlan<TB, NX, E>, IndexMajor<P>, false, sizeof(TB) == 8>;
+    using F = PencilFFT<TB, NX, TPP, +1, XInvPlan<TB, NX, E>, IndexMajor<P>, false, PIN_P1<TB, NX>>;
     __shared__ cplx<TB> lds[NX * P];
     __shared__ cplx<TB> tw[NX];
     const int bid0 = xcd_tile();
@@ -1431,8 +1433,9 @@ k_x_fwd_epi(const cplx<TB>* D, cplx<TB>* A, long nc, int Ny, int Mz, int Ms, int
         } else {
             // the standalone P1's plan on half the threads for each transform
             constexpr int TPI = XYPlan<NX, EI>::TPP;
+            static_assert(!CHAIN || PIN_P1<TB, NX>, "the standalone P1 rounds alike");
             static_assert(!CHAIN || TPP == 2 * TPI, "half of a pencil's threads run each of its two inverse transforms");
-            using FI = PencilFFT<TB, NX, TPI, +1, typename XYPlan<NX, EI>::R, IndexMajor<P>>;
+            using FI = PencilFFT<TB, NX, TPI, +1, typename XYPlan<NX, EI>::R, IndexMajor<P>, false, PIN_P1<TB, NX>>;
 #pragma unroll
             for (int e = 0; e < NO; e++) {
                 const int q = e / F::RL, j = F::out_index(t, q, e % F::RL);

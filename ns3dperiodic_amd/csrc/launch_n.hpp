@@ -18,7 +18,7 @@ int launch_x_inv(ns3d_ctx* c, const cplx<TS>* const* in, const cplx<TS>* const* 
     constexpr int OS = NS3D_OS_XINV;
     dim3 grid = xgrid(nb, 3 * nf * (OS ? 2 : 1), nz), blk(P * XYPlan<NX, E>::TPP);
     if (nf == 1 && in2) {
-        if constexpr (std::is_same<TS, float>::value && !CHAINS<TB, NX, EPI_INC>) {
+        if constexpr (std::is_same<TS, float>::value) {
             PtrArr<const cplx<TS>, 3> w{{in[0], in[1], in[2]}};
             PtrArr<const cplx<TS>, 3> w2{{in2[0], in2[1], in2[2]}};
             hipLaunchKernelGGL((k_x_inv_grad<TB, NX, P, 1, E, OS, TS, 1>), grid, blk, 0, s, w, A, nc, c->Ny, c->Mz, mw, Mi, nlt, nb, c->tab,

@@ -243,6 +243,7 @@ int ensure_fp64(ns3d_ctx* c, zd** p, int fields) {
 template <int MODE>
 bool can_chain(const ns3d_ctx* c) {
     bool r = false;
+    if (c->flags & NS3D_FLAG_NO_CHAIN) return r;
     with_size(c->Nx, [&](auto NXc) -> int {
         constexpr int NX = decltype(NXc)::value;
         r = c->precision == NS3D_FP64 ? CHAINS<double, NX, MODE> : CHAINS<float, NX, MODE>;

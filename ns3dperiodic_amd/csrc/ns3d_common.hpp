@@ -20,10 +20,18 @@ template <typename T> __device__ __forceinline__ cplx<T> mk(T a, T b) { cplx<T> 
 template <typename T> __device__ __forceinline__ cplx<T> operator+(cplx<T> a, cplx<T> b) { return mk<T>(a.x + b.x, a.y + b.y); }
 template <typename T> __device__ __forceinline__ cplx<T> operator-(cplx<T> a, cplx<T> b) { return mk<T>(a.x - b.x, a.y - b.y); }
 template <typename T> __device__ __forceinline__ cplx<T> cmul(cplx<T> a, cplx<T> b) { return mk<T>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
-// The same with the fused multiply-adds spelled out, for transforms that two kernels have to
-// round alike (elsewhere the compiler's own choice gives shorter schedules).
+// One fused multiply-add a b + c of the operands' precision.
+__device__ __forceinline__ double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+// cmul with the fused multiply-adds spelled out, for transforms that two kernels have to
+// round alike (elsewhere the compiler's own choice gives shorter schedules).  In FP32 the second
+// component as the compiler forms it for a conjugate twiddle.
 template <typename T> __device__ __forceinline__ cplx<T> cmul_pinned(cplx<T> a, cplx<T> b) {
-    return mk<T>(__builtin_fma(a.x, b.x, -(a.y * b.y)), __builtin_fma(a.x, b.y, a.y * b.x));
+    return mk<T>(fma_t(a.x, b.x, -(a.y * b.y)), sizeof(T) == 8 ? fma_t(a.x, b.y, a.y * b.x) : fma_t(a.y, b.x, a.x * b.y));
+}
+// a s + b, each component one fused multiply-add.
+template <typename T> __device__ __forceinline__ cplx<T> fma_c(cplx<T> a, T s, cplx<T> b) {
+    return mk<T>(fma_t(a.x, s, b.x), fma_t(a.y, s, b.y));
 }
 // A product rounded by itself, never contracted into a following addition.
 template <typename T> __device__ __forceinline__ T mul_rounded(T a, T b) {

@@ -34,7 +34,7 @@ class NS3D:
 
     def __init__(self, Nx, Ny=None, Nz=None, Lx=2 * math.pi, Ly=2 * math.pi, Lz=2 * math.pi,
                  Re=100.0, dt=1e-3, precision="fp64", ipq=True, weno_zfix=False, device=0, stream=None,
-                 mask_nyquist=False, check_finite=False):
+                 mask_nyquist=False, check_finite=False, chain_stages=True):
         self.lib = _lib.load()
         Ny = Nx if Ny is None else Ny
         Nz = Nx if Nz is None else Nz
@@ -44,7 +44,8 @@ class NS3D:
         self.device = torch.device("cuda", device)
         flags = ((0 if ipq else _lib.NS3D_FLAG_NO_IPQ) | (_lib.NS3D_FLAG_WENO_ZFIX if weno_zfix else 0)
                  | (_lib.NS3D_FLAG_MASK_NYQUIST if mask_nyquist else 0)
-                 | (_lib.NS3D_FLAG_CHECK_FINITE if check_finite else 0))
+                 | (_lib.NS3D_FLAG_CHECK_FINITE if check_finite else 0)
+                 | (0 if chain_stages else _lib.NS3D_FLAG_NO_CHAIN))
         # "fp32": FP32 transforms, FP64 state; "fp32s": also FP32 state inside the RK3 loops;
         # "fp32i": FP32 transforms and FP32 stage increments over the FP64 state
         prec = {"fp64": _lib.NS3D_FP64, "fp32": _lib.NS3D_FP32_BULK, "fp32s": _lib.NS3D_FP32_STATE,
