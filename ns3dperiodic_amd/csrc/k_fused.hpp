@@ -1074,19 +1074,14 @@ __device__ __forceinline__ void flag_nonfinite(int* nf, bool bad) {
 }
 template <typename T> __device__ __forceinline__ bool finite2(cplx<T> a) { return isfinite(a.x) && isfinite(a.y); }
 
-// Projection/diffusion/update at one mode (Source/diffusion.cu:96-365).
+// Projection/diffusion/update at one mode (Source/diffusion.cu:96-365), k_update's.
 template <int MODE>
 __device__ __forceinline__ void epilogue(const EpiArgs& ea, const SpecTables& tab, int j, int k, int l,
                                          cplx<double> Qx, cplx<double> Qy, cplx<double> Qz) {
     const long row = (long)j * ea.ny + k;
-    const long gw = row * ea.mw + l, gu = row * ea.mu0 + l, go = row * ea.mo + l, gf = row * ea.mf + l;
-    if (MODE == EPI_Q) {
-        ea.out[0][go] = Qx;
-        ea.out[1][go] = Qy;
-        ea.out[2][go] = Qz;
-        flag_nonfinite(ea.nf, !(finite2(Qx) && finite2(Qy) && finite2(Qz)));
-        return;
-    }
+    const long gw = row * ea.mw + l, go = row * ea.mo + l, gf = row * ea.mf + l;
+    static_assert(MODE == EPI_STAGE || MODE == EPI_RHS || MODE == EPI_UV || MODE == EPI_UV_RHS || MODE == EPI_IUV,
+                  "the updates of ns3d_project_update");
     bool bad = false;
     const ProjCoef c = proj_coef(tab, j, k, l);
     const double AQr[3] = {c.a11 * Qx.x + c.a12 * Qy.x + c.a13 * Qz.x, c.a12 * Qx.x + c.a22 * Qy.x + c.a23 * Qz.x,
@@ -1098,52 +1093,6 @@ __device__ __forceinline__ void epilogue(const EpiArgs& ea, const SpecTables& ta
 #pragma unroll
     for (int b = 0; b < 3; b++) {
         cplx<double> r;
-        if (MODE == EPI_STAGE32) {
-            const cplx<double> w = cvt<double>(reinterpret_cast<const cplx<float>*>(ea.w[b])[gw]);
-            const double G = (1.0 - c.din * ea.dtnu);
-            cplx<double> f = mk<double>(0.0, 0.0);
-            if (ea.f[b]) f = ea.f[b][gf];
-            r.x = dt * AQr[b] + G * w.x + dt * f.x - dt * Q[b].x;
-            r.y = dt * AQi[b] + G * w.y + dt * f.y - dt * Q[b].y;
-            if (ea.u0[b]) {
-                const cplx<double> u0 = cvt<double>(reinterpret_cast<const cplx<float>*>(ea.u0[b])[gu]);
-                r.x = ea.a0 * u0.x + ea.a1 * r.x;
-                r.y = ea.a0 * u0.y + ea.a1 * r.y;
-            }
-            const cplx<float> rf = cvt<float>(r);
-            reinterpret_cast<cplx<float>*>(ea.out[b])[go] = rf;
-            bad |= !finite2(rf);
-            continue;
-        }
-        if (MODE == EPI_INC || MODE == EPI_INC_FINAL) {
-            cplx<float>* hi = reinterpret_cast<cplx<float>*>(ea.w[b]);
-            cplx<double> base = cvt<double>(hi[gw]);
-            if (MODE == EPI_INC_FINAL) {
-                const cplx<float> lo = ea.out32[b][gw];
-                base.x += (double)lo.x;
-                base.y += (double)lo.y;
-            }
-            const cplx<double> d =
-                ea.u0[b] ? cvt<double>(reinterpret_cast<const cplx<float>*>(ea.u0[b])[gu]) : mk<double>(0.0, 0.0);
-            cplx<double> f = mk<double>(0.0, 0.0);
-            if (ea.f[b]) f = ea.f[b][gf];
-            const double Gd = c.din * ea.dtnu;
-            r.x = ea.a1 * (d.x + (dt * AQr[b] - Gd * (base.x + d.x) + dt * f.x - dt * Q[b].x));
-            r.y = ea.a1 * (d.y + (dt * AQi[b] - Gd * (base.y + d.y) + dt * f.y - dt * Q[b].y));
-            if (MODE == EPI_INC) {
-                const cplx<float> rf = cvt<float>(r);
-                reinterpret_cast<cplx<float>*>(ea.out[b])[go] = rf;
-                bad |= !finite2(rf);
-            } else {
-                r.x += base.x;
-                r.y += base.y;
-                const cplx<float> h = cvt<float>(r);
-                hi[gw] = h;
-                ea.out32[b][gw] = mk<float>((float)(r.x - (double)h.x), (float)(r.y - (double)h.y));
-                bad |= !finite2(r);
-            }
-            continue;
-        }
         const cplx<double> w = ea.w[b][gw];
         if (MODE == EPI_STAGE) {
             const double G = (1.0 - c.din * ea.dtnu);
@@ -1151,11 +1100,6 @@ __device__ __forceinline__ void epilogue(const EpiArgs& ea, const SpecTables& ta
             if (ea.f[b]) f = ea.f[b][gf];
             r.x = dt * AQr[b] + G * w.x + dt * f.x - dt * Q[b].x;
             r.y = dt * AQi[b] + G * w.y + dt * f.y - dt * Q[b].y;
-            if (ea.u0[b]) {
-                const cplx<double> u0 = ea.u0[b][gu];
-                r.x = ea.a0 * u0.x + ea.a1 * r.x;
-                r.y = ea.a0 * u0.y + ea.a1 * r.y;
-            }
             ea.out[b][go] = r;
             bad |= !finite2(r);
         } else if (MODE == EPI_RHS) {
@@ -1203,7 +1147,7 @@ __device__ __forceinline__ void ipq_rule(cplx<double>& Qx, cplx<double>& Qy, cpl
     }
 }
 
-// ---- P5 kernel: the epilogue above, its operands read ahead.
+// ---- P5 kernel: the epilogues of every mode, their operands read ahead.
 // Scalar type of the state operands w, u0 and out in memory.
 template <int MODE>
 using EpiState = typename std::conditional<MODE == EPI_STAGE32 || MODE == EPI_INC || MODE == EPI_INC_FINAL, float,
