@@ -34,8 +34,9 @@ def pass_bytes(nc, bulk_bytes, state_bytes=16):
     reads 9, writes 3; P4 reads 3, writes 3; P5 reads 3 bulk + 3 state (+3
     u^n in stages 2-3) and writes 3 state.  State fields are FP64 complex
     (16 B) except in the FP32-state loop (8 B); bulk fields use the bulk
-    precision.  With one precision throughout the RK3 step totals 159 S, the
-    algorithmic byte count of the path.
+    precision.  With one precision throughout an RK3 step whose three stages
+    launch all five passes totals 159 S; launched_bytes counts what a call
+    launches.
     """
     s, b = state_bytes * nc, bulk_bytes * nc
     p5_avg = 3 * b + 3 * s + 3 * s + (2.0 / 3.0) * 3 * s
@@ -59,6 +60,30 @@ def pass_bytes_incr(nc):
     not counted)."""
     S = 8 * nc
     return [11 * S, 15 * S, 12 * S, 6 * S, 13 * S]
+
+
+def launched_bytes(pb, nc, bulk_bytes, steps, p1_launches, p1_bytes=None):
+    """Algorithmic HBM bytes per step of one call of `steps` RK3 steps with
+    p1_launches launches of P1 (p1_bytes each, pb[0] by default): the other
+    stages' P1 output (6 bulk fields) is written by the x-forward pass of the
+    stage before, and their P1 reads nothing.  pb: pass_bytes or
+    pass_bytes_incr."""
+    n = 3 * steps
+    p1 = p1_launches * (pb[0] if p1_bytes is None else p1_bytes) + (n - p1_launches) * 6 * bulk_bytes * nc
+    return (p1 + n * sum(pb[1:])) / steps
+
+
+def profiled_passes(g, call):
+    """Device ms and launches of each pass during call()."""
+    import ctypes
+    import torch
+    ms, calls = (ctypes.c_double * 5)(), (ctypes.c_longlong * 5)()
+    g.lib.ns3d_profile_enable(g.ctx, 1)
+    call()
+    torch.cuda.synchronize()
+    g.lib.ns3d_profile_read(g.ctx, ms, calls)
+    g.lib.ns3d_profile_enable(g.ctx, 0)
+    return list(ms), list(calls)
 
 
 def profiled_traffic(precision, kernel_prefix):
@@ -88,8 +113,6 @@ def run_gpu(N, precision, steps, warmup, u0, Re, dt):
     u = [torch.from_numpy(c).to("cuda:0") for c in u0]
     g.RK3_SSP(u, None, steps=warmup)
     torch.cuda.synchronize()
-    lib = g.lib
-    import ctypes
     # the timed steps run without per-pass events; a shorter run with them
     # (HIP events around every pass, on the library's stream) gives the pass times
     stream = torch.cuda.current_stream()
@@ -101,13 +124,7 @@ def run_gpu(N, precision, steps, warmup, u0, Re, dt):
     e1.record(stream)
     torch.cuda.synchronize()
     wall = time.perf_counter() - t0
-    lib.ns3d_profile_enable(g.ctx, 1)
-    g.RK3_SSP(u, None, steps=max(1, min(steps, 10)))
-    torch.cuda.synchronize()
-    ms = (ctypes.c_double * 5)()
-    calls = (ctypes.c_longlong * 5)()
-    lib.ns3d_profile_read(g.ctx, ms, calls)
-    lib.ns3d_profile_enable(g.ctx, 0)
+    ms, calls = profiled_passes(g, lambda: g.RK3_SSP(u, None, steps=max(1, min(steps, 10))))
     total_ms = e0.elapsed_time(e1)
     finite = bool(torch.isfinite(u[0]).all().item())
     g.close()
@@ -115,7 +132,9 @@ def run_gpu(N, precision, steps, warmup, u0, Re, dt):
     state = 8 if precision == "fp32s" else 16
     nc = N * N * (N // 2 + 1)
     pb = pass_bytes_incr(nc) if precision == "fp32i" else pass_bytes(nc, bulk, state)
-    sb = 3 * sum(pb) if precision == "fp32i" else step_bytes(nc, bulk, state)
+    # the timed call launched P1 for its first stage only, or for every stage (the first reads hi alone in fp32i)
+    p1_launches = 1 if calls[0] < calls[4] else 3 * steps
+    sb = launched_bytes(pb, nc, bulk, steps, p1_launches, 9 * bulk * nc if precision == "fp32i" and p1_launches == 1 else None)
     # an x-forward launch that no P1 launch follows writes the next stage's P1 output (6 bulk fields) itself
     if calls[4]:
         pb[4] += 6 * bulk * nc * max(0, calls[4] - calls[0]) / calls[4]
@@ -140,7 +159,7 @@ def run_gpu(N, precision, steps, warmup, u0, Re, dt):
 
 def run_scalar(N, steps, warmup, u0, theta0, Re, dt):
     """RK3 of the velocity plus a WENO5-advected passive scalar (FP64), timed
-    like run_gpu; algorithmic bytes 159 S + 26 R per step (R = one physical
+    like run_gpu; algorithmic bytes those of the passes launched plus 26 R per step (R = one physical
     field: the stage's velocity written by the z pass (3), read by the scalar
     update with theta_s (3 + 1), theta written (1), theta^n in stages 2-3)."""
     import torch
@@ -158,10 +177,11 @@ def run_scalar(N, steps, warmup, u0, theta0, Re, dt):
     e1.record(stream)
     torch.cuda.synchronize()
     total_ms = e0.elapsed_time(e1)
+    _, calls = profiled_passes(g, lambda: g.RK3_SSP_scalar(u, th, None, steps=2))
     finite = bool(torch.isfinite(th).all().item())
     g.close()
     nc = N * N * (N // 2 + 1)
-    sb = step_bytes(nc, 16) + 26 * 8 * N ** 3
+    sb = launched_bytes(pass_bytes(nc, 16), nc, 16, steps, 1 if calls[0] < calls[4] else 3 * steps) + 26 * 8 * N ** 3
     ms_step = total_ms / steps
     return {"steps_per_s": steps / (total_ms * 1e-3), "ms_per_step": ms_step, "step_alg_bytes": sb,
             "step_roofline_frac": sb / (ms_step * 1e-3) / 1e9 / HBM_PEAK_GBS, "finite": finite}
