@@ -54,7 +54,12 @@ SPACE = {
     "NS3D_ZTWREG": (1, [0, 1], ["fp64"], "pow2"),
     "NS3D_ZTWREG32": (0, [0, 1], ["fp32", "fp32s", "fp32i"], "pow2"),
     "NS3D_WAVES_Z32": (2, [2, 3], ["fp32", "fp32s", "fp32i"], "pow2"),
-    "NS3D_WAVES_XFWD32": (2, [2, 3, 4], ["fp32", "fp32s", "fp32i"], "pow2"),
+    "NS3D_XFWD_UM64": (4, [2, 4], ["fp64"], "pow2"),
+    "NS3D_XFWD_RING64": (2, [1, 2, 3], ["fp64"], "pow2"),
+    "NS3D_WAVES_XFWD64": (2, [1, 2, 3], ["fp64"], "pow2"),
+    "NS3D_XFWD_UM32": (1, [1, 2, 4], ["fp32", "fp32s", "fp32i"], "pow2"),
+    "NS3D_XFWD_RING32": (2, [1, 2, 3], ["fp32", "fp32s", "fp32i"], "r3"),    # (these two: below 256 points)
+    "NS3D_WAVES_XFWD32": (2, [2, 3, 4], ["fp32", "fp32s", "fp32i"], "r3"),
     "NS3D_R3_PXINV64": (4, [4, 8], ["fp64"], "r3"),
     "NS3D_R3_PYINV64": (4, [4, 8], ["fp64"], "r3"),
     "NS3D_R3_PZT64": (256, [128, 256], ["fp64"], "r3"),

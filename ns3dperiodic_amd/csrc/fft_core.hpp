@@ -513,9 +513,9 @@ struct PencilFFT {
             pass2<I + 1>(va, vb, la, lb, tw, t, p, tr);
         }
     }
-    // The first exchange without LDS: an LDS store of 16 B a lane takes the CU 13.7 cycles (a
-    // load 5.0), 75 a radix-4 exchange; the swaps are 16 VALU instructions.  After a radix-4 first pass the register index (2 bits)
-    // changes places with the top two bits of t, which SwapLanes puts at lane bits 5 and 4;
+    // The first exchange without LDS: 16 VALU instructions take the place of eight LDS
+    // instructions of 16 B a lane and the waits behind them (z pass: ZPencil::SWAP).  After a
+    // radix-4 first pass the register index (2 bits) changes places with the top two bits of t, which SwapLanes puts at lane bits 5 and 4;
     // after a radix-2 one (two butterflies a thread, v[2q + r]) r with lane bit 5.
     __device__ __forceinline__ static void lane_swap(cplx<T>* v) {
         static_assert(!SWAP || (E == 4 && (R0 == 4 || R0 == 2) && (TPP & (TPP - 1)) == 0 && TPP >= 16), "plan of lane_swap");

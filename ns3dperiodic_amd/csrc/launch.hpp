@@ -250,14 +250,19 @@ template <typename TB> cplx<TB>* d_at(const ns3d_ctx* c, int nf, bool chain) {
     return (cplx<TB>*)c->scratch + (chain ? 6 * nf : 3) * c->nci;
 }
 
-// Nontemporal stores of a pass's output: for outputs beyond the 256 MiB Infinity Cache,
-// written in full 128-B lines (P modes to a row segment).  At 256^3 FP64 the pass that reads
-// them next is 4-9% faster (step 4.10 -> 3.87 ms); smaller outputs are read back from the
-// cache and lose by it (192^3 y-inverse 0.175 -> 0.195 ms, 128^3 pencil copies 0.022 -> 0.029),
-// and so do partial lines (512^3 y-inverse, 64-B segments, 2.56 -> 2.91 ms; 320^3 FP32
-// y-forward, 96-B segments, 0.155 -> 0.276 ms); 128-B segments that start in the
-// middle of a line, as FP32 rows of 136 modes have every other time, still gain: 256^3 FP32
-// step 2.71 -> 2.66 ms.
+// Nontemporal stores of a pass's output, written in full 128-B lines (P modes to a row segment),
+// where the next pass does not find it in the 256 MiB Infinity Cache anyway: FP64 from 256 MiB of
+// output, FP32 from 128 MiB.  FP64 at 256^3: the pass that reads it next is 4-9% faster (step 4.10
+// -> 3.87 ms); smaller outputs are read back from the cache and lose by it (192^3 y-inverse 0.175
+// -> 0.195 ms, 128^3 pencil copies 0.022 -> 0.029), and so do partial lines (512^3 y-inverse, 64-B
+// segments, 2.56 -> 2.91 ms; 320^3 FP32 y-forward, 96-B segments, 0.155 -> 0.276 ms).  In FP32 only
+// the y-forward pass up to 256 points in y fills lines; its reader brings the FP64 state and mostly
+// six more fields of A through the cache, so its output is lost to it from half the size on.  Five
+// steps without and with, outputs between the two lines: 256^3 15.24 and 15.00 ms (FP32 state 13.27
+// and 12.93, increments 13.88 and 13.57), 192x256x256 11.54 and 11.33, 256x192x256 12.02 and 11.81,
+// 256x256x320 20.58 and 20.37, 320x256x256 21.66 and 21.42, a step of 16 x 96^3 2.93 and 2.86; above
+// both, 384x256x256 26.33 and 26.12, 256x256x512 30.0 and 29.8, 512x256x256 34.31 and 34.23.  (Every
+// other segment of FP32 rows of 136 modes starts in the middle of a line; it pays all the same.)
 template <typename TB> int nt_for(const ns3d_ctx* c, int P, double fields) {
     return P * sizeof(cplx<TB>) >= 128 &&
            fields * (double)c->nci * c->batch * sizeof(cplx<TB>) > (sizeof(TB) == 8 ? 256.0 : 128.0) * (1 << 20);

@@ -1,5 +1,8 @@
 // tuned.hpp -- written by ns3dperiodic_amd/autotune.py (select), then NS3D_ZSWZ set from per-pass timings (its note).
 // Timed on AMD Radeon Graphics (gfx950): RK3 steps at 256^3 (power-of-two parameters) and 192^3 (NS3D_R3_*); a value replaces the baseline only when its step is faster by more than 0.5%.
+// The summed step times in the notes are those of that sweep, of kernels before the chained x-forward pass, the lane
+// swaps and the range-checked y-inverse loads (256^3 FP64 3.8 ms now); the values were not swept again since.  The
+// operand units of the x-forward pass (NS3D_XFWD_*, NS3D_WAVES_XFWD64) came later and have no note.
 #pragma once
 // NS3D_EYINV64 = 4 (kept; fp64 step at 256^3 4.3406 ms summed)
 // NS3D_PXINV64 = 8 (kept; fp64 step at 256^3 4.3406 ms summed)
