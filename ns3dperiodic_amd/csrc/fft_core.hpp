@@ -106,21 +106,26 @@ template <> struct Radix<8> {
         Radix<4>::dft<DIR>(e);
         Radix<4>::dft<DIR>(o);
         // W8^1 = (1 + DIR i)/sqrt2, W8^2 = DIR i, W8^3 = (-1 + DIR i)/sqrt2
-        const cplx<T> s1 = o[1] + mul_i<DIR>(o[1]), s3 = mul_i<DIR>(o[3]) - o[3];
-        cplx<T> o2 = mul_i<DIR>(o[2]);
-        v[0] = e[0] + o[0];
-        v[4] = e[0] - o[0];
-        v[2] = e[2] + o2;
-        v[6] = e[2] - o2;
         if constexpr (PIN) {
+            const cplx<T> s1 = o[1] + mul_i<DIR>(o[1]), s3 = mul_i<DIR>(o[3]) - o[3], o2 = mul_i<DIR>(o[2]);
+            v[0] = e[0] + o[0];
+            v[4] = e[0] - o[0];
             v[1] = fma_c(s1, c, e[1]);
             v[5] = fma_c(s1, -c, e[1]);
+            v[2] = e[2] + o2;
+            v[6] = e[2] - o2;
             v[3] = fma_c(s3, c, e[3]);
             v[7] = fma_c(s3, -c, e[3]);
         } else {
-            const cplx<T> o1 = cscale(s1, c), o3 = cscale(s3, c);
+            cplx<T> o1 = cscale(o[1] + mul_i<DIR>(o[1]), c);
+            cplx<T> o2 = mul_i<DIR>(o[2]);
+            cplx<T> o3 = cscale(mul_i<DIR>(o[3]) - o[3], c);
+            v[0] = e[0] + o[0];
+            v[4] = e[0] - o[0];
             v[1] = e[1] + o1;
             v[5] = e[1] - o1;
+            v[2] = e[2] + o2;
+            v[6] = e[2] - o2;
             v[3] = e[3] + o3;
             v[7] = e[3] - o3;
         }

@@ -292,12 +292,34 @@ k_y_inv_grad(const cplx<TB>* __restrict__ A, cplx<TB>* __restrict__ B, long nc, 
         }
     }
     auto load = [&](cplx<TB>* x, int field) __attribute__((always_inline)) {
-        const cplx<TB>* __restrict__ src = A + (long)field * nc;
-        if constexpr (RANGE) {
-            const auto rs = buf_rsrc(src, (int)(nc * (long)sizeof(cplx<TB>)));
+        const auto src = buf_rsrc(A + (long)field * nc, (int)(nc * (long)sizeof(cplx<TB>)));
 #pragma unroll
-            for (int e = 0; e < F::B0 * F::R0; e++) x[e] = buf_load<TB>(rs, off[e]);
+        for (int e = 0; e < F::B0 * F::R0; e++) x[e] = buf_load<TB>(src, off[RANGE ? e : 0]);
+    };
+    // x-derivative input, loaded before the first transforms when both are done here
+    cplx<TB> v2[(!OS && NS3D_HOIST) ? F::E : 1];
+    if constexpr (!OS && NS3D_HOIST && RANGE) {
+        load(v2, s_ * 6 + 3 + b);
+    } else if constexpr (!OS && NS3D_HOIST) {
+        const cplx<TB>* __restrict__ src = A + (long)(s_ * 6 + 3 + b) * nc;
+#pragma unroll
+        for (int q = 0; q < F::B0; q++) {
+#pragma unroll
+            for (int r = 0; r < F::R0; r++) {
+                const int kk = F::in_index(t, q, r);
+                cplx<TB> s = mk<TB>(0, 0);
+                if (F::in_active(t, q) && lv && column_kept(tab, kk, l)) s = src[base + kk * S];
+                v2[q * F::R0 + r] = s;
+            }
+        }
+    }
+    // velocity component: produce w_b and dy w_b
+    if (!OS || which < 2) {
+        cplx<TB> v[F::E], d[OS ? 1 : F::E];
+        if constexpr (RANGE) {
+            load(v, s_ * 6 + b);
         } else {
+            const cplx<TB>* __restrict__ src = A + (long)(s_ * 6 + b) * nc;
 #pragma unroll
             for (int q = 0; q < F::B0; q++) {
 #pragma unroll
@@ -305,18 +327,10 @@ k_y_inv_grad(const cplx<TB>* __restrict__ A, cplx<TB>* __restrict__ B, long nc, 
                     const int kk = F::in_index(t, q, r);
                     cplx<TB> s = mk<TB>(0, 0);
                     if (F::in_active(t, q) && lv && column_kept(tab, kk, l)) s = src[base + kk * S];
-                    x[q * F::R0 + r] = s;
+                    v[q * F::R0 + r] = s;
                 }
             }
         }
-    };
-    // x-derivative input, loaded before the first transforms when both are done here
-    cplx<TB> v2[(!OS && NS3D_HOIST) ? F::E : 1];
-    if constexpr (!OS && NS3D_HOIST) load(v2, s_ * 6 + 3 + b);
-    // velocity component: produce w_b and dy w_b
-    if (!OS || which < 2) {
-        cplx<TB> v[F::E], d[OS ? 1 : F::E];
-        load(v, s_ * 6 + b);
         if (NS3D_TW_LATE) stage_twiddles<TB, NY>(tw, twg);
 #pragma unroll
         for (int q = 0; q < F::B0; q++) {
@@ -358,8 +372,20 @@ k_y_inv_grad(const cplx<TB>* __restrict__ A, cplx<TB>* __restrict__ B, long nc, 
         if constexpr (!OS && NS3D_HOIST) {
 #pragma unroll
             for (int e = 0; e < F::E; e++) v[e] = v2[e];
-        } else {
+        } else if constexpr (RANGE) {
             load(v, s_ * 6 + 3 + b);
+        } else {
+            const cplx<TB>* __restrict__ src = A + (long)(s_ * 6 + 3 + b) * nc;
+#pragma unroll
+            for (int q = 0; q < F::B0; q++) {
+#pragma unroll
+                for (int r = 0; r < F::R0; r++) {
+                    const int kk = F::in_index(t, q, r);
+                    cplx<TB> s = mk<TB>(0, 0);
+                    if (F::in_active(t, q) && lv && column_kept(tab, kk, l)) s = src[base + kk * S];
+                    v[q * F::R0 + r] = s;
+                }
+            }
         }
         // with OS these blocks skip the velocity branch, where the table is staged otherwise
         if (NS3D_TW_LATE && OS) stage_twiddles<TB, NY>(tw, twg);
