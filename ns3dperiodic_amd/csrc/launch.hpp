@@ -231,15 +231,14 @@ inline dim3 xgrid(long nb, int nfy = 1, int nz = 1) {
 
 // Whether the x-forward pass carries the next stage's P1 (k_x_fwd_epi<..., CHAIN = 1>).
 // FP64 up to 256 points in x: above, its operands and the two inverse transforms pass 256
-// VGPRs (512^3: 4.10 ms chained against 1.51 + 2.62 ms apart).  FP32: not at radix-5
-// lengths, where the compiler contracts the 5-point butterfly's products differently in the
-// two kernels and the chained results are not bitwise those of the standalone P1; at 512,
-// where a row segment is 32 B, in the increment loop only, whose P1 reads two fields (five
-// steps chained and apart: increments 512x256x256 30.5 and 31.2 ms, FP32 bulk 34.9 and 33.9,
-// 512^3 135.0 and 131.7, FP32 state 512^3 118.0 and 116.4).
+// VGPRs (512^3: 4.10 ms chained against 1.51 + 2.62 ms apart).  FP32: not at radix-5 lengths,
+// whose 5-point butterfly is not pinned there; at 512, where a row segment is 32 B, not over the
+// FP64 state (five steps chained and apart: FP32 bulk 512x256x256 34.9 and 33.9 ms, 512^3 135.0
+// and 131.7; the increments 512x256x256 30.5 and 31.2; the FP32 state 512x64x64 1.58 and 1.66,
+// 512^3 106.0 and 106.8, with forcing 119.4 and 118.2).
 template <typename TB, int NX, int MODE>
 constexpr bool CHAINS = sizeof(TB) == 8 ? MIRROR_P1<TB, NX>
-                                          : NX % 5 != 0 && (NX < 512 || MODE == EPI_INC || MODE == EPI_INC_FINAL);
+                                          : NX % 5 != 0 && (NX < 512 || MODE != EPI_STAGE);
 
 // D of nf fields.  Where the x-forward pass writes the next stage's P1 output over A
 // (chain), D is at the head of region B; else behind C in A, on memory the z pass has not
